@@ -96,10 +96,9 @@ extern "C" {
 #define SG_F_TAIL_KERNEL (1u << 21)    /* the opposite: always the kernel behind the call (for experiments) */
 #define SG_F_SMALL_GROUPS (1u << 22)   /* sg_hip_reassemble: the call is meant to run BESIDE a long copy
                                           kernel of another stream (another receive queue's gather, or
-                                          this queue's previous burst): its kernels then come in
-                                          workgroups of 256 threads, which find room on a chip that such a
-                                          kernel keeps full, where the usual ones of 1024 wait until it
-                                          ends.  Same results.  A call that runs alone is faster without. */
+                                          this queue's previous burst).  Its kernels come in workgroups of
+                                          256 threads, which find room on a chip that such a kernel keeps
+                                          full, with or without this flag: accepted, and without effect. */
 
 /* States of an application slot (APP_RR_STATUS, src/p2p_rpc_app_ctx.h:22). */
 #define SG_SLOT_FREE 0u
@@ -494,7 +493,8 @@ int sg_hip_gather_batch_static(int device_id, void *stream, const sg_gather_args
  * the counts are where counts_out says.  counts_host_out (4 words, or NULL):
  * requests completed, their fragments, arrivals dropped, requests still in
  * flight.  The first call on a context allocates the request table and the
- * record pool (8 KiB per request of max_reqs): make it, or
+ * its records (32 KiB per request of max_reqs; less where the device has no
+ * room for that): make it, or
  * sg_hip_reassemble_reset, before recording calls into a graph. */
 int sg_hip_reassemble(sg_hip_ctx *ctx, const sg_reassemble_args *args, uint32_t *counts_host_out);
 

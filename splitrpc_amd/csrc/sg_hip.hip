@@ -128,8 +128,7 @@ struct sg_hip_ctx {
   // reassembly scratch, allocated by the first sg_hip_reassemble call
   void *ra_mem = nullptr;
   uint32_t ra_cells = 0;    // cells of the request table (power of two >= 4 * max_reqs)
-  uint32_t ra_records = 0;  // records of the pool (power of two >= max_reqs)
-  uint32_t *h_counts = nullptr;  // pinned: requests, fragments, dropped, in flight (written by k_ra_scan itself)
+  uint32_t *h_counts = nullptr;  // pinned: requests, fragments, dropped, in flight (written by the reassembly's kernels themselves)
   char err[512] = {0};
 };
 
@@ -1495,11 +1494,7 @@ uint32_t pow2_at_least(uint64_t v)
 int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
 {
   const uint32_t n_max = c->max_frames;
-  const uint32_t cells = pow2_at_least(4ull * c->max_reqs < 2 * kRaBucket ? 2 * kRaBucket : 4ull * c->max_reqs);
-  const uint32_t records = pow2_at_least(c->max_reqs);
-  const size_t n_blk = (n_max + kRaSmallBlock - 1) / kRaSmallBlock + 1;  // a total per workgroup of k_ra_flag, the small ones
-  const size_t bytes = (size_t)cells * (8 + 8 + 4 * 4) + (size_t)records * SG_MAX_BI_SIZE * 8 + (size_t)records * 4 +
-                       kRaWords * 4 + (size_t)n_max * (3 * 4 + 8) + n_blk * 8 + 256;
+  const size_t n_blk = ((size_t)n_max + kRaBlock - 1) / kRaBlock + 1;
   *fresh = false;
   if (!c->ra_mem) {
     // the small allocation first: a context never holds the state without its pinned counts
@@ -1507,29 +1502,41 @@ int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
       HIP_TRY(c, hipHostMalloc((void **)&c->h_counts, 4 * sizeof(uint32_t), hipHostMallocDefault));
       memset(c->h_counts, 0, 4 * sizeof(uint32_t));
     }
-    HIP_TRY(c, hipMalloc(&c->ra_mem, bytes));
+    // Four cells for every request that may be in flight: a bucket of 32 then holds 8 on average and
+    // never fills up.  Where the device has no room for that many records (32 KiB per request), fewer:
+    // a bucket may then be full before max_reqs are in flight, which refuses the call that finds it so.
+    const uint32_t least = pow2_at_least(c->max_reqs);
+    uint32_t cells = pow2_at_least(4ull * c->max_reqs < 2 * kRaBucket ? 2 * kRaBucket : 4ull * c->max_reqs);
+    for (;;) {
+      const size_t bytes = (size_t)cells * (SG_MAX_BI_SIZE * 8 + 8 + 8 + 3 * 4) + kRaWords * 4 + (size_t)n_max * (8 + 4) +
+                           n_blk * 2 * 8 + 256;
+      const hipError_t e = hipMalloc(&c->ra_mem, bytes);
+      if (e == hipSuccess) break;
+      c->ra_mem = nullptr;
+      (void)hipGetLastError();
+      if (e != hipErrorOutOfMemory || cells <= least || cells <= 2 * kRaBucket)
+        return fail(c, SG_E_NOMEM, "request table of %zu bytes: %s", bytes, hipGetErrorString(e));
+      cells >>= 1;
+    }
     c->ra_cells = cells;
-    c->ra_records = records;
     *fresh = true;
   }
+  const uint32_t cells = c->ra_cells;
   memset(r, 0, sizeof *r);
   uint8_t *m = static_cast<uint8_t *>(c->ra_mem);
+  r->tab = reinterpret_cast<unsigned long long *>(m); m += (size_t)cells * SG_MAX_BI_SIZE * 8;
   r->keys = reinterpret_cast<unsigned long long *>(m); m += (size_t)cells * 8;
   r->acc = reinterpret_cast<unsigned long long *>(m); m += (size_t)cells * 8;
-  r->tab = reinterpret_cast<unsigned long long *>(m); m += (size_t)records * SG_MAX_BI_SIZE * 8;
-  r->arr_pack = reinterpret_cast<unsigned long long *>(m); m += (size_t)n_max * 8;
   r->blk = reinterpret_cast<unsigned long long *>(m); m += n_blk * 8;
+  r->blk_new = reinterpret_cast<unsigned long long *>(m); m += n_blk * 8;
+  r->arr_pack = reinterpret_cast<unsigned long long *>(m); m += (size_t)n_max * 8;
   r->want = reinterpret_cast<uint32_t *>(m); m += (size_t)cells * 4;
   r->last = reinterpret_cast<uint32_t *>(m); m += (size_t)cells * 4;
-  r->rec = reinterpret_cast<uint32_t *>(m); m += (size_t)cells * 4;
   r->seen = reinterpret_cast<uint32_t *>(m); m += (size_t)cells * 4;
-  r->free_ring = reinterpret_cast<uint32_t *>(m); m += (size_t)records * 4;
   r->words = reinterpret_cast<uint32_t *>(m); m += kRaWords * 4;
-  r->arr_cell = reinterpret_cast<uint32_t *>(m); m += (size_t)n_max * 4;
-  r->arr_len = reinterpret_cast<uint32_t *>(m); m += (size_t)n_max * 4;
-  r->arr_fidx = reinterpret_cast<uint32_t *>(m);
+  r->arr_cell = reinterpret_cast<uint32_t *>(m);
   r->bmask = cells / kRaBucket - 1;
-  r->rmask = records - 1;
+  r->pool = pow2_at_least(c->max_reqs);
   r->counts_host = c->h_counts;
   r->status = c->status;
   r->status_flag = c->h_flag;
@@ -1538,9 +1545,8 @@ int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
 
 void ra_launch_reset(sg_hip_ctx *c, const RaArgs &r)
 {
-  const size_t items = (size_t)c->ra_records * SG_MAX_BI_SIZE > c->ra_cells ? (size_t)c->ra_records * SG_MAX_BI_SIZE
-                                                                            : c->ra_cells;
-  k_ra_reset<<<(uint32_t)((items + 255) / 256), 256, 0, c->stream>>>(r, c->ra_cells, c->ra_records);
+  const size_t items = (size_t)c->ra_cells * (SG_MAX_BI_SIZE / 2);  // two entries per thread: more than there are cells
+  k_ra_reset<<<(uint32_t)((items + 255) / 256), 256, 0, c->stream>>>(r, c->ra_cells);
 }
 
 }  // namespace
@@ -1605,10 +1611,6 @@ int sg_hip_reassemble(sg_hip_ctx *c, const sg_reassemble_args *a, uint32_t *coun
   r.req_size = a->req_size;
   r.max_req = c->max_reqs;
   r.max_frag = c->max_frames;
-  // workgroups of 256 threads where the caller says the call runs beside a long kernel
-  const bool small_groups = (a->flags & SG_F_SMALL_GROUPS) != 0;
-  r.blk_size = small_groups ? kRaSmallBlock : kRaBlock;
-  r.n_blocks = (a->n_arrivals + r.blk_size - 1) / r.blk_size;
   r.frag_slot = a->frag_slot;
   r.frag_len = a->frag_len;
   r.req_first = a->req_first;
@@ -1616,24 +1618,18 @@ int sg_hip_reassemble(sg_hip_ctx *c, const sg_reassemble_args *a, uint32_t *coun
   r.req_hdr_slot = a->req_hdr_slot;
   r.counts_out = a->counts_out;
 
-  const uint32_t g_take = (a->n_arrivals + kRaTakeBlock - 1) / kRaTakeBlock;
   rc = prof_begin(c, 5);
   if (rc != SG_OK) return rc;
-  if (a->n_arrivals <= (uint32_t)kRaTakeBlock) {
+  if (a->n_arrivals <= (uint32_t)kRaSmallBurst) {
+    k_ra_burst<kRaSmallBurst><<<1, kRaSmallBurst, 0, c->stream>>>(r);
+  } else if (a->n_arrivals <= (uint32_t)kRaBurst) {
     // a NIC burst (an empty one still leaves its counts): one workgroup, one launch
-    k_ra_burst<<<1, kRaTakeBlock, 0, c->stream>>>(r);
+    k_ra_burst<kRaBurst><<<1, kRaBurst, 0, c->stream>>>(r);
   } else {
-    if (small_groups) {
-      k_ra_insert<kRaSmallBlock><<<r.n_blocks, kRaSmallBlock, 0, c->stream>>>(r);
-      k_ra_flag<kRaSmallBlock><<<r.n_blocks, kRaSmallBlock, 0, c->stream>>>(r);
-      k_ra_scan<kRaSmallBlock><<<1, kRaSmallBlock, 0, c->stream>>>(r);
-      k_ra_emit<kRaSmallBlock><<<r.n_blocks, kRaSmallBlock, 0, c->stream>>>(r);
-    } else {
-      k_ra_insert<kRaTakeBlock><<<g_take, kRaTakeBlock, 0, c->stream>>>(r);
-      k_ra_flag<kRaBlock><<<r.n_blocks, kRaBlock, 0, c->stream>>>(r);
-      k_ra_scan<kRaBlock><<<1, kRaBlock, 0, c->stream>>>(r);
-      k_ra_emit<kRaTakeBlock><<<g_take, kRaTakeBlock, 0, c->stream>>>(r);
-    }
+    const uint32_t grid = (a->n_arrivals + kRaBlock - 1) / kRaBlock;
+    k_ra_insert<kRaBlock><<<grid, kRaBlock, 0, c->stream>>>(r);
+    k_ra_flag<kRaBlock><<<grid, kRaBlock, 0, c->stream>>>(r);
+    k_ra_emit<kRaBlock><<<grid, kRaBlock, 0, c->stream>>>(r);
   }
   rc = prof_end(c);
   if (rc != SG_OK) return rc;

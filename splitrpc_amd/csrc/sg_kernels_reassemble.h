@@ -21,38 +21,53 @@ namespace {
 //   request table   token -> cell, open addressing in buckets of kRaBucket
 //                   cells: a lookup reads the whole bucket, so emptying a cell
 //                   (a completed request) never hides another request, and a
-//                   new token claims the lowest empty cell by atomicCAS
-//   record pool     one record per request in flight: SG_MAX_BI_SIZE entries
+//                   new token claims an empty cell by atomicCAS
+//   records         every cell has a record of its own: SG_MAX_BI_SIZE entries
 //                   {slot, length} indexed by sequence number (p2p_bufs of the
-//                   reference's rr); free records wait in a ring with a head
-//                   and a tail word on the device (the rr pool's free ring,
-//                   src/p2p_rpc_rr_pool_ng.h:121-147: consume_rr / reap_rr)
-//   k_ra_insert  one thread per arrival: find or claim the request's cell (a
-//                claimed cell takes a record off the free ring), add to its
-//                fragment count / byte total, note the arrival's position
-//   k_ra_flag    every arrival files its entry in its request's record; the
-//                thread of a complete request's LAST arrival flags that
+//                   reference's rr).  The cell a token is found in says where
+//                   its fragments are filed; a record is neither taken nor
+//                   given back.
+//   k_ra_insert  one thread per arrival.  The workgroup first sorts its
+//                arrivals by token in LDS; one thread per DISTINCT token finds
+//                or claims the request's cell and adds the workgroup's share
+//                to its fragment count, byte total and last position; then
+//                every arrival files its entry in the request's record
+//   k_ra_flag    the thread of a complete request's LAST arrival flags that
 //                position with the request's fragment count; workgroup-local
 //                scan of the packed (requests, fragments) flags
-//   k_ra_scan    one workgroup scans the workgroup totals and leaves the counts
-//                on the device and in pinned host memory
 //   k_ra_emit    batch index of a request = number of requests completed before
 //                it in this call (completion order, the order of the rx-ready
-//                ring); the wavefront of the completing arrival copies the
-//                record into the output tables, empties it, returns it to the
-//                free ring and empties the cell
-// Nothing waits on another thread: every probe and every ring operation makes
-// progress by itself.
+//                ring); a wavefront in which requests complete adds up the
+//                totals of the workgroups before its own, copies the records
+//                into the output tables, empties them and their cells; the
+//                first wavefront closes the call: counts, epoch
+// Nothing waits on another thread: every probe makes progress by itself.
+//
+// What bounds it: dependent round trips (arrival -> header -> bucket -> claim -> entry), not bytes.
+// So each is made once, for all of a workgroup's tokens side by side, and nothing is added to a word
+// that other workgroups add to as well except the request's own totals.  Kernel trace, us:
+//                                          220672 arrivals of        65536 interleaved arrivals of
+//                                          512 requests (431 each)   32768 requests (2 each)
+//   a group of lanes after the other goes
+//   to the table, records from a ring:
+//     insert / flag / scan / emit          23.2 / 5.5 / 4.9 / 8.4    30.1 / 9.7 / 4.7 / 13.0
+//   this form: insert / flag / emit        11.3 / 4.9 / 6.6          14.6 / 4.8 / 7.7
+//   64 arrivals in one launch              8.6 -> 5.4
+// (a launch that does nothing shows as 2 to 4 us there).  Workgroups of 512 threads: 11.9 / 5.2 / 6.0
+// and 14.0 / 5.1 / 9.4; of 1024: 12.2 / 5.2 / 5.8 and 20.5 / 6.8 / 10.8.  The ring of free records
+// cost a returning addition per workgroup to one word, 35 to 70 ns each and one after the other, and
+// two dependent reads per new request; a record per cell takes four times the room.
 
 constexpr uint32_t kRaBucket = 32;
-static_assert(kRaBucket == 32, "ra_find_cell takes a token's first cell from the top five bits of its hash");
-constexpr uint32_t kRaNoCell = 0xffffffffu;
-constexpr uint32_t kRaNoRec = 0xffffffffu;
-constexpr int kRaBlock = 1024;
+static_assert(kRaBucket == 32, "ra_find_cell keeps one bit per cell and takes a token's first cell from the top five bits of its hash");
+constexpr uint32_t kRaNoCell = 0x7fffffffu;
+// beside the cell of an arrival: its thread is the one that went to the table for the token
+constexpr uint32_t kRaOwner = 0x80000000u;
+constexpr int kRaBlock = 256;       // workgroup of the three kernels
+constexpr int kRaBurst = 1024;      // most arrivals that one workgroup takes in one launch
+constexpr int kRaSmallBurst = 256;  // most that a smaller one takes
 // device words of the reassembly state
-// kRaHeadSeen: where k_ra_scan last saw the head -- how far it has moved since is the number of
-// cells claimed in between
-enum { kRaHead = 0, kRaTail, kRaEpoch, kRaInFlight, kRaHeadSeen, kRaDropped, kRaOverflow, kRaEvicted, kRaWords = 16 };
+enum { kRaEpoch = 0, kRaInFlight, kRaEvicted, kRaWords = 16 };
 
 struct RaArgs {
   const uint8_t *ring;
@@ -63,22 +78,21 @@ struct RaArgs {
   const uint32_t *len_nic;
   uint64_t req_size;  // REF64 readiness: bytes == req_size; BL58: fragments == num_frags
   uint32_t bmask;     // buckets - 1
-  uint32_t rmask;     // records - 1
+  uint32_t pool;      // requests that may be in flight
   uint32_t max_req, max_frag;  // room in the output tables
   // request table: cells
   unsigned long long *keys;
-  unsigned long long *acc;  // fragments so far << 40 | payload bytes so far: one atomic addition per arrival
-  uint32_t *want, *last, *rec, *seen;
-  // record pool
-  unsigned long long *tab;  // records x SG_MAX_BI_SIZE entries: slot | length << 32
-  uint32_t *free_ring;
-  uint32_t *words;          // kRa* above
+  unsigned long long *acc;   // fragments so far << 40 | payload bytes so far: one atomic addition per workgroup and token
+  uint32_t *last;            // position in this call of the token's latest arrival; zero between calls
+  uint32_t *want, *seen;     // fragments of the request; epoch of the latest call that brought one
+  unsigned long long *tab;   // a record per cell: SG_MAX_BI_SIZE entries slot | length << 32
+  uint32_t *words;           // kRa* above
   // per arrival of this call
-  uint32_t *arr_cell, *arr_len, *arr_fidx;
-  unsigned long long *arr_pack;  // (1 << 32 | fragments) at the completing arrival, else 0; then its local scan
-  unsigned long long *blk;       // workgroup totals, then their scan
-  uint32_t n_blocks;
-  uint32_t blk_size;  // threads per workgroup of k_ra_flag: one entry of blk each
+  uint32_t *arr_cell;            // | kRaOwner
+  unsigned long long *arr_pack;  // RaPack at the completing arrival, else 0
+  // per workgroup of k_ra_insert / k_ra_flag
+  unsigned long long *blk;       // packed (requests, fragments) completed in it
+  unsigned long long *blk_new;   // cells claimed << 32 | arrivals dropped
   // outputs
   uint32_t *frag_slot, *frag_len, *req_first, *req_hdr_slot;
   uint64_t *req_token;
@@ -95,7 +109,7 @@ __device__ __forceinline__ uint32_t ra_n(const RaArgs &a)
 
 // A cell's fragment count and byte total in one word (a request has at most SG_MAX_BI_SIZE
 // fragments and far fewer than 2^40 bytes): device-scope atomics are what a burst of many small
-// requests pays for, one per arrival instead of two.
+// requests pays for, one per addition instead of two.
 constexpr int kRaCntShift = 40;
 __device__ __forceinline__ unsigned long long ra_pack(uint32_t n, unsigned long long bytes)
 {
@@ -105,6 +119,19 @@ __device__ __forceinline__ uint32_t ra_cnt(unsigned long long acc) { return (uin
 __device__ __forceinline__ unsigned long long ra_bytes(unsigned long long acc)
 {
   return acc & ((1ull << kRaCntShift) - 1ull);
+}
+
+// What k_ra_flag leaves at a completing arrival: top bit set, the request's fragment count (at most
+// 1024: 11 bits), the requests (11 bits) and fragments (21 bits) completed before it in its workgroup.
+static_assert(SG_MAX_BI_SIZE <= 1024, "eleven bits for a fragment count");
+__device__ __forceinline__ unsigned long long ra_done(uint32_t cnt, uint64_t before)
+{
+  return 1ull << 63 | (unsigned long long)cnt << 48 | (before >> 32) << 32 | (uint32_t)before;
+}
+__device__ __forceinline__ uint32_t ra_done_cnt(unsigned long long d) { return (uint32_t)(d >> 48) & 0x7fffu; }
+__device__ __forceinline__ uint64_t ra_done_before(unsigned long long d)
+{
+  return d & 0x0000ffffffffffffull;
 }
 
 __device__ __forceinline__ uint32_t ra_hash(unsigned long long k)
@@ -120,8 +147,8 @@ __device__ __forceinline__ unsigned long long ra_key(const unsigned long long *p
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Find or claim the cell of `token`.  The whole bucket is read first: the
-// request may sit anywhere in it (cells empty as requests complete).  Only then
+// Find or claim the cell of `token`.  The whole bucket is read first, all of it asked for at once:
+// the request may sit anywhere in it (cells empty as requests complete).  Only then
 // is an empty cell claimed.  Every token walks the bucket in an order of its
 // own -- cyclically from a cell its hash picks -- starting at the first cell of
 // that order it has seen empty and trying every empty cell on the way; cells
@@ -131,34 +158,30 @@ __device__ __forceinline__ unsigned long long ra_key(const unsigned long long *p
 // order for all tokens -- lowest cell first -- the new requests of a burst that
 // share a bucket queued up on its lowest empty cells, one failed
 // compare-and-swap round trip after the other.)
-__device__ __forceinline__ uint32_t ra_find_cell(const RaArgs &a, unsigned long long token, bool *claimed)
+__device__ __forceinline__ uint32_t ra_find_cell(const RaArgs &a, unsigned long long token, uint32_t hash, bool *claimed)
 {
-  const uint32_t hash = ra_hash(token);
   const uint32_t b = (hash & a.bmask) * kRaBucket;
-  const uint32_t start = hash >> 27;  // kRaBucket == 32: the top five bits, the bucket takes the low ones
+  const uint32_t start = hash >> 27;  // the top five bits: the bucket takes the low ones
   *claimed = false;
-  uint32_t first_rank = kRaBucket;  // place in this token's order of the first cell seen empty
-#pragma unroll 1
-  for (uint32_t h = 0; h < kRaBucket; h += 16) {
-    // Ordinary 16-byte loads, two keys each.  While arrivals are being filed a key only ever goes
-    // from empty to a token, so all a load that is behind the times can show is an empty cell that
-    // has just been taken -- and the claim below goes through atomicCAS, which then returns the
-    // taker (this thread's own token included).
-    unsigned long long k[16];
-    const ulonglong2 *kp = reinterpret_cast<const ulonglong2 *>(a.keys + b + h);
+  // Ordinary 16-byte loads, two keys each.  While arrivals are being filed a key only ever goes
+  // from empty to a token, so all a load that is behind the times can show is an empty cell that
+  // has just been taken -- and the claim below goes through atomicCAS, which then returns the
+  // taker (this thread's own token included).
+  const ulonglong2 *kp = reinterpret_cast<const ulonglong2 *>(a.keys + b);
+  ulonglong2 v[kRaBucket / 2];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const ulonglong2 v = kp[j];
-      k[2 * j] = v.x;
-      k[2 * j + 1] = v.y;
-    }
+  for (uint32_t j = 0; j < kRaBucket / 2; j++) v[j] = kp[j];
+  uint32_t found = 0, empty = 0;  // a bit per cell
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
-      if (k[j] == token) return b + h + j;
-      const uint32_t rank = (h + j - start) & (kRaBucket - 1);
-      if (k[j] == 0ull && rank < first_rank) first_rank = rank;
-    }
+  for (uint32_t j = 0; j < kRaBucket / 2; j++) {
+    found |= (v[j].x == token ? 1u << (2 * j) : 0u) | (v[j].y == token ? 2u << (2 * j) : 0u);
+    empty |= (v[j].x == 0ull ? 1u << (2 * j) : 0u) | (v[j].y == 0ull ? 2u << (2 * j) : 0u);
   }
+  if (found) return b + (uint32_t)__ffs((int)found) - 1;
+  if (!empty) return kRaNoCell;
+  // place in this token's order of the first cell seen empty
+  const uint32_t turned = start ? (empty >> start) | (empty << (32u - start)) : empty;
+  const uint32_t first_rank = (uint32_t)__ffs((int)turned) - 1;
 #pragma unroll 1
   for (uint32_t rank = first_rank; rank < kRaBucket; rank++) {
     const uint32_t j = (start + rank) & (kRaBucket - 1);
@@ -175,422 +198,453 @@ __device__ __forceinline__ uint32_t ra_find_cell(const RaArgs &a, unsigned long 
   return kRaNoCell;  // bucket full
 }
 
-// Positions on a ring word for a whole workgroup with ONE addition: every wavefront says how many it
-// needs and gets its first.  (A returning addition per wavefront on a word that thousands of wavefronts
-// on eight XCDs add to takes some 70 ns, one after the other: 0.29 ms of a 0.35-ms k_ra_insert on a
-// burst of 131072 new requests.)  Every thread of the workgroup has to call this.
-constexpr int kRaTakeBlock = 1024;
-// The same steps in workgroups of kRaSmallBlock threads, for a call that runs beside a long copy
-// kernel of another stream: a workgroup of sixteen wavefronts finds no room on a chip that such a
-// kernel keeps full (it needs sixteen free slots on one CU at once) and waits until that kernel
-// ends; one of four wavefronts takes the slots the copy's own workgroups leave.  Four times the
-// additions to the ring words, which is why this is not the form of a call that runs alone.
-constexpr int kRaSmallBlock = 256;
+// The distinct tokens among a workgroup's arrivals, open addressing in LDS, twice as many entries
+// as arrivals: what the workgroup brings of each -- fragments and bytes, last position -- and, once
+// the thread that put the token in has been to the table, its cell.
 template <int B>
-__device__ __forceinline__ uint32_t ra_block_take(uint32_t *word, uint32_t n_wave, uint32_t *lds)
-{
-  constexpr uint32_t kWaves = B / kWave;
-  const uint32_t wv = threadIdx.x / kWave;
-  if ((threadIdx.x & (kWave - 1)) == 0) lds[wv] = n_wave;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t tot = 0;
-    for (uint32_t w = 0; w < kWaves; w++) {
-      const uint32_t t = lds[w];
-      lds[w] = tot;
-      tot += t;
-    }
-    lds[kWaves] = tot ? atomicAdd(word, tot) : 0u;
-  }
-  __syncthreads();
-  return lds[kWaves] + lds[wv];
-}
-
-// Records for the cells the threads of this workgroup have just claimed: one addition to the
-// ring's head for all of them.  The tail does not move during the kernel that takes records
-// (returns happen in k_ra_emit), so a position at or beyond the tail read here means the pool is
-// exhausted: the cell then gets no record, the call is refused, and k_ra_scan puts the head back
-// to the tail.
-template <int B>
-__device__ __forceinline__ void ra_open_cells(const RaArgs &a, bool claimed, uint32_t cell, uint32_t lane, uint32_t *lds)
-{
-  const unsigned long long cl = __ballot(claimed);
-  const uint32_t base = ra_block_take<B>(&a.words[kRaHead], (uint32_t)__popcll(cl), lds);
-  if (claimed) {
-    const uint32_t h = base + (uint32_t)__popcll(cl & ((1ull << lane) - 1ull));
-    const uint32_t tail = a.words[kRaTail];
-    const uint32_t r = (int32_t)(tail - h) > 0 ? a.free_ring[h & a.rmask] : kRaNoRec;
-    a.rec[cell] = r;
-    if (r == kRaNoRec) refuse(a.status, a.status_flag, kStPoolFull);
-  }
-}
-
-// Fragments of one request tend to arrive together, so the lanes of a
-// wavefront are first grouped by token: a group's first lane looks the cell up
-// once and adds the group's fragment count, bytes and last position in one
-// atomic each.  After kRaRounds groups the lanes still waiting go one by one
-// (bursts that interleave many requests).
-constexpr int kRaRounds = 4;
-
-// The four steps of a call as functions of the arrival's index: launched as four kernels, or --
-// a burst that fits one workgroup, which is what a NIC delivers -- one behind the other in ONE
-// kernel (FUSED), with workgroup barriers where the kernel boundaries were.  What a step reads of
-// what other threads left through device-scope atomics in an earlier step of the same kernel
-// (counts and bytes, last positions, keys, ring words) it then reads with device-scope loads: an
-// ordinary load could still find the line as a cache held it before the atomic went to memory.
-template <bool FUSED>
-__device__ __forceinline__ unsigned long long ra_acc(const RaArgs &a, uint32_t cell)
-{
-  return FUSED ? __hip_atomic_load(a.acc + cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.acc[cell];
-}
-template <bool FUSED>
-__device__ __forceinline__ uint32_t ra_word(const uint32_t *p)
-{
-  return FUSED ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
-}
-
-// What a thread knows of its arrival from one step to the next.  The four-kernel form keeps it in
-// device memory (arr_cell / arr_len / arr_fidx / arr_pack); a burst handled by one workgroup keeps
-// it in registers: every thread only ever reads its own entries, and a store followed by a load of
-// the same word is a memory round trip the burst's latency is made of.
-struct RaMine {
-  uint32_t slot = 0, cell = kRaNoCell, len = 0, fidx = 0;
-  unsigned long long pack = 0;
+struct RaLds {
+  static constexpr uint32_t kEntries = 2 * B;
+  unsigned long long key[kEntries];
+  unsigned long long acc[kEntries];
+  uint32_t last[kEntries];  // thread index
+  uint32_t cell[kEntries];
 };
 
-template <bool FUSED, int B>
-__device__ __forceinline__ void ra_insert_step(const RaArgs &a, uint32_t i, uint32_t *take, RaMine &mine)
+template <int B>
+__device__ __forceinline__ void ra_lds_clear(RaLds<B> &l)
 {
-  const uint32_t n = ra_n(a);
-  const uint32_t lane = threadIdx.x & (kWave - 1);
-  const bool in_range = i < n;
-  const uint32_t epoch = a.words[kRaEpoch];  // advanced by k_ra_scan, behind this kernel
-  uint32_t cell = kRaNoCell, len = 0, fidx = 0, want = 0;
-  uint32_t opened = kRaNoCell;  // the cell this lane has claimed for a new request, if any
-  unsigned long long token = 0;
-  bool pending = false;
-  if (in_range) {
-    const uint32_t slot = a.arrivals[i];
-    mine.slot = slot;
-    if (slot >= a.n_slots) {
-      refuse(a.status, a.status_flag, kStBadSlot);
-    } else {
-      const uint8_t *h = a.ring + (size_t)slot * a.slot_size;
-      const uint32_t t0 = load32_any(h + 42), t1 = load32_any(h + 46);
-      token = ((unsigned long long)t1 << 32) | t0;
-      if (a.ref64) {
-        fidx = load32_any(h + 58) & 0xffffu;
-        len = a.len_nic[slot];
-      } else {
-        const uint32_t w = load32_any(h + 50);
-        fidx = w & 0xffffu;
-        want = w >> 16;
-        len = a.len_nic ? a.len_nic[slot] : load32_any(h + 54);
-      }
-      const uint32_t hl = a.ref64 ? 64u : 58u;
-      if (len > a.slot_size - hl) {
-        refuse(a.status, a.status_flag, kStBadLen);
-        len = 0;
-      } else {
-        pending = token != 0;  // token 0: dropped (src/transport/dpdk_transport_ng.h:231)
+#pragma unroll
+  for (uint32_t k = 0; k < RaLds<B>::kEntries / B; k++) {
+    l.key[k * B + threadIdx.x] = 0;
+    l.acc[k * B + threadIdx.x] = 0;
+    l.last[k * B + threadIdx.x] = 0;
+  }
+}
+
+// The entry of `token`; *owner: this thread has put it in.
+template <int B>
+__device__ __forceinline__ uint32_t ra_lds_entry(RaLds<B> &l, unsigned long long token, uint32_t hash, bool *owner)
+{
+  constexpr uint32_t kMask = RaLds<B>::kEntries - 1;
+  uint32_t e = (hash >> 7) & kMask;
+  for (;;) {  // at most B distinct tokens: an empty entry is always found
+    unsigned long long k = __hip_atomic_load(&l.key[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (k == 0ull) {
+      k = atomicCAS(&l.key[e], 0ull, token);
+      if (k == 0ull) {
+        *owner = true;
+        return e;
       }
     }
+    if (k == token) return e;
+    e = (e + 1) & kMask;
   }
-  for (int round = 0; round < kRaRounds; round++) {
-    const unsigned long long waiting = __ballot(pending);
-    if (!waiting) break;
-    const int first = __ffsll((long long)waiting) - 1;
-    const unsigned long long t = ((unsigned long long)(uint32_t)__shfl((int)(token >> 32), first, kWave) << 32) |
-                                 (uint32_t)__shfl((int)(uint32_t)token, first, kWave);
-    const bool mine = pending && token == t;
-    const unsigned long long group = __ballot(mine);
-    // a burst that interleaves many requests: groups of one or two lanes, each a chain of
-    // dependent round trips that the other lanes sit out -- every lane for itself then
-    if (round == 0 && 8 * __popcll(group) < __popcll(waiting)) break;
-    const uint32_t g_bytes = wave_sum(mine ? len : 0u);
-    uint32_t c = kRaNoCell;
+}
+
+// An arrival as its thread knows it.
+struct RaMine {
+  uint32_t slot = 0, len = 0, fidx = 0, want = 0;
+  unsigned long long token = 0;  // 0: not to be filed (no such arrival, token 0, refused)
+};
+
+__device__ __forceinline__ RaMine ra_read(const RaArgs &a, uint32_t i, bool in_range)
+{
+  RaMine m;
+  if (!in_range) return m;
+  m.slot = a.arrivals[i];
+  if (m.slot >= a.n_slots) {
+    refuse(a.status, a.status_flag, kStBadSlot);
+    return m;
+  }
+  const uint8_t *h = a.ring + (size_t)m.slot * a.slot_size;
+  // token and, with the 58-byte header, everything else as well: bytes 42..57 in one load (every
+  // lane has a cache line of its own, so what counts is the number of loads)
+  const u32x4 w = load128_any(h + 42);
+  if (a.ref64) {
+    m.fidx = load32_any(h + 58) & 0xffffu;
+    m.len = a.len_nic[m.slot];
+  } else {
+    m.fidx = w[2] & 0xffffu;
+    m.want = w[2] >> 16;
+    m.len = a.len_nic ? a.len_nic[m.slot] : w[3];
+  }
+  const uint32_t hl = a.ref64 ? 64u : 58u;
+  if (m.len > a.slot_size - hl) {
+    refuse(a.status, a.status_flag, kStBadLen);
+    m.len = 0;
+  } else {
+    m.token = ((unsigned long long)w[1] << 32) | w[0];  // token 0: dropped (src/transport/dpdk_transport_ng.h:231)
+  }
+  return m;
+}
+
+// Enters the workgroup's arrivals into the LDS table.  Fragments of one request tend to arrive
+// together: where the first waiting lane's token is that of many lanes, they go in with one
+// addition (LDS atomics of a wavefront on one word take a turn per lane).
+template <int B>
+__device__ __forceinline__ uint32_t ra_group(RaLds<B> &l, const RaMine &m, uint32_t hash, uint32_t lane, bool *owner)
+{
+  uint32_t e = 0;
+  bool waiting = m.token != 0;
+  const unsigned long long all = __ballot(waiting);
+  *owner = false;
+  if (!all) return 0;
+  const int first = __ffsll((long long)all) - 1;
+  const unsigned long long t = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(m.token >> 32), first) << 32) |
+                               (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)m.token, first);
+  const bool same = waiting && m.token == t;
+  const unsigned long long group = __ballot(same);
+  if (__popcll(group) >= 8) {
+    const uint32_t bytes = wave_sum_uniform(same ? m.len : 0u);
     if ((int)lane == first) {
-      bool claimed;
-      c = ra_find_cell(a, t, &claimed);
-      if (c != kRaNoCell) {
-        if (claimed) opened = c;
-        atomicAdd(&a.acc[c], ra_pack((uint32_t)__popcll(group), g_bytes));
-        atomicMax(&a.last[c], i - lane + (63u - (uint32_t)__clzll((long long)group)));
-        if (!a.ref64) a.want[c] = want;  // every fragment of a request says the same
-        a.seen[c] = epoch;
-      }
+      e = ra_lds_entry<B>(l, t, hash, owner);
+      atomicAdd(&l.acc[e], ra_pack((uint32_t)__popcll(group), bytes));
+      atomicMax(&l.last[e], threadIdx.x - lane + (63u - (uint32_t)__clzll((long long)group)));
     }
-    c = (uint32_t)__shfl((int)c, first, kWave);
-    if (mine) {
-      cell = c;
-      pending = false;
+    const uint32_t eg = (uint32_t)__builtin_amdgcn_readlane((int)e, first);
+    if (same) {
+      e = eg;
+      waiting = false;
     }
   }
-  if (pending) {
-    bool claimed;
-    cell = ra_find_cell(a, token, &claimed);
-    if (cell != kRaNoCell) {
-      if (claimed) opened = cell;
-      atomicAdd(&a.acc[cell], ra_pack(1u, len));
-      atomicMax(&a.last[cell], i);
-      if (!a.ref64) a.want[cell] = want;
-      a.seen[cell] = epoch;
-    }
+  if (waiting) {
+    e = ra_lds_entry<B>(l, m.token, hash, owner);
+    atomicAdd(&l.acc[e], ra_pack(1u, m.len));
+    atomicMax(&l.last[e], threadIdx.x);
   }
-  // the cells this wavefront has claimed get their records (a lane claims one cell at most)
-  ra_open_cells<B>(a, opened != kRaNoCell, opened, lane, take);
-  mine.cell = cell;
-  mine.len = len;
-  mine.fidx = fidx;
-  if (in_range) {
-    if (!FUSED) {
-      a.arr_cell[i] = cell;
-      a.arr_len[i] = len;
-      a.arr_fidx[i] = fidx;
-    }
-    if (cell == kRaNoCell && token != 0) refuse(a.status, a.status_flag, kStPoolFull);  // bucket full
-  }
-  // arrivals that belong to no request: token 0, refused, no room
-  const unsigned long long lost = __ballot(in_range && cell == kRaNoCell);
-  if (lane == 0 && lost) atomicAdd(&a.words[kRaDropped], (uint32_t)__popcll(lost));
+  return e;
+}
+
+// rr_emplace_mbuf: the entry goes where its sequence number says.
+__device__ __forceinline__ void ra_file(const RaArgs &a, uint32_t cell, const RaMine &m)
+{
+  if (m.fidx < SG_MAX_BI_SIZE)
+    a.tab[(size_t)cell * SG_MAX_BI_SIZE + m.fidx] = (unsigned long long)m.slot | ((unsigned long long)m.len << 32);
+  else
+    refuse(a.status, a.status_flag, kStBadTable);  // beyond what a request's tables hold (src/p2p_bufs.h:10)
+}
+
+// Arrivals that belong to no request (token 0, refused, no room) and cells claimed, counted over
+// the workgroup.  Every thread calls this; the totals are thread 0's.
+template <int B>
+__device__ __forceinline__ unsigned long long ra_count_new(bool claimed, bool lost, uint32_t lane, unsigned long long *lds)
+{
+  const unsigned long long c = __ballot(claimed), d = __ballot(lost);
+  if (lane == 0) lds[threadIdx.x / kWave] = (unsigned long long)__popcll(c) << 32 | (uint32_t)__popcll(d);
+  __syncthreads();
+  unsigned long long t = 0;
+  if (threadIdx.x == 0)
+    for (uint32_t w = 0; w < B / kWave; w++) t += lds[w];
+  return t;
 }
 
 template <int B>
 __global__ __launch_bounds__(B) void k_ra_insert(RaArgs a)
 {
-  __shared__ uint32_t take[B / kWave + 1];
-  RaMine mine;
-  ra_insert_step<false, B>(a, blockIdx.x * B + threadIdx.x, take, mine);
-}
-
-__device__ __forceinline__ bool ra_complete(const RaArgs &a, uint32_t cell, unsigned long long acc)
-{
-  return a.ref64 ? ra_bytes(acc) == a.req_size : ra_cnt(acc) == a.want[cell];
-}
-
-// Returns the workgroup's packed (requests, fragments) total.
-template <bool FUSED, int B>
-__device__ __forceinline__ uint64_t ra_flag_step(const RaArgs &a, uint32_t i, uint64_t *wave_tot, RaMine &mine)
-{
+  __shared__ RaLds<B> l;
+  __shared__ unsigned long long wave_new[B / kWave];
+  const uint32_t i0 = blockIdx.x * B, i = i0 + threadIdx.x;
   const uint32_t n = ra_n(a);
-  unsigned long long pack = 0;
-  if (i < n) {
-    const uint32_t cell = FUSED ? mine.cell : a.arr_cell[i];
-    const uint32_t r = cell != kRaNoCell ? a.rec[cell] : kRaNoRec;
-    if (r != kRaNoRec) {
-      const uint32_t fidx = FUSED ? mine.fidx : a.arr_fidx[i];
-      if (fidx < SG_MAX_BI_SIZE) {
-        // rr_emplace_mbuf: the entry goes where its sequence number says
-        a.tab[(size_t)r * SG_MAX_BI_SIZE + fidx] =
-            (unsigned long long)(FUSED ? mine.slot : a.arrivals[i]) | ((unsigned long long)(FUSED ? mine.len : a.arr_len[i]) << 32);
-      } else {
-        refuse(a.status, a.status_flag, kStBadTable);  // beyond what a request's tables hold (src/p2p_bufs.h:10)
-      }
-      const unsigned long long acc = ra_acc<FUSED>(a, cell);
-      const uint32_t cnt = ra_cnt(acc);
-      if (ra_word<FUSED>(a.last + cell) == i && ra_complete(a, cell, acc)) {
-        if (cnt <= SG_MAX_BI_SIZE) pack = (1ull << 32) | cnt;
-        else refuse(a.status, a.status_flag, kStBadTable);
-      }
+  if (i0 >= n) return;  // the whole workgroup
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const bool in_range = i < n;
+  const uint32_t epoch = sload(a.words + kRaEpoch);  // advanced by k_ra_emit, two kernels behind
+  const RaMine m = ra_read(a, i, in_range);
+  ra_lds_clear(l);
+  __syncthreads();
+  const uint32_t hash = ra_hash(m.token);
+  bool owner, claimed = false;
+  const uint32_t e = ra_group<B>(l, m, hash, lane, &owner);
+  __syncthreads();
+  if (owner) {
+    const uint32_t c = ra_find_cell(a, m.token, hash, &claimed);
+    l.cell[e] = c;
+    if (c != kRaNoCell) {
+      atomicAdd(&a.acc[c], l.acc[e]);
+      atomicMax(&a.last[c], i0 + l.last[e]);
+      a.seen[c] = epoch;
+      if (!a.ref64) a.want[c] = m.want;  // every fragment of a request says the same
+    } else {
+      refuse(a.status, a.status_flag, kStPoolFull);  // bucket full
     }
   }
-  uint64_t tot;
-  const uint64_t ex = block_exclusive_scan<B>(pack, wave_tot, &tot);
-  mine.pack = pack ? (ex | (1ull << 63)) : 0;  // top bit: "a request completes here"
-  if (!FUSED && i < n) a.arr_pack[i] = mine.pack;
-  return tot;
+  __syncthreads();
+  const uint32_t cell = m.token ? l.cell[e] : kRaNoCell;
+  if (cell != kRaNoCell) ra_file(a, cell, m);
+  if (in_range) a.arr_cell[i] = cell | (owner ? kRaOwner : 0u);
+  const unsigned long long t = ra_count_new<B>(claimed, in_range && cell == kRaNoCell, lane, wave_new);
+  if (threadIdx.x == 0) a.blk_new[blockIdx.x] = t;
+}
+
+__device__ __forceinline__ bool ra_complete(const RaArgs &a, uint32_t want, unsigned long long acc)
+{
+  return a.ref64 ? ra_bytes(acc) == a.req_size : ra_cnt(acc) == want;
+}
+
+// Whether a complete request of this many fragments can be handed over.
+__device__ __forceinline__ bool ra_fits(const RaArgs &a, uint32_t cnt)
+{
+  if (cnt <= SG_MAX_BI_SIZE) return true;
+  refuse(a.status, a.status_flag, kStBadTable);
+  return false;
 }
 
 template <int B>
 __global__ __launch_bounds__(B) void k_ra_flag(RaArgs a)
 {
   __shared__ uint64_t wave_tot[B / kWave];
-  RaMine mine;
-  const uint64_t tot = ra_flag_step<false, B>(a, blockIdx.x * B + threadIdx.x, wave_tot, mine);
+  const uint32_t i = blockIdx.x * B + threadIdx.x;
+  const uint32_t n = ra_n(a);
+  if (blockIdx.x * B >= n) return;  // the whole workgroup
+  uint64_t mine = 0;
+  if (i < n) {
+    const uint32_t cell = a.arr_cell[i] & ~kRaOwner;
+    if (cell != kRaNoCell) {
+      const unsigned long long acc = a.acc[cell];
+      const uint32_t last = a.last[cell], want = a.want[cell];
+      if (last == i && ra_complete(a, want, acc) && ra_fits(a, ra_cnt(acc)))
+        mine = 1ull << 32 | ra_cnt(acc);
+    }
+  }
+  uint64_t tot;
+  const uint64_t before = block_exclusive_scan<B>(mine, wave_tot, &tot);
+  if (i < n) a.arr_pack[i] = mine ? ra_done((uint32_t)mine, before) : 0ull;
   if (threadIdx.x == 0) a.blk[blockIdx.x] = tot;
 }
 
-// One thread closes the call: counts, the free ring's head, the epoch.  `run` is the packed
-// (requests, fragments) total of the call.  Returns whether the output tables overflowed.
-template <bool FUSED>
-__device__ __forceinline__ uint32_t ra_scan_finish(const RaArgs &a, uint64_t run)
+// Closes the call (one wavefront's lane 0): counts and epoch.  `tot` is the packed (requests,
+// fragments) total of the call, `fresh` the cells claimed << 32 | arrivals dropped.  The kernel's
+// other wavefronts read none of the words written here.
+__device__ __forceinline__ void ra_close(const RaArgs &a, uint64_t tot, unsigned long long fresh, bool overflow)
 {
-  uint32_t n_req = (uint32_t)(run >> 32), n_frag = (uint32_t)run;
-  uint32_t overflow = 0;
-  if (n_req > a.max_req || n_frag > a.max_frag) {
-    // the output tables cannot take what completed: nothing is emitted, the requests stay parked
-    refuse(a.status, a.status_flag, kStBadTable);
-    overflow = 1;
-    n_req = n_frag = 0;
-  }
-  a.words[kRaOverflow] = overflow;
-  // cells claimed since the last call: as far as the head has moved
-  uint32_t head = ra_word<FUSED>(a.words + kRaHead);
-  const uint32_t claims = head - a.words[kRaHeadSeen];
-  // claims beyond the pool ran the head past the tail
-  if ((int32_t)(head - a.words[kRaTail]) > 0) head = a.words[kRaTail];
-  a.words[kRaHead] = head;
-  a.words[kRaHeadSeen] = head;
+  const uint32_t n_req = overflow ? 0u : (uint32_t)(tot >> 32), n_frag = overflow ? 0u : (uint32_t)tot;
+  const uint32_t claims = (uint32_t)(fresh >> 32), before = a.words[kRaInFlight];
+  if (claims && before + claims > a.pool) refuse(a.status, a.status_flag, kStPoolFull);
+  // the output tables cannot take what completed: nothing is emitted, the requests stay parked
+  if (overflow) refuse(a.status, a.status_flag, kStBadTable);
+  const uint32_t in_flight = before + claims - n_req;
   a.req_first[n_req] = n_frag;
-  const uint32_t in_flight = a.words[kRaInFlight] + claims - n_req;
-  const uint32_t dropped = ra_word<FUSED>(a.words + kRaDropped);
   a.words[kRaInFlight] = in_flight;
-  a.words[kRaDropped] = 0;
   a.words[kRaEpoch] += 1;
-  const uint32_t c[4] = {n_req, n_frag, dropped, in_flight};
+  const uint32_t c[4] = {n_req, n_frag, (uint32_t)fresh, in_flight};
   for (int k = 0; k < 4; k++) {
     if (a.counts_out) a.counts_out[k] = c[k];
     a.counts_host[k] = c[k];  // straight into pinned host memory: nothing to copy back
   }
-  return overflow;
 }
 
-// B: this kernel's own workgroup size; a.blk_size: that of the k_ra_flag before it (a total per workgroup).
-template <int B>
-__global__ __launch_bounds__(B) void k_ra_scan(RaArgs a)
+// Empties the cell of a request that has been handed over (its record is empty already).
+__device__ __forceinline__ void ra_free_cell(const RaArgs &a, uint32_t cell)
 {
-  __shared__ uint64_t wave_tot[B / kWave];
-  const uint32_t n = ra_n(a);
-  const uint32_t n_blocks = (n + a.blk_size - 1) / a.blk_size;
-  uint64_t run = 0;
-  for (uint32_t base = 0; base < n_blocks; base += B) {
-    const uint32_t b = base + threadIdx.x;
-    const uint64_t v = b < n_blocks ? a.blk[b] : 0;
-    uint64_t tot;
-    const uint64_t ex = block_exclusive_scan<B>(v, wave_tot, &tot);
-    if (b < n_blocks) a.blk[b] = run + ex;
-    run += tot;
-  }
-  if (threadIdx.x == 0) (void)ra_scan_finish<false>(a, run);
+  a.acc[cell] = 0;
+  __hip_atomic_store(&a.keys[cell], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The wavefront of a completing arrival hands the request over: its record goes
-// into the output tables in sequence order, the record is emptied and returned
-// to the free ring, the cell is emptied.  The request's rank and first fragment
-// index hang on that arrival (arr_pack there plus its workgroup's scanned total).
-template <bool FUSED, int B>
-__device__ __forceinline__ void ra_emit_step(const RaArgs &a, uint32_t i, uint32_t *take, bool overflow, const RaMine &mine)
+// Hands over the requests that complete on this wavefront's lanes: `done` what k_ra_flag left
+// there (0 on the other lanes).  `base` gives the packed (requests, fragments) completed before
+// the wavefront's workgroup, or returns false where nothing is to be handed over after all; it is
+// asked once the first records are on their way.  Every lane of the wavefront calls this.
+template <class Base>
+__device__ __forceinline__ void ra_emit(const RaArgs &a, uint32_t cell, unsigned long long done, uint32_t lane, Base base)
 {
-  const uint32_t n = ra_n(a);
-  const uint32_t lane = threadIdx.x & (kWave - 1);
-  uint32_t cell = kRaNoCell;
-  unsigned long long v = 0;
-  bool completes = false;
-  if (i < n) {
-    cell = FUSED ? mine.cell : a.arr_cell[i];
-    const unsigned long long p = FUSED ? mine.pack : a.arr_pack[i];
-    completes = cell != kRaNoCell && (p >> 63) && !overflow;
-    if (completes) v = (p & ~(1ull << 63)) + (FUSED ? 0ull : a.blk[i / B]);  // one workgroup: nothing before it
-    // the position of a request's last arrival counts per call
-    if (cell != kRaNoCell && !completes) a.last[cell] = 0;
-  }
-  unsigned long long todo = __ballot(completes);
-  // reap_rr for all of this workgroup's requests: one addition to the ring's tail
-  const uint32_t tail0 = ra_block_take<B>(&a.words[kRaTail], (uint32_t)__popcll(todo), take);
   // requests of a few fragments are handed over by the completing lane itself, all such lanes
-  // at once; the wavefront then walks the larger ones together
-  constexpr uint32_t kOwn = 8;
-  const uint32_t my_rank = (uint32_t)__popcll(todo & ((1ull << lane) - 1ull));
-  bool own = false;
-  if (completes) {
-    const uint32_t cnt = ra_cnt(ra_acc<FUSED>(a, cell));
-    own = cnt <= kOwn;
-    if (own) {
-      const uint32_t r = (uint32_t)(v >> 32), first = (uint32_t)v, rc = a.rec[cell];
-      unsigned long long *t = a.tab + (size_t)rc * SG_MAX_BI_SIZE;
-      unsigned long long e[kOwn];
+  // at once; the wavefront then walks the larger ones together, eight entries per lane asked for
+  // before the first is stored
+  constexpr uint32_t kOwn = 8, kAhead = 8;
+  const uint32_t cnt = ra_done_cnt(done);
+  const bool own = done && cnt <= kOwn;
+  unsigned long long todo = __ballot(done && !own);
+  unsigned long long *t = a.tab + (size_t)cell * SG_MAX_BI_SIZE;
+  unsigned long long e[kOwn], f[kAhead];
+  if (own) {
 #pragma unroll
-      for (uint32_t j = 0; j < kOwn; j++) e[j] = j < cnt ? t[j] : 0ull;
-#pragma unroll
-      for (uint32_t j = 0; j < kOwn; j++) {
-        if (j < cnt) {
-          a.frag_slot[first + j] = (uint32_t)e[j];
-          a.frag_len[first + j] = (uint32_t)(e[j] >> 32);
-          t[j] = 0;
-        }
-      }
-      a.req_first[r] = first;
-      if (a.req_token) a.req_token[r] = ra_key(a.keys + cell);
-      if (a.req_hdr_slot) a.req_hdr_slot[r] = (uint32_t)e[0];
-      a.free_ring[(tail0 + my_rank) & a.rmask] = rc;
-      a.acc[cell] = 0;
-      a.last[cell] = 0;
-      a.want[cell] = 0;
-      a.rec[cell] = kRaNoRec;
-      __hip_atomic_store(&a.keys[cell], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    for (uint32_t j = 0; j < kOwn; j++) e[j] = j < cnt ? t[j] : 0ull;
   }
-  const unsigned long long all_done = todo;
-  todo &= ~__ballot(own);
+  auto ask = [&](const unsigned long long *rec, uint32_t k, uint32_t j0) {
+#pragma unroll
+    for (uint32_t q = 0; q < kAhead; q++) {
+      const uint32_t j = j0 + q * kWave + lane;
+      f[q] = j < k ? rec[j] : 0ull;
+    }
+  };
+  if (todo) {
+    const int l = __ffsll((long long)todo) - 1;
+    ask(a.tab + (size_t)(uint32_t)__builtin_amdgcn_readlane((int)cell, l) * SG_MAX_BI_SIZE,
+        (uint32_t)__builtin_amdgcn_readlane((int)cnt, l), 0);
+  }
+  uint64_t before;
+  if (!base(&before)) return;
+  const uint64_t at = before + ra_done_before(done);
+  if (own) {
+    const uint32_t r = (uint32_t)(at >> 32), first = (uint32_t)at;
+#pragma unroll
+    for (uint32_t j = 0; j < kOwn; j++) {
+      if (j < cnt) {
+        a.frag_slot[first + j] = (uint32_t)e[j];
+        a.frag_len[first + j] = (uint32_t)(e[j] >> 32);
+        t[j] = 0;  // a fresh request finds an empty record
+      }
+    }
+    a.req_first[r] = first;
+    if (a.req_token) a.req_token[r] = ra_key(a.keys + cell);
+    if (a.req_hdr_slot) a.req_hdr_slot[r] = (uint32_t)e[0];  // the slot whose header the responses answer
+    ra_free_cell(a, cell);
+  }
+  bool asked = true;
   while (todo) {
     const int l = __ffsll((long long)todo) - 1;
     todo &= todo - 1;
-    const uint32_t nth = (uint32_t)__popcll(all_done & ((1ull << l) - 1ull));
-    const uint32_t c = (uint32_t)__shfl((int)cell, l, kWave);
-    const uint32_t r = (uint32_t)__shfl((int)(uint32_t)(v >> 32), l, kWave);
-    const uint32_t first = (uint32_t)__shfl((int)(uint32_t)v, l, kWave);
-    const uint32_t rc = a.rec[c], cnt = ra_cnt(ra_acc<FUSED>(a, c));
-    unsigned long long *t = a.tab + (size_t)rc * SG_MAX_BI_SIZE;
-    for (uint32_t j = lane; j < cnt; j += kWave) {
-      const unsigned long long e = t[j];
-      a.frag_slot[first + j] = (uint32_t)e;
-      a.frag_len[first + j] = (uint32_t)(e >> 32);
-      t[j] = 0;  // a fresh request finds an empty record
-      if (j == 0) {
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cell, l);
+    const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)cnt, l);
+    const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(at >> 32), l);
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)at, l);
+    unsigned long long *rec = a.tab + (size_t)c * SG_MAX_BI_SIZE;
+    for (uint32_t j0 = 0; j0 < k; j0 += kAhead * kWave) {
+      if (!asked) ask(rec, k, j0);
+      asked = false;
+#pragma unroll
+      for (uint32_t q = 0; q < kAhead; q++) {
+        const uint32_t j = j0 + q * kWave + lane;
+        if (j < k) {
+          a.frag_slot[first + j] = (uint32_t)f[q];
+          a.frag_len[first + j] = (uint32_t)(f[q] >> 32);
+          rec[j] = 0;
+        }
+      }
+      if (j0 == 0 && lane == 0) {
         a.req_first[r] = first;
         if (a.req_token) a.req_token[r] = ra_key(a.keys + c);
-        if (a.req_hdr_slot) a.req_hdr_slot[r] = (uint32_t)e;  // the slot whose header the responses answer
+        if (a.req_hdr_slot) a.req_hdr_slot[r] = (uint32_t)f[0];
+        ra_free_cell(a, c);
       }
-    }
-    if (lane == 0) {
-      // the record goes back to the free ring, the token leaves the table
-      a.free_ring[(tail0 + nth) & a.rmask] = rc;
-      a.acc[c] = 0;
-      a.last[c] = 0;
-      a.want[c] = 0;
-      a.rec[c] = kRaNoRec;
-      __hip_atomic_store(&a.keys[c], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
 }
 
+// Sum over the wavefront of words that hold two counts of 32 bits each (neither sum leaves its half).
+__device__ __forceinline__ uint64_t wave_sum_pairs(uint64_t v)
+{
+  return (uint64_t)wave_sum_uniform((uint32_t)(v >> 32)) << 32 | wave_sum_uniform((uint32_t)v);
+}
+
+// A word per workgroup, `n` of them, added up over the wavefront: all of them, and those before
+// number `upto`.  Eight per lane are asked for before the first is added.
+__device__ __forceinline__ void ra_sum_blocks(const unsigned long long *p, uint32_t n, uint32_t upto, uint32_t lane,
+                                              uint64_t *all, uint64_t *before)
+{
+  uint64_t t = 0, b = 0;
+  for (uint32_t q0 = lane; q0 < n; q0 += 8 * kWave) {
+    uint64_t v[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; k++) v[k] = q0 + k * kWave < n ? p[q0 + k * kWave] : 0ull;
+#pragma unroll
+    for (uint32_t k = 0; k < 8; k++) {
+      t += v[k];
+      b += q0 + k * kWave < upto ? v[k] : 0ull;
+    }
+  }
+  *all = wave_sum_pairs(t);
+  *before = wave_sum_pairs(b);
+}
+
+// B: the workgroup size of this kernel and of the two before it (a total per workgroup).
 template <int B>
 __global__ __launch_bounds__(B) void k_ra_emit(RaArgs a)
 {
-  __shared__ uint32_t take[B / kWave + 1];
-  ra_emit_step<false, B>(a, blockIdx.x * B + threadIdx.x, take, a.words[kRaOverflow] != 0, RaMine());
+  const uint32_t n = ra_n(a);
+  const uint32_t i = blockIdx.x * B + threadIdx.x;
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const bool closer = __builtin_amdgcn_readfirstlane(i / kWave) == 0;
+  unsigned long long done = 0;
+  uint32_t cell = kRaNoCell;
+  if (i < n) {
+    done = a.arr_pack[i];
+    const uint32_t oc = a.arr_cell[i];
+    cell = oc & ~kRaOwner;
+    if ((oc & kRaOwner) && cell != kRaNoCell) a.last[cell] = 0;  // the position counts per call
+  }
+  if (!__any(done != 0) && !closer) return;
+  // What completed in the workgroups before this one, and in all of them: every wavefront that
+  // has something to hand over adds the few hundred totals up by itself.
+  const uint32_t n_blocks = (n + B - 1) / B;
+  ra_emit(a, cell, done, lane, [&](uint64_t *base) {
+    uint64_t tot;
+    ra_sum_blocks(a.blk, n_blocks, blockIdx.x, lane, &tot, base);
+    const bool overflow = (uint32_t)(tot >> 32) > a.max_req || (uint32_t)tot > a.max_frag;
+    if (closer) {
+      uint64_t fresh, none;
+      ra_sum_blocks(a.blk_new, n_blocks, 0, lane, &fresh, &none);
+      if (lane == 0) ra_close(a, tot, fresh, overflow);
+    }
+    return !overflow;
+  });
 }
 
-// A burst of at most kRaTakeBlock arrivals: the four steps by one workgroup in one launch.
-static_assert(kRaTakeBlock == kRaBlock, "one workgroup size for all steps of a burst");
-__global__ __launch_bounds__(kRaTakeBlock) void k_ra_burst(RaArgs a)
+// A burst that one workgroup takes, which is what a NIC delivers: the three steps in ONE kernel.
+// Nothing else touches the table meanwhile, so the owner of a token works on its cell with
+// ordinary loads and stores and hands the new total to the token's other arrivals through LDS.
+template <int B>
+__global__ __launch_bounds__(B) void k_ra_burst(RaArgs a)
 {
-  __shared__ uint32_t take[kRaTakeBlock / kWave + 1];
-  __shared__ uint64_t wave_tot[kRaBlock / kWave];
-  __shared__ uint32_t overflow;
+  __shared__ RaLds<B> l;
+  __shared__ unsigned long long wave_new[B / kWave];
+  __shared__ uint64_t wave_tot[B / kWave];
   const uint32_t i = threadIdx.x;
-  RaMine mine;
-  ra_insert_step<true, kRaTakeBlock>(a, i, take, mine);
+  const uint32_t n = ra_n(a);
+  const uint32_t lane = i & (kWave - 1);
+  const bool in_range = i < n;
+  const uint32_t epoch = a.words[kRaEpoch];
+  const RaMine m = ra_read(a, i, in_range);
+  ra_lds_clear(l);
   __syncthreads();
-  const uint64_t tot = ra_flag_step<true, kRaBlock>(a, i, wave_tot, mine);
-  if (threadIdx.x == 0) overflow = ra_scan_finish<true>(a, tot);
+  const uint32_t hash = ra_hash(m.token);
+  bool owner, claimed = false;
+  const uint32_t e = ra_group<B>(l, m, hash, lane, &owner);
   __syncthreads();
-  ra_emit_step<true, kRaTakeBlock>(a, i, take, overflow != 0, mine);
+  if (owner) {
+    const uint32_t c = ra_find_cell(a, m.token, hash, &claimed);
+    l.cell[e] = c;
+    if (c != kRaNoCell) {
+      const unsigned long long acc = (claimed ? 0ull : a.acc[c]) + l.acc[e];  // an empty cell's total is zero
+      a.acc[c] = acc;
+      l.acc[e] = acc;
+      a.seen[c] = epoch;
+    } else {
+      refuse(a.status, a.status_flag, kStPoolFull);  // bucket full
+    }
+  }
+  __syncthreads();
+  const uint32_t cell = m.token ? l.cell[e] : kRaNoCell;
+  uint64_t mine = 0;
+  if (cell != kRaNoCell) {
+    ra_file(a, cell, m);
+    const unsigned long long acc = l.acc[e];
+    if (l.last[e] == i && ra_complete(a, m.want, acc) && ra_fits(a, ra_cnt(acc))) mine = 1ull << 32 | ra_cnt(acc);
+  }
+  uint64_t tot;
+  const uint64_t before = block_exclusive_scan<B>(mine, wave_tot, &tot);
+  // (its barriers also stand between the entries filed above and the records read below)
+  const bool overflow = (uint32_t)(tot >> 32) > a.max_req || (uint32_t)tot > a.max_frag;
+  const unsigned long long fresh = ra_count_new<B>(claimed, in_range && cell == kRaNoCell, lane, wave_new);
+  if (i == 0) ra_close(a, tot, fresh, overflow);
+  ra_emit(a, cell, mine ? ra_done((uint32_t)mine, before) : 0ull, lane, [&](uint64_t *base) {
+    *base = 0;
+    return !overflow;
+  });
 }
 
-// Empties the table: every cell, every record, all records back in the ring.
-__global__ __launch_bounds__(256) void k_ra_reset(RaArgs a, uint32_t cells, uint32_t records)
+// Empties the table: every cell, every record.
+__global__ __launch_bounds__(256) void k_ra_reset(RaArgs a, uint32_t cells)
 {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i < cells) {
     a.keys[i] = 0;
     a.acc[i] = 0;
-    a.want[i] = a.last[i] = a.seen[i] = 0;
-    a.rec[i] = kRaNoRec;
+    a.last[i] = a.want[i] = a.seen[i] = 0;
   }
-  if (i < records) a.free_ring[i] = (uint32_t)i;
-  if (i < (size_t)records * SG_MAX_BI_SIZE) a.tab[i] = 0;
-  if (i < kRaWords) a.words[i] = i == kRaTail ? records : 0u;
+  // two entries per thread
+  if (2 * i < (size_t)cells * SG_MAX_BI_SIZE) reinterpret_cast<u32x4 *>(a.tab)[i] = (u32x4){0u, 0u, 0u, 0u};
+  if (i < kRaWords) a.words[i] = 0;
 }
 
 // Drops the requests no fragment has come in for during the last max_age calls
@@ -604,20 +658,10 @@ __global__ __launch_bounds__(256) void k_ra_evict(RaArgs a, uint32_t cells, uint
   if (c >= cells) return;
   if (a.keys[c] == 0ull) return;
   if (a.words[kRaEpoch] - a.seen[c] <= max_age) return;
-  const uint32_t rc = a.rec[c];
-  if (rc != kRaNoRec) {
-    unsigned long long *t = a.tab + (size_t)rc * SG_MAX_BI_SIZE;
-    for (uint32_t j = lane; j < SG_MAX_BI_SIZE; j += kWave) t[j] = 0;
-  }
+  unsigned long long *t = a.tab + (size_t)c * SG_MAX_BI_SIZE;
+  for (uint32_t j = lane; j < SG_MAX_BI_SIZE; j += kWave) t[j] = 0;
   if (lane == 0) {
-    if (rc != kRaNoRec) {
-      const uint32_t tl = atomicAdd(&a.words[kRaTail], 1u);
-      a.free_ring[tl & a.rmask] = rc;
-    }
     a.acc[c] = 0;
-    a.last[c] = 0;
-    a.want[c] = 0;
-    a.rec[c] = kRaNoRec;
     a.keys[c] = 0;
     atomicSub(&a.words[kRaInFlight], 1u);
     atomicAdd(&a.words[kRaEvicted], 1u);
