@@ -273,9 +273,13 @@ class SgContext:
     def reassemble_raw(self, a: capi.ReassembleArgs):
         """Returns (requests completed, their fragments, arrivals dropped,
         requests still in flight); all zero for an SG_F_ASYNC call."""
+        if a.flags & capi.F_ASYNC:  # the counts stay on the device
+            rc = self.lib.sg_hip_reassemble(self.h, C.byref(a), None)
+            if rc != capi.SG_OK:
+                self._check(rc)
+            return (0, 0, 0, 0)
         counts = (C.c_uint32 * 4)()
-        if not (a.flags & capi.F_ASYNC):
-            self._after_torch()
+        self._after_torch()
         rc = self.lib.sg_hip_reassemble(self.h, C.byref(a), C.byref(counts))
         if rc != capi.SG_OK:
             self._check(rc)
