@@ -32,11 +32,6 @@ __device__ __forceinline__ uint32_t load32_any(const uint8_t *p)
 {
   return reinterpret_cast<const u32_unaligned *>(p)->v;
 }
-struct __attribute__((packed, aligned(1))) u32x4_unaligned { u32x4 v; };
-__device__ __forceinline__ u32x4 load128_any(const uint8_t *p)
-{
-  return reinterpret_cast<const u32x4_unaligned *>(p)->v;
-}
 
 // Payload chunks are touched once: read from a ring slot, written to a tensor
 // (or the other way round) and not looked at again by this library.  The

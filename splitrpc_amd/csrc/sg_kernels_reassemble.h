@@ -241,6 +241,12 @@ __device__ __forceinline__ uint32_t ra_lds_entry(RaLds<B> &l, unsigned long long
   }
 }
 
+struct __attribute__((packed, aligned(1))) u32x4_unaligned { u32x4 v; };
+__device__ __forceinline__ u32x4 load128_any(const uint8_t *p)
+{
+  return reinterpret_cast<const u32x4_unaligned *>(p)->v;
+}
+
 // An arrival as its thread knows it.
 struct RaMine {
   uint32_t slot = 0, len = 0, fidx = 0, want = 0;
