@@ -320,10 +320,9 @@ int launch_prep(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const PrepArgs
 
 // Behind the copy kernel: advance the cursor (single-kernel calls on a packed
 // arena) and publish slot states (where the caller keeps a slot ring).
-void launch_finish(const Scratch &sc, hipStream_t st, uint64_t *cursor, uint64_t size, uint64_t cap, uint32_t n_req,
-                   const uint32_t *counts, uint32_t *state, uint32_t n_states, int which, bool all_or_nothing)
+FinishArgs finish_args(const Scratch &sc, uint64_t *cursor, uint64_t size, uint64_t cap, uint32_t n_req, const uint32_t *counts,
+                       uint32_t *state, uint32_t n_states, int which, bool all_or_nothing)
 {
-  if (!cursor && !state) return;
   FinishArgs f;
   memset(&f, 0, sizeof f);
   f.cursor = cursor;
@@ -342,7 +341,16 @@ void launch_finish(const Scratch &sc, hipStream_t st, uint64_t *cursor, uint64_t
   f.all_or_nothing = all_or_nothing ? 1u : 0u;
   f.status = sc.status;
   f.status_flag = sc.flag;
-  k_finish<<<1, kBlock, 0, st>>>(f);
+  return f;
+}
+
+void launch_finish(const Scratch &sc, hipStream_t st, uint64_t *cursor, uint64_t size, uint64_t cap, uint32_t n_req,
+                   const uint32_t *counts, uint32_t *state, uint32_t n_states, int which, bool all_or_nothing)
+{
+  if (!cursor && !state) return;
+  FinishPair p;
+  p.h[0] = p.h[1] = finish_args(sc, cursor, size, cap, n_req, counts, state, n_states, which, all_or_nothing);
+  k_finish<<<1, kBlock, 0, st>>>(p);
 }
 
 int finish(sg_hip_ctx *c, uint32_t flags)
@@ -493,14 +501,16 @@ static void launch_gather_rule(hipStream_t st, const GatherRuleArgs &ga, uint32_
   }
 }
 
-// One direction's share of a launch that carries both (sg_hip_shunt_batch).
+// What the two directions bring to a launch that carries both (sg_hip_shunt_batch).
 struct ShuntHalf {
-  GatherRuleArgs g;
-  ScatterArgs s;
-  uint32_t g_grid = 0, s_grid = 0;
-  uint32_t g_small = 0;  // lanes of the gather's short last fragments (0: none)
-  uint32_t s_small = 0;  // lanes of the scatter's frames when all are short (0: a wavefront each)
+  ShuntArgs sh;
+  uint32_t g_grid = 0, s_grid = 0, s_small_grid = 0;  // workgroups
   bool full_csum = false;
+  // the cursor of a packed arena ([0] gather, [1] scatter; nullptr: tensor-major), and whether a
+  // launch of its own would advance it itself
+  uint64_t *cursor[2] = {nullptr, nullptr};
+  bool self[2] = {false, false};
+  FinishArgs fin[2];
 };
 constexpr int kNoShare = 1;  // the call needs kernels of its own
 
@@ -938,13 +948,20 @@ static int gather_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const s
               (app.n_tensors > 1 ? kOptMultiTensor : 0u) | (small_last ? kOptSmallLast : 0u) |
               ((((uintptr_t)a->ring.base | a->ring.slot_size) & 15u) ? 0u : kOptHdrChunk);
     if (half) {
-      // one wavefront per fragment (short last fragments may ride along), the cursor advanced by the
-      // kernel itself: the shapes k_shunt carries
-      if (!self_advance || small_all || ga.pieces != 1) return kNoShare;
-      ga.call_seq = ++*sc.call_seq;
-      half->g = ga;
+      if (a->slot_state) return kNoShare;
+      half->sh.g = ga;
+      const uint32_t lng = ga.pieces > 1 ? 1u : 0u;
+      if (small_all) {
+        const uint32_t per_group = kWave / small_all * kWavesPerBlock;
+        grid = (n_items + per_group - 1) / per_group;
+        half->sh.g_kind = small_all == 8 ? kShuntSmall8 : small_all == 16 ? kShuntSmall16 : kShuntSmall32;
+      } else {
+        half->sh.g_kind = (small_last == 16 ? kShuntFull16 : small_last == 32 ? kShuntFull32 : kShuntFull) + lng;
+      }
       half->g_grid = grid;
-      half->g_small = small_last;
+      half->cursor[0] = packed ? sc.cursor[0] : nullptr;
+      half->self[0] = self_advance;
+      half->fin[0] = finish_args(sc, half->cursor[0], a->fixed_req_size, app.cap, a->n_req, a->counts, nullptr, 0, 0, false);
       return SG_OK;
     }
     if (self_advance) ga.call_seq = ++*sc.call_seq;
@@ -1126,18 +1143,27 @@ static int scatter_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const 
     const bool self_advance = self_advancing(sc, packed, a->slot_state, (uint64_t)n_items * sa.pieces, a->flags);
     sa.rule.cursor = const_cast<uint64_t *>(plain_cursor(sc, 1));
     if (half) {
-      // one kernel that advances the cursor itself: a wavefront per frame, or eight short frames to a wavefront
-      const bool own_small_launch = !small_all && small_last;
-      if (!self_advance || own_small_launch || sa.pieces != 1 || (small_all && (small_all != 8 || full_csum)))
-        return kNoShare;
-      sa.rule.call_seq = ++*sc.call_seq;
+      const bool defer = csum_in_two_phases(sc, sa.pieces, full_csum);
+      if (a->slot_state || (full_csum && sa.pieces > 1 && !small_all && !defer)) return kNoShare;
+      if (small_last) sa.rule.per_launch = (uint32_t)per - 1;
       magic_div(sa.rule.per_launch, &sa.rule.lmul, &sa.rule.lshift);
-      if (small_all) grid = (n_items + 8 * kWavesPerBlock - 1) / (8 * kWavesPerBlock);
-      else geometry((uint64_t)n_items, !(a->flags & SG_F_NO_XCD_REMAP), &grid, &sa.remap);
-      half->s = sa;
-      half->s_grid = grid;
-      half->s_small = small_all;
+      if (defer) {
+        sa.csum_part = sc.csum_part;
+        sa.csum_valid = sc.csum_valid;
+      }
+      const uint32_t lanes = small_all ? small_all : small_last;
+      half->sh.s_lanes = lanes;
+      if (lanes) {
+        const uint32_t per_group = kWave / lanes * kWavesPerBlock;
+        half->s_small_grid = ((small_all ? n_items : a->n_req) + per_group - 1) / per_group;
+      }
+      if (!small_all) geometry((uint64_t)a->n_req * sa.rule.per_launch * sa.pieces, !(a->flags & SG_F_NO_XCD_REMAP), &half->s_grid, &sa.remap);
+      half->sh.s = sa;
+      half->sh.s_long = !small_all && sa.pieces > 1;
       half->full_csum = full_csum;
+      half->cursor[1] = packed ? sc.cursor[1] : nullptr;
+      half->self[1] = self_advance;
+      half->fin[1] = finish_args(sc, half->cursor[1], a->fixed_resp_size, app.cap, a->n_req, a->counts, nullptr, 0, 1, false);
       return SG_OK;
     }
     if (self_advance) sa.rule.call_seq = ++*sc.call_seq;
@@ -1315,43 +1341,64 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
   // Both halves are looked at before either is launched: a call the host refuses launches nothing.
   // A half that cannot share a launch leaves no trace; both are then made as calls of their own.
   ShuntHalf h;
-  const uint32_t seq0 = c->call_seq;
   const int rg = gather_impl(c, c->sc, c->stream, g, &h);
   if (rg < 0) return rg;
   const int rs = scatter_impl(c, c->sc, c->stream, s, &h);
   if (rs < 0) return rs;
-  // a shared launch pays while the chip holds the whole call at once (one resnet50-sized batch 8.9 ->
-  // 7.8 us per step, two batches 10.9 -> 11.5 us)
-  constexpr uint32_t kAtOnce = 2048;  // workgroups of 256 threads resident on 256 CUs
-  if (apart && rg == SG_OK && rs == SG_OK && h.g_grid + h.s_grid <= kAtOnce) {
-    ShuntArgs sh;
-    sh.g = h.g;
-    sh.s = h.s;
-    sh.s_blocks = h.s_grid;
-    const uint32_t total = h.g_grid + h.s_grid;
+  if (apart && rg == SG_OK && rs == SG_OK) {
+    ShuntArgs &sh = h.sh;
+    // the kernel advances the cursors itself where each half's own would; a workgroup for either
+    // direction behind it does otherwise
+    const bool adv = (h.cursor[0] || h.cursor[1]) && (!h.cursor[0] || h.self[0]) && (!h.cursor[1] || h.self[1]);
+    if (adv) {
+      sh.g.call_seq = ++c->call_seq;
+      sh.s.rule.call_seq = ++c->call_seq;
+    }
+    sh.s_small_end = h.s_small_grid;
+    sh.s_end = sh.s_small_end + h.s_grid;
+    const uint32_t total = sh.s_end + h.g_grid;
     int rc = prof_begin(c, 1);
     if (rc != SG_OK) return rc;
     const hipStream_t st = c->stream;
-#define SG_SHUNT(G, S, C) k_shunt<G, S, C><<<total, kBlock, 0, st>>>(sh)
-    if (h.s_small) {
-      if (h.g_small == 16) SG_SHUNT(16, 8, false);
-      else if (h.g_small == 32) SG_SHUNT(32, 8, false);
-      else SG_SHUNT(0, 8, false);
-    } else if (h.full_csum) {
-      if (h.g_small == 16) SG_SHUNT(16, 0, true);
-      else if (h.g_small == 32) SG_SHUNT(32, 0, true);
-      else SG_SHUNT(0, 0, true);
-    } else {
-      if (h.g_small == 16) SG_SHUNT(16, 0, false);
-      else if (h.g_small == 32) SG_SHUNT(32, 0, false);
-      else SG_SHUNT(0, 0, false);
-    }
+    // (8192 requests of 3136 bytes, five rounds of resident wavefronts: 14.5 us through k_shunt, 15.0 through k_shunt_any)
+    const bool g_plain = sh.g_kind == kShuntFull || sh.g_kind == kShuntFull16 || sh.g_kind == kShuntFull32;
+    const bool s_plain = sh.s_small_end == 0 ? !sh.s_long : sh.s_small_end == sh.s_end && sh.s_lanes == 8 && !h.full_csum;
+    if (adv && g_plain && s_plain) {
+#define SG_SHUNT(S, C)                                                                       \
+  do {                                                                                       \
+    if (sh.g_kind == kShuntFull16) k_shunt<16, S, C><<<total, kBlock, 0, st>>>(sh);          \
+    else if (sh.g_kind == kShuntFull32) k_shunt<32, S, C><<<total, kBlock, 0, st>>>(sh);     \
+    else k_shunt<0, S, C><<<total, kBlock, 0, st>>>(sh);                                     \
+  } while (0)
+      if (sh.s_small_end) SG_SHUNT(8, false);
+      else if (h.full_csum) SG_SHUNT(0, true);
+      else SG_SHUNT(0, false);
 #undef SG_SHUNT
+    } else if (h.full_csum && adv) {
+      k_shunt_any<true, true><<<total, kBlock, 0, st>>>(sh);
+    } else if (h.full_csum) {
+      k_shunt_any<true, false><<<total, kBlock, 0, st>>>(sh);
+    } else if (adv) {
+      k_shunt_any<false, true><<<total, kBlock, 0, st>>>(sh);
+    } else {
+      k_shunt_any<false, false><<<total, kBlock, 0, st>>>(sh);
+    }
+    if (h.full_csum && sh.s_long) k_udp_finish<true><<<(sh.s.n_items + kBlock - 1) / kBlock, kBlock, 0, st>>>(sh.s);
     rc = prof_end(c);
     if (rc != SG_OK) return rc;
+    if (!adv && (h.cursor[0] || h.cursor[1])) {
+      FinishPair p;
+      uint32_t n = 0;
+      for (int k = 0; k < 2; k++) {
+        if (!h.cursor[k]) continue;
+        h.fin[k].clamp = h.self[k] ? 1u : 0u;  // as in the call of its own
+        p.h[n++] = h.fin[k];
+      }
+      if (n == 1) p.h[1] = p.h[0];
+      k_finish<<<n, kBlock, 0, st>>>(p);
+    }
     return finish(c, async);
   }
-  c->call_seq = seq0;
   int rc = gather_impl(c, c->sc, c->stream, g);
   if (rc != SG_OK) return rc;
   return scatter_impl(c, c->sc, c->stream, s);

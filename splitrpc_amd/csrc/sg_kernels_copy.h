@@ -44,7 +44,7 @@ __device__ __forceinline__ uint32_t item_of_wave(bool remap, uint32_t block)
 struct FinishArgs {
   uint64_t *cursor;       // advanced by n_req * size modulo cap; nullptr: nothing to advance
   uint32_t cursor_cells;  // the cursor is a context's pair of cells, not a plain word
-  uint32_t pad;
+  uint32_t clamp;         // a device-resident count beyond n_req is cut to it and not refused
   uint64_t size;
   uint64_t cap;
   uint32_t n_req;         // requests of the call, or their upper bound with `counts`
@@ -61,14 +61,20 @@ struct FinishArgs {
   volatile uint32_t *status_flag;
 };
 
-__global__ __launch_bounds__(kBlock) void k_finish(FinishArgs a)
+// A launch that carried both directions is followed by one with a workgroup for either.
+struct FinishPair {
+  FinishArgs h[2];
+};
+
+__global__ __launch_bounds__(kBlock) void k_finish(FinishPair p)
 {
+  const FinishArgs &a = blockIdx.x ? p.h[1] : p.h[0];
   const uint32_t refused = *a.status;  // what earlier kernels left
   __syncthreads();                     // read by every thread before this kernel adds to it
   uint32_t n = a.n_req;
   if (a.counts) {
     const uint32_t v = sload(a.counts);
-    if (v > n && threadIdx.x == 0) refuse(a.status, a.status_flag, kStBadSize);  // the launch was sized for fewer
+    if (v > n && !a.clamp && threadIdx.x == 0) refuse(a.status, a.status_flag, kStBadSize);  // the launch was sized for fewer
     n = v < n ? v : n;
   }
   if (a.all_or_nothing && refused) return;
@@ -1018,8 +1024,10 @@ __global__ __launch_bounds__(kBlock) void k_udp_finish(ScatterArgs a)
 // == rule.per_req) or the last frame of every response (the remainder; the full
 // frames then go through k_scatter).  Addressing is per lane, the header is two
 // 16-bit words per lane, sums are row reductions.
+// `may_advance`: wavefront 0 is the one of the launch that advances a self-advancing cursor (where the
+// same launch moves the full frames, theirs does).
 template <int L, bool FULL_CSUM, bool ADV>
-__device__ __forceinline__ void scatter_small_wave(const ScatterArgs &a, uint32_t wave, size_t kernarg_base = 0)
+__device__ __forceinline__ void scatter_small_wave(const ScatterArgs &a, uint32_t wave, bool may_advance, size_t kernarg_base = 0)
 {
   constexpr uint32_t G = kWave / L;
   // every argument of the common path in one burst of scalar loads (left to their first uses they
@@ -1072,7 +1080,7 @@ __device__ __forceinline__ void scatter_small_wave(const ScatterArgs &a, uint32_
     uint32_t cur_live = 0;
     if (ADV) c0 = cursor_take(a.rule.cursor - kCurPlain, a.rule.call_seq, &cur_live, &cur_stamp);
     if (c0 >= a.app.cap) c0 %= a.app.cap;  // only after a set_cursor beyond the capacity
-    if (ADV && wave == 0 && lane == 0)
+    if (ADV && may_advance && wave == 0 && lane == 0)
       cursor_advance(a.rule.cursor - kCurPlain, a.rule.call_seq, cur_live, cur_stamp, cursor_bump(c0, n_req, a.rule.size, a.app.cap));
     uint64_t o = c0 + (uint64_t)r * a.rule.size;
     if (a.rule.single_wrap) o = o >= a.app.cap ? o - a.app.cap : o;
@@ -1146,38 +1154,91 @@ __device__ __forceinline__ void scatter_small_wave(const ScatterArgs &a, uint32_
 template <int L, bool FULL_CSUM, bool ADV>
 __global__ __launch_bounds__(kBlock) void k_scatter_small(ScatterArgs a)
 {
-  scatter_small_wave<L, FULL_CSUM, ADV>(a, blockIdx.x * kWavesPerBlock + threadIdx.x / kWave);
+  scatter_small_wave<L, FULL_CSUM, ADV>(a, blockIdx.x * kWavesPerBlock + threadIdx.x / kWave, true);
 }
 
 // One pass of the shunter's loop (src/splitrpc_server/p2p_rpc_dpdk_server.cc:117-189) in ONE
-// launch: the first s_blocks workgroups scatter the responses that are done (one response size),
-// the others gather the requests that became ready (declared rule), each half exactly as the
-// kernel of its own would.  Both halves advance their cursors themselves.  For calls that the chip
-// holds at once (a batch or two) a launch costs more than the bytes it moves; this halves the
-// launches of a step.  The scatter's wavefronts live longest (a header to fetch, rewrite and store
-// besides the payload) and are few: their workgroups come first, so that they end with the others,
-// not after.  (Larger calls lose by sharing a launch -- 8 resnet50-sized batches 30.2 -> 32.2 us
-// per step, 2048 lenet-sized ones 86.4 -> 96.9 us, wherever in the grid the scatter's workgroups
-// are put: first, or spread through the gather's in groups of eight, one per XCD -- and are made
-// as two calls on a stream each.)
-// G_SMALL: the gather's short last fragments go SMALL lanes each (gather_rule_body); S_SMALL: all
-// of the scatter's frames are short and go S_SMALL lanes each (scatter_small_wave).
+// launch: first the workgroups that scatter the responses that are done (one response size: short
+// frames, then the others), then those that gather the requests that became ready (declared rule),
+// every workgroup exactly as in the kernel of its own.
+//
+// What it is for: a kernel that follows another on a stream starts when the last wavefront of that
+// one has ended, so every launch costs a drained chip, 3 to 5 us; kernels of one call have no order
+// among themselves.  One pass on a stream, a launch per kind of wavefront -> one launch, us:
+//   8192 requests of 3136 bytes, 40 back        18.4 -> 15.0
+//   512 of 602112, 4000 back                   108.8 -> 103.6
+//   131072 of 2048, 3072 back                  284.7 -> 275.2
+//   four bursts of 32768 of the last, with the reassembly in front of each      460 -> 423
+// The scatter's wavefronts live longest (a header to fetch, rewrite and store besides the payload):
+// their workgroups come first, so that they end with the others, not after.
 struct alignas(64) ShuntArgs {
   GatherRuleArgs g;
   ScatterArgs s;
-  uint32_t s_blocks;
+  // workgroups: [0, s_small_end) short frames, [.., s_end) the other frames, behind them the gather
+  uint32_t s_small_end, s_end;
+  uint32_t s_lanes;  // lanes per short frame (8, 16, 32)
+  uint32_t s_long;   // frames of several wavefronts
+  uint32_t g_kind;   // kShunt* below
 };
+// All fragments short, this many lanes each; a wavefront per fragment (Long: per piece of one), with
+// remainders of 16 or 32 lanes each dealt in where a number says so.
+enum { kShuntSmall8 = 0, kShuntSmall16, kShuntSmall32, kShuntFull, kShuntLong, kShuntFull16, kShuntLong16, kShuntFull32, kShuntLong32 };
 
+// The shapes a call of a batch or two comes in, each compiled by itself: a wavefront's walk from
+// its arguments to its stores is most of such a call, and is shorter where nothing is chosen at run
+// time and every argument comes in one burst (32 requests of 3136 bytes 5.2 us per pass, 6.2 us
+// through k_shunt_any; 16 of 602112 bytes 7.15 and 7.4 us).
+// G_SMALL: the gather's short last fragments go SMALL lanes each (gather_rule_body); S_SMALL: all
+// of the scatter's frames are short and go S_SMALL lanes each (scatter_small_wave).
 template <int G_SMALL, int S_SMALL, bool FULL_CSUM>
 __global__ __launch_bounds__(kBlock) void k_shunt(ShuntArgs a)
 {
   const uint32_t b = blockIdx.x;
-  if (b >= a.s_blocks) {
-    gather_rule_body<false, G_SMALL, true>(a.g, b - a.s_blocks, offsetof(ShuntArgs, g));
+  if (b >= a.s_end) {
+    gather_rule_body<false, G_SMALL, true>(a.g, b - a.s_end, offsetof(ShuntArgs, g));
   } else if (S_SMALL) {
-    scatter_small_wave<(S_SMALL ? S_SMALL : 8), FULL_CSUM, true>(a.s, b * kWavesPerBlock + threadIdx.x / kWave, offsetof(ShuntArgs, s));
+    scatter_small_wave<(S_SMALL ? S_SMALL : 8), FULL_CSUM, true>(a.s, b * kWavesPerBlock + threadIdx.x / kWave, true, offsetof(ShuntArgs, s));
   } else {
     scatter_body<FULL_CSUM, true, false, false, true>(a.s, b, offsetof(ShuntArgs, s));
+  }
+}
+
+// Every other shape, chosen by the workgroup.  ADV: the kernel takes both cursors from the context's
+// cells and advances them itself; else k_finish follows.  (Eight wavefronts per SIMD: left to itself
+// the compiler takes 104 scalar registers here, which is seven.)
+template <bool FULL_CSUM, bool ADV>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_shunt_any(ShuntArgs)
+{
+  // the argument where it lies: with this many uses of its parts a by-value copy goes to private memory
+  const ShuntArgs &a = *(const ShuntArgs *)(const __attribute__((address_space(4))) ShuntArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr size_t kS = offsetof(ShuntArgs, s), kG = offsetof(ShuntArgs, g);
+  const uint32_t b = blockIdx.x;
+  if (b < a.s_end) {
+    if (b < a.s_small_end) {
+      const uint32_t wave = b * kWavesPerBlock + threadIdx.x / kWave;
+      const bool alone = a.s_small_end == a.s_end;  // else the others' wavefront 0 advances the cursor
+      if (a.s_lanes == 8) scatter_small_wave<8, FULL_CSUM, ADV>(a.s, wave, alone, kS);
+      else if (a.s_lanes == 16) scatter_small_wave<16, FULL_CSUM, ADV>(a.s, wave, alone, kS);
+      else scatter_small_wave<32, FULL_CSUM, ADV>(a.s, wave, alone, kS);
+    } else if (a.s_long) {
+      scatter_body<FULL_CSUM, true, true, FULL_CSUM, ADV>(a.s, b - a.s_small_end, kS);
+    } else {
+      scatter_body<FULL_CSUM, true, false, false, ADV>(a.s, b - a.s_small_end, kS);
+    }
+    return;
+  }
+  const uint32_t gb = b - a.s_end;
+  const uint32_t gwave = gb * kWavesPerBlock + threadIdx.x / kWave;
+  switch (a.g_kind) {
+    case kShuntSmall8: gather_small_wave<8, ADV>(a.g, gwave, true, kG); break;
+    case kShuntSmall16: gather_small_wave<16, ADV>(a.g, gwave, true, kG); break;
+    case kShuntSmall32: gather_small_wave<32, ADV>(a.g, gwave, true, kG); break;
+    case kShuntFull: gather_rule_body<false, 0, ADV>(a.g, gb, kG); break;
+    case kShuntLong: gather_rule_body<true, 0, ADV>(a.g, gb, kG); break;
+    case kShuntFull16: gather_rule_body<false, 16, ADV>(a.g, gb, kG); break;
+    case kShuntLong16: gather_rule_body<true, 16, ADV>(a.g, gb, kG); break;
+    case kShuntFull32: gather_rule_body<false, 32, ADV>(a.g, gb, kG); break;
+    default: gather_rule_body<true, 32, ADV>(a.g, gb, kG); break;
   }
 }
 

@@ -2,9 +2,9 @@
 ONE launch where the two calls can share one -- against the CPU oracle's
 gather followed by its scatter, bit for bit, through the C ABI: arenas, TX
 ring, offsets and both bump-ring cursors, over calls in a row and over graph
-replays.  Pairs of calls that cannot share a launch (long frames, short-frame
-kernels, tensors against an arena, an echo answered in place) must come out the
-same through the two-call path the entry point then takes."""
+replays.  Pairs of calls that cannot share a launch (sizes that differ, an
+echo answered in place) must come out the same through the two-call path the
+entry point then takes, and so must tensors and larger calls either way."""
 import numpy as np
 import pytest
 import torch
@@ -41,7 +41,7 @@ SHARED = {
     "one-request": lambda p: synth.make_custom([1400 * 9 + 1], [1400], seed=73, profile=p),
     # short last fragments riding in the gather's half, eight short frames to a wavefront in the scatter's
     "lenet-9": lambda p: synth.make_workload(1, 9, profile=p),
-    "lenet-1500": lambda p: synth.make_workload(1, 1500, profile=p),   # 6128 wavefronts: the most that shares
+    "lenet-1500": lambda p: synth.make_workload(1, 1500, profile=p),   # 6128 wavefronts
 }
 
 
@@ -84,13 +84,13 @@ def test_one_launch_moves_what_two_calls_move(name, profile):
 
 
 APART = {
-    # (workload, why the two calls keep kernels of their own)
+    # (workload, what it is about)
     "jumbo": lambda: synth.make_workload(5, 1),                     # frames of several wavefronts
     "short-frames-16-lanes": lambda: synth.make_custom([300] * 50, [300] * 50, seed=78),  # short frames, 16 lanes each
     "bert": lambda: synth.make_workload(3, 20),                     # tensors; short last fragments
     "mixed-echo": lambda: synth.make_workload(4, 50),               # variable sizes, answered in place
     "sizes-differ": lambda: synth.make_custom([4200] * 12, [100 + 333 * k for k in range(12)], seed=74),
-    # more wavefronts than the chip holds at once: faster as two calls
+    # more wavefronts than the chip holds at once
     "lenet-4096": lambda: synth.make_workload(1, 4096),
     "two-frames-3000": lambda: synth.make_custom([4200] * 3000, [2800] * 3000, seed=77, flags=synth.F_UDP_CSUM_PSEUDO),
 }
@@ -125,6 +125,63 @@ def test_pairs_that_cannot_share_a_launch_take_two(name):
     if dw.resp_offsets is not None:
         assert np.array_equal(dw.resp_offsets.cpu().numpy().view(np.uint64), toffs)
         assert ctx.get_cursor(1) == tcur
+    ctx.close()
+
+
+# (request bytes, response bytes, mtu, slot size): every shape of either half at least once, beside different shapes of
+# the other -- short fragments 8, 16 and 32 lanes each, whole and long fragments with and without short last ones;
+# short frames, whole and long frames with and without short last ones
+ANY_SHAPE = [
+    (100, 100, 1400, 2048), (300, 300, 1400, 2048), (900, 900, 1400, 2048),
+    (2800, 1400 + 100, 1400, 2048), (2 * 1400 + 336, 1400 + 272, 1400, 2048), (1400 + 648, 2800 + 900, 1400, 2048),
+    (1399, 128, 1400, 2048), (128, 2800, 1400, 2048), (17, 16, 1400, 2048),
+    (17600, 17600, 8800, 9216), (8800 + 300, 8800 + 272, 8800, 9216), (8800 + 901, 8801, 8800, 9216), (17599, 129, 8800, 9216),
+]
+
+
+@pytest.mark.parametrize("n_req", [1, 37, 1100])
+@pytest.mark.parametrize("sizes", ANY_SHAPE, ids=lambda s: f"{s[0]}-{s[1]}")
+def test_every_shape_shares_a_launch(sizes, n_req):
+    """Shapes beside each other in one launch, with the cursors advanced by the kernel (small calls) and by the one
+    behind it (SG_F_TAIL_KERNEL on either half), the full UDP checksum on every second call."""
+    size, resp, mtu, slot = sizes
+    if n_req * (size + resp) > 6 << 20:
+        n_req = 160
+    profile = n_req & 1
+    w = synth.make_custom([size] * n_req, [resp] * n_req, mtu=mtu, slot_size=slot, seed=size + resp, profile=profile)
+    print(f"case shunt any {sizes} n_req={n_req}", flush=True)
+    ctx = SgContext(0, max_reqs=8192, max_frames=1 << 14)
+    dw = DeviceWorkload(w)
+    total = int(w.req_sizes.sum())
+    cap = 2 * total + 4096 + 10
+    arena = torch.zeros(cap, dtype=torch.uint8, device=DEV)
+    offs = torch.zeros(w.n_req + 1, dtype=torch.int64, device=DEV)
+    ga, sa = _args(ctx, dw, w, arena, cap, offs, dw.resp_offsets, flags=capi.F_FORCE_SMALL)
+    rcur, tcur = 6, 0
+    ctx.set_cursor(0, rcur)
+    ctx.set_cursor(1, tcur)
+    ctx.set_profiling(True)
+    g_flags, s_flags = ga.flags, sa.flags
+    calls = [(0, 0), (0, capi.F_UDP_CSUM_FULL), (capi.F_TAIL_KERNEL, capi.F_IPV4_CSUM),
+             (capi.F_TAIL_KERNEL, capi.F_UDP_CSUM_FULL), (0, capi.F_TAIL_KERNEL | capi.F_UDP_CSUM_PSEUDO)]
+    for call, (gf, sf) in enumerate(calls):
+        arena.zero_()
+        dw.tx_ring.copy_(torch.from_numpy(w.tx_ring_init).to(DEV))
+        torch.cuda.synchronize()
+        ga.flags, sa.flags = g_flags | gf, s_flags | sf
+        ctx.shunt_batch_raw(ga, sa)
+        exp, eoffs, ecur = expected_gather(w, arena_cap=cap, cursor=rcur)
+        got = arena.cpu().numpy()
+        assert np.array_equal(got, exp), f"call {call}: " + first_diff(got, exp)
+        assert np.array_equal(offs.cpu().numpy().view(np.uint64), eoffs)
+        assert ctx.get_cursor(0) == ecur
+        exp_tx, toffs, tnext = expected_scatter(w, None, resp_cap=dw.resp_app.cap, cursor=tcur, flags=sf & 0xf)
+        got = dw.tx_ring.cpu().numpy()
+        assert np.array_equal(got, exp_tx), f"call {call}: " + first_diff(got, exp_tx)
+        assert np.array_equal(dw.resp_offsets.cpu().numpy().view(np.uint64), toffs)
+        assert ctx.get_cursor(1) == tnext
+        rcur, tcur = ecur, tnext
+    assert ctx.kernel_time(1)[1] == len(calls) and ctx.kernel_time(2)[1] == 0 and ctx.kernel_time(0)[1] == 0
     ctx.close()
 
 
