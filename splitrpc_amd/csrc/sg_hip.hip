@@ -1664,6 +1664,7 @@ int sg_hip_reassemble(sg_hip_ctx *c, const sg_reassemble_args *a, uint32_t *coun
   r.req_token = a->req_token;
   r.req_hdr_slot = a->req_hdr_slot;
   r.counts_out = a->counts_out;
+  if (a->flags & SG_F_ASYNC) r.counts_host = nullptr;  // a kernel has not ended before its stores across the bus are through
 
   rc = prof_begin(c, 5);
   if (rc != SG_OK) return rc;

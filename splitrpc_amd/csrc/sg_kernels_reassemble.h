@@ -97,7 +97,7 @@ struct RaArgs {
   uint32_t *frag_slot, *frag_len, *req_first, *req_hdr_slot;
   uint64_t *req_token;
   uint32_t *counts_out;            // device: requests, fragments, arrivals dropped, requests in flight
-  volatile uint32_t *counts_host;  // the same four, pinned host memory
+  volatile uint32_t *counts_host;  // the same four, pinned host memory; nullptr: the host does not ask
   uint32_t *status;
   volatile uint32_t *status_flag;  // pinned host word: non-zero once any kernel refused something
 };
@@ -435,7 +435,7 @@ __device__ __forceinline__ void ra_close(const RaArgs &a, uint64_t tot, unsigned
   const uint32_t c[4] = {n_req, n_frag, (uint32_t)fresh, in_flight};
   for (int k = 0; k < 4; k++) {
     if (a.counts_out) a.counts_out[k] = c[k];
-    a.counts_host[k] = c[k];  // straight into pinned host memory: nothing to copy back
+    if (a.counts_host) a.counts_host[k] = c[k];  // straight into pinned host memory: nothing to copy back
   }
 }
 
