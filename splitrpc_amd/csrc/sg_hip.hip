@@ -277,6 +277,17 @@ bool self_advancing(const Scratch &sc, bool packed, const void *slot_state, uint
 }
 
 
+// Most requests (sizes in a table) and most fragments (lengths in a table) of which every workgroup
+// of the descriptor pass adds up those before its own, instead of a scan behind it.  Whole call,
+// scan -> this, us:     requests          scatter          requests / fragments   gather
+//                       1000              12.7 ->  9.0     1000 / 1000            11.2 ->  8.8
+//                       4000              13.7 -> 10.7     4000 / 7601            14.6 -> 11.6
+//                       8000              18.9 -> 12.2     2500 / 13722           18.2 -> 16.6
+//                      16000              20.0 -> 18.9     16000 / 16000          17.3 -> 14.8
+//                      24000              24.2 -> 27.2     24000 / 24000          20.0 -> 19.5
+//                      32000              28.5 -> 37.4     32000 / 32000          23.2 -> 26.2
+constexpr uint32_t kSelfScanReqs = 16384, kSelfScanItems = 16384;
+
 // Descriptor build: kernel shape by the average request, then the bump-ring
 // scan of the request totals where offsets are not plain multiples.
 int launch_prep(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const PrepArgs &args)
@@ -288,7 +299,11 @@ int launch_prep(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const PrepArgs
   const bool tiled = p.packed && !p.fixed_offsets && !(p.n_req <= 2 * kScanTile || p.counts);
   // requests per entry of the workgroup sums k_prep_group leaves for the tiled scan
   const uint32_t per_part = avg <= 8 ? 4 * kWavesPerBlock : avg <= 16 ? 2 * kWavesPerBlock : 0;
-  if (tiled && per_part) p.part = sc.tile_tot;
+  // Few requests (a response's size stands in a table) or few fragments (so does its length): the
+  // descriptor kernel's workgroups add up what lies before them and no scan is launched.
+  p.self_scan = p.packed && !p.fixed_offsets && !p.counts &&
+                (p.mode == 1 ? p.sizes && p.n_req <= kSelfScanReqs : p.item_len && p.n_items <= kSelfScanItems);
+  if (tiled && per_part && !p.self_scan) p.part = sc.tile_tot;
   if (avg <= 8) {
     k_prep_group<16><<<(p.n_req + 4 * kWavesPerBlock - 1) / (4 * kWavesPerBlock), kBlock, 0, st>>>(p);
   } else if (avg <= 16) {
@@ -300,13 +315,14 @@ int launch_prep(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const PrepArgs
   } else {
     k_prep_block<1024><<<p.n_req, 1024, 0, st>>>(p);
   }
-  if (p.packed && !p.fixed_offsets) {
+  if (p.packed && !p.fixed_offsets && !p.self_scan) {
     if (p.n_req <= 2 * kScanTile || p.counts) {  // counts on the device: one workgroup walks whatever is there
       k_req_scan<<<1, kScanBlock, 0, st>>>(p);
     } else {
       const uint32_t n_tiles = (p.n_req + kScanTile - 1) / kScanTile;
       if (p.part) {
-        k_req_scan_parts<<<n_tiles, kScanBlock, 0, st>>>(p, per_part, n_tiles);
+        const uint32_t n_parts = (p.n_req + kPartsTile - 1) / kPartsTile;
+        k_req_scan_parts<<<n_parts, kPartsBlock, 0, st>>>(p, per_part, n_parts);
       } else {
         // (one launch in which every workgroup adds up the REQUEST sizes before its tile by itself
         // was measured at 32768 requests: 30.6 us for the descriptor pass against 26.9 us with these)

@@ -81,6 +81,9 @@ struct PrepArgs {
   // k_prep_group: where every workgroup leaves the sum of its requests' totals (for the tiled
   // scan of many requests, which then needs no launch of its own to total the tiles); or nullptr
   uint64_t *part;
+  // The sizes of the requests before a workgroup's own are few and stand in a table (response sizes,
+  // or lengths): every workgroup adds them up and writes its requests' offsets itself, no scan follows.
+  uint32_t self_scan;
   // What this pass leaves for a later call that wants to reuse its descriptors
   // (SG_F_REUSE_DESC): desc_tag = {gen, requests, items, slot size the lengths were held
   // against, arena base, arena capacity} (kTag*, eight 32-bit words).
@@ -146,17 +149,36 @@ __device__ __forceinline__ uint64_t block_exclusive_scan(uint64_t v, uint64_t *l
   return base + inc - v;
 }
 
-// Length and slot of item f of request r; raises status bits for what it refuses.
-__device__ __forceinline__ void prep_item(const PrepArgs &a, uint32_t f, uint32_t i, uint64_t size,
-                                          uint32_t *slot, uint32_t *len, uint32_t *bad)
+// Length and slot of item f of request r, which is its item i: raises status bits for what it
+// refuses.  In two steps, so that a caller with several items per lane has all of one step's loads
+// in flight together: what the tables say of item f ...
+struct PrepItem {
+  uint32_t slot, len, hdr;
+};
+__device__ __forceinline__ PrepItem prep_ask(const PrepArgs &a, uint32_t f, bool on)
 {
-  uint32_t s = a.item_slot[f];
-  uint32_t l = 0;
+  PrepItem t = {0u, 0u, 0u};
+  if (on) {
+    t.slot = a.item_slot[f];
+    if (a.mode == 0 && a.item_len) t.len = a.item_len[f];
+    if (a.mode == 1 && a.hdr_src_slot) t.hdr = a.hdr_src_slot[f];
+  }
+  return t;
+}
+// ... and what its header says, where lengths come from there.
+__device__ __forceinline__ void prep_look(const PrepArgs &a, PrepItem &t, bool on)
+{
+  if (on && a.mode == 0 && !a.item_len && t.slot < a.n_slots) t.len = load32_any(a.ring + (size_t)t.slot * a.slot_size + 54);
+}
+__device__ __forceinline__ void prep_item(const PrepArgs &a, const PrepItem &t, uint32_t i, uint64_t size, uint32_t *slot,
+                                          uint32_t *len, uint32_t *bad)
+{
+  uint32_t s = t.slot, l = 0;
   if (s >= a.n_slots) {
     *bad |= kStBadSlot;
     s = 0;
   } else if (a.mode == 0) {
-    l = a.item_len ? a.item_len[f] : load32_any(a.ring + (size_t)s * a.slot_size + 54);
+    l = t.len;
     if (l > a.slot_size - a.hl) {
       *bad |= kStBadLen;
       l = 0;
@@ -166,7 +188,7 @@ __device__ __forceinline__ void prep_item(const PrepArgs &a, uint32_t f, uint32_
     const uint64_t taken = (uint64_t)i * a.mtu;
     const uint64_t rem = taken < size ? size - taken : 0;
     l = (uint32_t)(rem <= a.mtu ? rem : a.mtu);
-    if (a.hdr_src_slot && a.hdr_src_slot[f] >= a.rx_n_slots) *bad |= kStBadSlot;
+    if (a.hdr_src_slot && t.hdr >= a.rx_n_slots) *bad |= kStBadSlot;
   }
   *slot = s;
   *len = l;
@@ -234,6 +256,74 @@ __device__ __forceinline__ void prep_finish(const PrepArgs &a, uint32_t r, uint6
   }
 }
 
+// Bytes of the requests before request r0, whose first item is f0, added up by a workgroup of
+// BLOCK threads out of the table the sizes come from (self_scan).  A size or length that is refused
+// counts as it stands: the batch then moves nothing.
+template <int BLOCK>
+__device__ __forceinline__ uint64_t prep_before(const PrepArgs &a, uint32_t r0, uint32_t f0, uint64_t *lds_wave_tot)
+{
+  constexpr uint32_t kAhead = 8;
+  uint64_t s = 0;
+  if (a.mode == 1) {
+    for (uint32_t q = threadIdx.x; q < r0; q += kAhead * BLOCK) {
+      uint64_t v[kAhead];
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) v[k] = q + k * BLOCK < r0 ? a.sizes[q + k * BLOCK] : 0ull;
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) s += v[k];
+    }
+  } else {
+    f0 = f0 <= a.n_items ? f0 : 0u;  // no such table: refused
+    for (uint32_t q = threadIdx.x; q < f0; q += kAhead * BLOCK) {
+      uint32_t v[kAhead];
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) v[k] = q + k * BLOCK < f0 ? a.item_len[q + k * BLOCK] : 0u;
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) s += v[k];
+    }
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
+  if ((threadIdx.x & (kWave - 1)) == 0) lds_wave_tot[threadIdx.x / kWave] = s;
+  __syncthreads();
+  s = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < BLOCK / kWave; w++) s += lds_wave_tot[w];
+  return s;
+}
+
+// A gathered batch larger than its arena would lap itself: wavefronts of the
+// first and of the last requests would then write the same bytes in no
+// particular order.  Refused instead.
+__device__ __forceinline__ void scan_check_batch(const PrepArgs &a, uint64_t batch_bytes)
+{
+  if (a.mode == 0 && batch_bytes > a.cap) refuse(a.status, a.status_flag, kStBadSize);
+}
+
+// Where byte `at` of the batch goes in the bump ring, from the cursor's place c0 < capacity.
+__device__ __forceinline__ uint64_t ring_at(const PrepArgs &a, uint64_t c0, uint64_t at)
+{
+  if (at >= a.cap) at %= a.cap;
+  const uint64_t o = c0 + at;
+  return o >= a.cap ? o - a.cap : o;
+}
+
+// Offset of request r, `before` bytes behind the batch's first, by the thread that owns it (self_scan).
+__device__ __forceinline__ void prep_offset(const PrepArgs &a, uint32_t r, uint64_t before, uint64_t total)
+{
+  uint64_t c0 = *a.cursor;
+  if (c0 >= a.cap) c0 %= a.cap;
+  const uint64_t off = ring_at(a, c0, before);
+  a.req_off[r] = off;
+  if (a.offsets_out) a.offsets_out[r] = off;
+  if (r == a.n_req - 1) {
+    const uint64_t end = ring_at(a, c0, before + total);
+    *a.next_cursor = end;
+    if (a.offsets_out) a.offsets_out[a.n_req] = end;
+    scan_check_batch(a, before + total);
+  }
+}
+
 // One workgroup of BLOCK threads per request: block-wide exclusive scan of the
 // fragment lengths, all header reads of a pass in flight together.
 template <int BLOCK>
@@ -250,7 +340,9 @@ __global__ __launch_bounds__(BLOCK) void k_prep_block(PrepArgs a)
   for (uint32_t base = f0; base < f1; base += BLOCK) {
     const uint32_t f = base + threadIdx.x;
     uint32_t len = 0, slot = 0;
-    if (f < f1) prep_item(a, f, f - f0, size, &slot, &len, &bad);
+    PrepItem t = prep_ask(a, f, f < f1);
+    prep_look(a, t, f < f1);
+    if (f < f1) prep_item(a, t, f - f0, size, &slot, &len, &bad);
     uint64_t tot;
     const uint64_t ex = block_exclusive_scan<BLOCK>(len, wave_tot, &tot);
     if (f < f1) {
@@ -263,23 +355,32 @@ __global__ __launch_bounds__(BLOCK) void k_prep_block(PrepArgs a)
   bad = wave_or(bad);
   if ((threadIdx.x & (kWave - 1)) == 0 && bad) refuse(a.status, a.status_flag, bad);
   if (threadIdx.x == 0) prep_finish(a, r, carry, 0);
+  if (a.self_scan) {
+    const uint64_t before = prep_before<BLOCK>(a, r, f0, wave_tot);
+    if (threadIdx.x == 0) prep_offset(a, r, before, carry);
+  }
 }
 
 // One wavefront per request (requests of at most a few dozen fragments).
 __global__ __launch_bounds__(kBlock) void k_prep_wave(PrepArgs a)
 {
+  __shared__ uint64_t wave_tot[kWavesPerBlock], req_tot[kWavesPerBlock];
   prep_effective(a);
-  const uint32_t r = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-  if (r >= a.n_req) return;
+  const uint32_t r0 = blockIdx.x * kWavesPerBlock, wv = threadIdx.x / kWave;
+  const uint32_t r = r0 + wv;
+  const bool live = r < a.n_req;
+  if (r0 >= a.n_req || (!live && !a.self_scan)) return;  // (with self_scan the whole workgroup has barriers to come to)
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  uint32_t f0, f1;
-  uint64_t size;
-  uint32_t bad = prep_range(a, r, &f0, &f1, &size);
+  uint32_t f0 = 0, f1 = 0, bad = 0;
+  uint64_t size = 0;
+  if (live) bad = prep_range(a, r, &f0, &f1, &size);
   uint64_t carry = 0;
   for (uint32_t base = f0; base < f1; base += kWave) {
     const uint32_t f = base + lane;
     uint32_t len = 0, slot = 0;
-    if (f < f1) prep_item(a, f, f - f0, size, &slot, &len, &bad);
+    PrepItem t = prep_ask(a, f, f < f1);
+    prep_look(a, t, f < f1);
+    if (f < f1) prep_item(a, t, f - f0, size, &slot, &len, &bad);
     uint64_t tot;
     const uint64_t ex = block_exclusive_scan<kWave>(len, nullptr, &tot);
     if (f < f1) {
@@ -289,7 +390,15 @@ __global__ __launch_bounds__(kBlock) void k_prep_wave(PrepArgs a)
     carry += tot;
   }
   bad = wave_or(bad);
-  if (lane == 0) prep_finish(a, r, carry, bad);
+  if (live && lane == 0) prep_finish(a, r, carry, bad);
+  if (a.self_scan) {
+    if (lane == 0) req_tot[wv] = carry;
+    uint64_t before = prep_before<kBlock>(a, r0, a.first[r0], wave_tot);  // its barrier also stands behind req_tot
+    if (live && lane == 0) {
+      for (uint32_t k = 0; k < wv; k++) before += req_tot[k];
+      prep_offset(a, r, before, carry);
+    }
+  }
 }
 
 // Several requests per wavefront, L = 16 or 32 lanes each (requests of a handful of fragments:
@@ -297,11 +406,13 @@ __global__ __launch_bounds__(kBlock) void k_prep_wave(PrepArgs a)
 // dependent round trips -- table, header, scan -- as there are requests).  The scan runs over the
 // L lanes of a group; a request of more than L fragments takes more steps, and the wavefront
 // keeps stepping while any of its groups has fragments left.
+// (Held to the scalar registers of eight wavefronts per SIMD instead of seven: 32768 requests 10.2 ->
+// 12.7 us, the arguments are then fetched again and again.)
 template <int L>
 __global__ __launch_bounds__(kBlock) void k_prep_group(PrepArgs a)
 {
   constexpr uint32_t G = kWave / L;
-  __shared__ uint64_t group_tot[kWavesPerBlock * G];
+  __shared__ uint64_t group_tot[kWavesPerBlock * G], wave_tot[kWavesPerBlock];
   prep_effective(a);
   const uint32_t lane = threadIdx.x & (kWave - 1), gl = lane & (L - 1);
   const uint32_t wave = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
@@ -311,26 +422,47 @@ __global__ __launch_bounds__(kBlock) void k_prep_group(PrepArgs a)
   uint64_t size = 0;
   if (live) bad = prep_range(a, r, &f0, &f1, &size);
   uint64_t carry = 0;
-  for (uint32_t base = f0; __any(base < f1); base += L) {
-    const uint32_t f = base + gl;
-    uint32_t len = 0, slot = 0;
-    if (f < f1) prep_item(a, f, f - f0, size, &slot, &len, &bad);
-    // inclusive scan over the group's lanes
-    uint32_t inc = len;
+  // kAhead steps' worth of table entries asked for together, then of headers: a request of several
+  // steps costs two round trips and not two per step
+  constexpr uint32_t kAhead = 64 / L;
+  for (uint32_t base0 = f0; __any(base0 < f1); base0 += kAhead * L) {
+    PrepItem t[kAhead];
 #pragma unroll
-    for (int d = 1; d < L; d <<= 1) {
-      const uint32_t up = __shfl_up(inc, d, L);
-      if ((int)gl >= d) inc += up;
+    for (uint32_t k = 0; k < kAhead; k++) t[k] = prep_ask(a, base0 + k * L + gl, base0 + k * L + gl < f1);
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; k++) prep_look(a, t[k], base0 + k * L + gl < f1);
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; k++) {
+      const uint32_t f = base0 + k * L + gl;
+      if (!__any(base0 + k * L < f1)) break;
+      uint32_t len = 0, slot = 0;
+      if (f < f1) prep_item(a, t[k], f - f0, size, &slot, &len, &bad);
+      // inclusive scan over the group's lanes
+      uint32_t inc = len;
+#pragma unroll
+      for (int d = 1; d < L; d <<= 1) {
+        const uint32_t up = __shfl_up(inc, d, L);
+        if ((int)gl >= d) inc += up;
+      }
+      if (f < f1) {
+        u32x4 d = {slot, len, (uint32_t)(carry + (inc - len)), r};
+        a.desc[f] = d;
+      }
+      carry += __shfl(inc, L - 1, L);
     }
-    if (f < f1) {
-      u32x4 d = {slot, len, (uint32_t)(carry + (inc - len)), r};
-      a.desc[f] = d;
-    }
-    carry += __shfl(inc, L - 1, L);
   }
 #pragma unroll
   for (int m = L / 2; m >= 1; m >>= 1) bad |= __shfl_xor(bad, m, L);
   if (live && gl == 0) prep_finish(a, r, carry, bad);
+  if (a.self_scan) {
+    const uint32_t r0 = blockIdx.x * kWavesPerBlock * G, mine = threadIdx.x / L;
+    if (gl == 0) group_tot[mine] = carry;
+    uint64_t before = prep_before<kBlock>(a, r0, a.first[r0], wave_tot);  // its barrier also stands behind group_tot
+    if (live && gl == 0) {
+      for (uint32_t k = 0; k < mine; k++) before += group_tot[k];
+      prep_offset(a, r, before, carry);
+    }
+  }
   if (a.part) {
     // the workgroup's requests added up: kWavesPerBlock * G consecutive requests per entry
     if (gl == 0) group_tot[threadIdx.x / L] = live ? carry : 0;
@@ -358,6 +490,7 @@ constexpr uint32_t kPartMin = 2 * kWavesPerBlock;
 
 // Exclusive scan of one tile; returns this thread's prefix for its first
 // request and leaves its requests' sizes in sz[].
+template <int BLOCK>
 __device__ __forceinline__ uint64_t scan_tile(const PrepArgs &a, uint32_t q0, uint64_t *sz,
                                               uint64_t *wave_tot, uint64_t *tot)
 {
@@ -367,7 +500,7 @@ __device__ __forceinline__ uint64_t scan_tile(const PrepArgs &a, uint32_t q0, ui
     sz[k] = (q0 + k < a.n_req) ? a.req_size[q0 + k] : 0;
     mine += sz[k];
   }
-  return block_exclusive_scan<kScanBlock>(mine, wave_tot, tot);
+  return block_exclusive_scan<BLOCK>(mine, wave_tot, tot);
 }
 
 __device__ __forceinline__ void scan_emit(const PrepArgs &a, uint32_t q0, const uint64_t *sz, uint64_t off)
@@ -384,14 +517,6 @@ __device__ __forceinline__ void scan_emit(const PrepArgs &a, uint32_t q0, const 
   }
 }
 
-// A gathered batch larger than its arena would lap itself: wavefronts of the
-// first and of the last requests would then write the same bytes in no
-// particular order.  Refused instead.
-__device__ __forceinline__ void scan_check_batch(const PrepArgs &a, uint64_t batch_bytes)
-{
-  if (a.mode == 0 && batch_bytes > a.cap) refuse(a.status, a.status_flag, kStBadSize);
-}
-
 __global__ __launch_bounds__(kScanBlock) void k_req_scan(PrepArgs a)
 {
   __shared__ uint64_t wave_tot[kScanBlock / kWave];
@@ -400,7 +525,7 @@ __global__ __launch_bounds__(kScanBlock) void k_req_scan(PrepArgs a)
   for (uint32_t base = 0; base < a.n_req; base += kScanTile) {
     const uint32_t q0 = base + threadIdx.x * kScanPerThread;
     uint64_t sz[kScanPerThread], tot;
-    const uint64_t ex = scan_tile(a, q0, sz, wave_tot, &tot);
+    const uint64_t ex = scan_tile<kScanBlock>(a, q0, sz, wave_tot, &tot);
     scan_emit(a, q0, sz, (run + ex) % a.cap);
     run = (run + tot) % a.cap;
     batch_bytes += tot;
@@ -418,38 +543,58 @@ __global__ __launch_bounds__(kScanBlock) void k_req_scan_local(PrepArgs a, uint6
   __shared__ uint64_t wave_tot[kScanBlock / kWave];
   const uint32_t q0 = blockIdx.x * kScanTile + threadIdx.x * kScanPerThread;
   uint64_t sz[kScanPerThread], tot;
-  (void)scan_tile(a, q0, sz, wave_tot, &tot);
+  (void)scan_tile<kScanBlock>(a, q0, sz, wave_tot, &tot);
   if (threadIdx.x == 0) tile_tot[blockIdx.x] = tot;
 }
 
-// Every tile sums the totals of the tiles before it (a few values) for its base
-// and scans again from there; the last tile also publishes the advanced cursor.
 // The tiled scan behind k_prep_group, in one launch: the sizes before a tile are the sums the
 // descriptor kernel's workgroups left (`per_part` requests each; a tile's worth of them is a few
-// hundred values), so no launch is spent on totalling the tiles.
-__global__ __launch_bounds__(kScanBlock) void k_req_scan_parts(PrepArgs a, uint32_t per_part, uint32_t n_tiles)
+// dozen values), so no launch is spent on totalling the tiles.  One dependent chain (sums -> base ->
+// offsets) and hardly a byte: small tiles, and the tile's own sizes asked for before the sums are
+// added up.
+constexpr int kPartsBlock = 256;
+constexpr uint32_t kPartsTile = kPartsBlock * kScanPerThread;
+__global__ __launch_bounds__(kPartsBlock) void k_req_scan_parts(PrepArgs a, uint32_t per_part, uint32_t n_tiles)
 {
-  __shared__ uint64_t wave_tot[kScanBlock / kWave];
+  __shared__ uint64_t wave_tot[kPartsBlock / kWave], wave_sum_lds[kPartsBlock / kWave];
   const bool is_last = blockIdx.x == n_tiles - 1;
-  const uint32_t parts_before = blockIdx.x * (kScanTile / per_part);  // a tile is a whole number of parts
-  uint64_t s = 0, before = 0;
-  for (uint32_t q = threadIdx.x; q < parts_before; q += kScanBlock) s += a.part[q];
-  (void)block_exclusive_scan<kScanBlock>(s, wave_tot, &before);
-  const uint64_t c0 = *a.cursor % a.cap;
-  const uint64_t tile_base = (c0 + before % a.cap) % a.cap;
-  const uint32_t q0 = blockIdx.x * kScanTile + threadIdx.x * kScanPerThread;
-  uint64_t sz[kScanPerThread], tot;
-  const uint64_t ex = scan_tile(a, q0, sz, wave_tot, &tot);
-  scan_emit(a, q0, sz, (tile_base + ex % a.cap) % a.cap);
+  const uint32_t parts_before = blockIdx.x * (kPartsTile / per_part);  // a tile is a whole number of parts
+  const uint32_t q0 = blockIdx.x * kPartsTile + threadIdx.x * kScanPerThread;
+  uint64_t c0 = *a.cursor;
+  uint64_t sz[kScanPerThread], tot, mine = 0;
+#pragma unroll
+  for (int k = 0; k < kScanPerThread; k++) sz[k] = q0 + k < a.n_req ? a.req_size[q0 + k] : 0;
+  uint64_t before = 0;
+  constexpr uint32_t kAhead = 8;
+  for (uint32_t q = threadIdx.x; q < parts_before; q += kAhead * kPartsBlock) {
+    uint64_t v[kAhead];
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; k++) v[k] = q + k * kPartsBlock < parts_before ? a.part[q + k * kPartsBlock] : 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; k++) before += v[k];
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) before += __shfl_xor(before, m, 64);
+  if ((threadIdx.x & (kWave - 1)) == 0) wave_sum_lds[threadIdx.x / kWave] = before;
+#pragma unroll
+  for (int k = 0; k < kScanPerThread; k++) mine += sz[k];
+  const uint64_t ex = block_exclusive_scan<kPartsBlock>(mine, wave_tot, &tot);  // its barriers stand behind the sums too
+  before = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < kPartsBlock / kWave; w++) before += wave_sum_lds[w];
+  if (c0 >= a.cap) c0 %= a.cap;
+  scan_emit(a, q0, sz, ring_at(a, c0, before + ex));
   if (is_last && threadIdx.x == 0) {
     const uint64_t batch_bytes = before + tot;
-    const uint64_t end = (c0 + batch_bytes % a.cap) % a.cap;
+    const uint64_t end = ring_at(a, c0, batch_bytes);
     *a.next_cursor = end;
     if (a.offsets_out) a.offsets_out[a.n_req] = end;
     scan_check_batch(a, batch_bytes);
   }
 }
 
+// Every tile sums the totals of the tiles before it (a few values) for its base
+// and scans again from there; the last tile also publishes the advanced cursor.
 __global__ __launch_bounds__(kScanBlock) void k_req_scan_add(PrepArgs a, const uint64_t *tile_tot, uint32_t n_tiles)
 {
   __shared__ uint64_t wave_tot[kScanBlock / kWave];
@@ -469,7 +614,7 @@ __global__ __launch_bounds__(kScanBlock) void k_req_scan_add(PrepArgs a, const u
   const uint64_t tile_base = (c0 + before % a.cap) % a.cap;
   const uint32_t q0 = blockIdx.x * kScanTile + threadIdx.x * kScanPerThread;
   uint64_t sz[kScanPerThread], tot;
-  const uint64_t ex = scan_tile(a, q0, sz, wave_tot, &tot);
+  const uint64_t ex = scan_tile<kScanBlock>(a, q0, sz, wave_tot, &tot);
   scan_emit(a, q0, sz, (tile_base + ex % a.cap) % a.cap);
   if (is_last && threadIdx.x == 0) {
     const uint64_t end = (c0 + batch_bytes % a.cap) % a.cap;
