@@ -117,6 +117,7 @@ struct sg_hip_ctx {
   Run *h_runs = nullptr;
   uint32_t h_runs_cap = 0;
   uint64_t *h_ptrs = nullptr;
+  bool staging_read = false;  // a launch that reads h_runs or h_ptrs has not been waited for
   uint64_t *h_probe = nullptr;   // pinned: what a probe launch saw of itself (queue address, dispatch id), twice
   uint32_t *h_status = nullptr;  // pinned: [0] copy of status (read back only after a refusal), [1] the refusal flag
   volatile uint32_t *h_flag = nullptr;
@@ -774,6 +775,34 @@ int sg_hip_kernel_time(sg_hip_ctx *c, int which, double *total_ms, uint64_t *lau
 // Runs longer than this are cut so that no single wavefront walks megabytes.
 static const uint64_t kRunChunk = 16384;
 
+// The pinned staging buffers are written by the host again: the launch that read them must be through.
+// (Every call waits for its own; one that failed on the way has not.)
+static int staging_free(sg_hip_ctx *c)
+{
+  if (!c->staging_read) return SG_OK;
+  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  c->staging_read = false;
+  return SG_OK;
+}
+
+// Copies the n runs staged in c->h_runs.
+static int launch_runs(sg_hip_ctx *c, uint32_t n)
+{
+  int rc = prof_begin(c, 3);
+  if (rc != SG_OK) return rc;
+  const uint32_t grid = (n + kWavesPerBlock - 1) / kWavesPerBlock;
+  if (n <= kInlineRuns) {
+    RunsInline a;
+    memcpy(a.run, c->h_runs, n * sizeof(Run));
+    a.n = n;
+    k_copy_runs_inline<<<grid, kBlock, 0, c->stream>>>(a);
+  } else {
+    c->staging_read = true;
+    k_copy_runs<<<grid, kBlock, 0, c->stream>>>(c->h_runs, n);
+  }
+  return prof_end(c);
+}
+
 static int copy_skb(sg_hip_ctx *c, const sg_sk_buf *skb)
 {
   if (!c || !skb) return fail(c, SG_E_INVAL, "null argument");
@@ -781,8 +810,8 @@ static int copy_skb(sg_hip_ctx *c, const sg_sk_buf *skb)
     return fail(c, SG_E_INVAL, "run table holds %llu runs; len[] has room for %d",
                 (unsigned long long)skb->num_items, SG_MAX_BI_SIZE - 1);
   DeviceGuard g(c->device);
-  // the pinned staging buffer is reused: the previous launch must have read it
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  int rc = staging_free(c);
+  if (rc != SG_OK) return rc;
   uint32_t n = 0;
   for (uint64_t i = 0; i < skb->num_items; i++) {
     uint64_t src = skb->i_buf[i], dst = skb->o_buf[i], len = skb->len[i];
@@ -795,12 +824,9 @@ static int copy_skb(sg_hip_ctx *c, const sg_sk_buf *skb)
       }
       if (n == c->h_runs_cap) {
         // flush what is staged and start over
-        int rc = prof_begin(c, 3);
+        rc = launch_runs(c, n);
+        if (rc == SG_OK) rc = staging_free(c);
         if (rc != SG_OK) return rc;
-        k_copy_runs<<<(n + kWavesPerBlock - 1) / kWavesPerBlock, kBlock, 0, c->stream>>>(c->h_runs, n);
-        rc = prof_end(c);
-        if (rc != SG_OK) return rc;
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
         n = 0;
       }
       c->h_runs[n++] = Run{src, dst, piece};
@@ -808,13 +834,12 @@ static int copy_skb(sg_hip_ctx *c, const sg_sk_buf *skb)
     }
   }
   if (n) {
-    int rc = prof_begin(c, 3);
-    if (rc != SG_OK) return rc;
-    k_copy_runs<<<(n + kWavesPerBlock - 1) / kWavesPerBlock, kBlock, 0, c->stream>>>(c->h_runs, n);
-    rc = prof_end(c);
+    rc = launch_runs(c, n);
     if (rc != SG_OK) return rc;
   }
-  return finish(c, 0);
+  rc = finish(c, 0);
+  if (rc == SG_OK || rc == SG_E_DATA) c->staging_read = false;  // waited for
+  return rc;
 }
 
 int sg_hip_gather(sg_hip_ctx *c, const sg_sk_buf *skb) { return copy_skb(c, skb); }
@@ -830,26 +855,39 @@ static int fill_hdrs(sg_hip_ctx *c, const sg_hbufs *hdrs, const uint8_t *tmpl, u
   if (flags & SG_F_UDP_CSUM_FULL) return fail(c, SG_E_INVAL, "a header-only rewrite cannot finish the UDP checksum");
   const uint32_t n = hdrs->num_items;
   if (n == 0) return SG_OK;
-  DeviceGuard g(c->device);
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  for (uint32_t i = 0; i < n; i++) {
+  for (uint32_t i = 0; i < n; i++)
     if (!hdrs->burst_items[i]) return fail(c, SG_E_INVAL, "header %u is null", i);
-    c->h_ptrs[i] = hdrs->burst_items[i];
-  }
-  // the template rides behind the pointer table in the same pinned block
-  const uint8_t *d_tmpl = nullptr;
-  if (tmpl) {
-    memcpy(c->h_ptrs + SG_MAX_BI_SIZE, tmpl, 64);
-    d_tmpl = reinterpret_cast<const uint8_t *>(c->h_ptrs + SG_MAX_BI_SIZE);
-  }
-  int rc = prof_begin(c, 4);
+  DeviceGuard g(c->device);
+  SwapInline s;
+  s.a.n = n;
+  s.a.hl = hdr_len_of(profile);
+  s.a.ref64 = profile == SG_HDR_REF64;
+  s.a.flags = flags & 0xfu;
+  s.a.payload_size = payload_size;
+  s.a.token = token;
+  s.a.mtu = mtu;
+  s.a.has_tmpl = tmpl != nullptr;
+  int rc = staging_free(c);
   if (rc != SG_OK) return rc;
-  k_swap_hdrs<<<(n + kWavesPerBlock - 1) / kWavesPerBlock, kBlock, 0, c->stream>>>(
-      c->h_ptrs, n, hdr_len_of(profile), profile == SG_HDR_REF64, flags & 0xfu, payload_size, mtu,
-      d_tmpl, token);
+  rc = prof_begin(c, 4);
+  if (rc != SG_OK) return rc;
+  const uint32_t grid = (n + kWavesPerBlock - 1) / kWavesPerBlock;
+  if (n <= kInlineHdrs) {
+    if (tmpl) memcpy(s.tmpl, tmpl, sizeof s.tmpl);
+    memcpy(s.hdr, hdrs->burst_items, n * sizeof(uint64_t));
+    k_swap_hdrs_inline<<<grid, kBlock, 0, c->stream>>>(s);
+  } else {
+    memcpy(c->h_ptrs, hdrs->burst_items, n * sizeof(uint64_t));
+    // the template rides behind the pointer table in the same pinned block
+    if (tmpl) memcpy(c->h_ptrs + SG_MAX_BI_SIZE, tmpl, 64);
+    c->staging_read = true;
+    k_swap_hdrs<<<grid, kBlock, 0, c->stream>>>(s.a, c->h_ptrs, reinterpret_cast<const uint8_t *>(c->h_ptrs + SG_MAX_BI_SIZE));
+  }
   rc = prof_end(c);
   if (rc != SG_OK) return rc;
-  return finish(c, 0);
+  rc = finish(c, 0);
+  if (rc == SG_OK || rc == SG_E_DATA) c->staging_read = false;  // waited for
+  return rc;
 }
 
 int sg_hip_swap_hdrs(sg_hip_ctx *c, const sg_hbufs *hdrs, uint32_t profile, uint64_t payload_size,

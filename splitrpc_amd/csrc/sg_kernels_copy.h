@@ -1252,34 +1252,75 @@ struct Run {
   uint64_t len;
 };
 
+__device__ __forceinline__ void copy_one_run(const Run &r, uint32_t lane)
+{
+  copy_run<false>(reinterpret_cast<const uint8_t *>(r.src), reinterpret_cast<uint8_t *>(r.dst), (uint32_t)r.len, lane);
+}
+
 __global__ __launch_bounds__(kBlock) void k_copy_runs(const Run *runs, uint32_t n)
 {
   const uint32_t item = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
   if (item >= n) return;
-  const uint32_t lane = threadIdx.x & (kWave - 1);
-  const Run r = runs[item];
-  copy_run<false>(reinterpret_cast<const uint8_t *>(r.src), reinterpret_cast<uint8_t *>(r.dst),
-                  (uint32_t)r.len, lane);
+  copy_one_run(runs[item], threadIdx.x & (kWave - 1));
 }
 
+// A call waits for its kernel, and a short table that lies in pinned host memory is a round trip
+// across the bus at the head of every wavefront: up to these many entries travel with the launch.
+constexpr uint32_t kInlineRuns = 32, kInlineHdrs = 64;
+struct RunsInline {
+  Run run[kInlineRuns];
+  uint32_t n;
+};
+
+__global__ __launch_bounds__(kBlock) void k_copy_runs_inline(RunsInline a)
+{
+  const uint32_t item = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave);
+  if (item >= a.n) return;
+  const uint64_t *p = reinterpret_cast<const uint64_t *>(kernarg_at(offsetof(RunsInline, run) + item * sizeof(Run)));
+  copy_one_run(Run{sload_here(p), sload_here(p + 1), sload_here(p + 2)}, threadIdx.x & (kWave - 1));
+}
+
+struct SwapArgs {
+  uint32_t n, hl, ref64, flags;
+  uint64_t payload_size;
+  uint64_t token;
+  uint32_t mtu;
+  uint32_t has_tmpl;
+};
+
 // tmpl == nullptr: swap each header in place; else every header is a copy of
-// the 64-byte template with `token` in it (the two ways the reference fills
+// the 64-byte template with the token in it (the two ways the reference fills
 // response headers: rr_swap_hdr and rr_set_hdr).
-__global__ __launch_bounds__(kBlock) void k_swap_hdrs(const uint64_t *hdr_ptrs, uint32_t n,
-                                                      uint32_t hl, uint32_t ref64, uint32_t flags,
-                                                      uint64_t payload_size, uint32_t mtu,
-                                                      const uint8_t *tmpl, uint64_t token)
+__device__ __forceinline__ void fill_one_hdr(const SwapArgs &a, uint8_t *h, uint32_t item, const uint8_t *tmpl)
+{
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const uint64_t taken = (uint64_t)item * a.mtu;
+  const uint64_t rem = taken < a.payload_size ? a.payload_size - taken : 0;
+  HdrFields hf{a.hl, a.ref64, a.flags & ~(1u << 2), item, a.n, (uint32_t)(rem <= a.mtu ? rem : a.mtu),
+               tmpl != nullptr, tmpl != nullptr, a.token};
+  const uint32_t b = hdr_finish(hdr_fetch(tmpl ? tmpl : h, lane, a.hl, tmpl == nullptr), lane, hf, 0);
+  if (lane < a.hl) h[lane] = (uint8_t)b;
+}
+
+__global__ __launch_bounds__(kBlock) void k_swap_hdrs(SwapArgs a, const uint64_t *hdr_ptrs, const uint8_t *tmpl)
 {
   const uint32_t item = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-  if (item >= n) return;
-  const uint32_t lane = threadIdx.x & (kWave - 1);
-  uint8_t *h = reinterpret_cast<uint8_t *>(hdr_ptrs[item]);
-  const uint64_t taken = (uint64_t)item * mtu;
-  const uint64_t rem = taken < payload_size ? payload_size - taken : 0;
-  HdrFields hf{hl, ref64, flags & ~(1u << 2), item, n, (uint32_t)(rem <= mtu ? rem : mtu),
-               tmpl != nullptr, tmpl != nullptr, token};
-  const uint32_t b = hdr_finish(hdr_fetch(tmpl ? tmpl : h, lane, hl, tmpl == nullptr), lane, hf, 0);
-  if (lane < hl) h[lane] = (uint8_t)b;
+  if (item >= a.n) return;
+  fill_one_hdr(a, reinterpret_cast<uint8_t *>(hdr_ptrs[item]), item, a.has_tmpl ? tmpl : nullptr);
+}
+
+struct SwapInline {
+  SwapArgs a;
+  uint8_t tmpl[64];
+  uint64_t hdr[kInlineHdrs];
+};
+
+__global__ __launch_bounds__(kBlock) void k_swap_hdrs_inline(SwapInline s)
+{
+  const uint32_t item = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave);
+  if (item >= s.a.n) return;
+  const uint64_t h = sload(reinterpret_cast<const uint64_t *>(kernarg_at(offsetof(SwapInline, hdr))) + item);
+  fill_one_hdr(s.a, reinterpret_cast<uint8_t *>(h), item, s.a.has_tmpl ? kernarg_at(offsetof(SwapInline, tmpl)) : nullptr);
 }
 
 // Sets `n` 32-bit words to zero (a fill kernel rather than a memset node, so
