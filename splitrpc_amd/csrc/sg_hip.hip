@@ -1370,10 +1370,10 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
   if (!c || !g || !s) return fail(c, SG_E_INVAL, "null argument");
   DeviceGuard guard(c->device);
   const uint32_t async = g->flags & s->flags & SG_F_ASYNC;
-  // What the gather writes (requests) against everything the scatter touches (responses, the ring
-  // its headers come from, TX slots), and what the scatter writes (TX slots) against what the gather
-  // reads (RX slots): halves that touch each other's memory run one after the other.  Application
-  // memory is an arena or, tensor-major, n_req rows per tensor.
+  // What the gather writes (requests, offsets) against everything the scatter touches (responses, the
+  // ring its headers come from, TX slots, tables), and what the scatter writes (TX slots, offsets)
+  // against what the gather reads: halves that touch each other's memory run one after the other.
+  // Application memory is an arena or, tensor-major, n_req rows per tensor.
   struct Range { const void *p; uint64_t n; };
   auto app_ranges = [](const sg_app_desc &app, uint32_t n_req, Range *out) {
     uint32_t k = 0;
@@ -1383,15 +1383,27 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
         out[k++] = Range{app.tensor_base[t], app.tensor_size[t] * n_req};
     return k;
   };
-  Range gw[SG_MAX_TENSORS + 1], st[SG_MAX_TENSORS + 3];
-  const uint32_t n_gw = app_ranges(g->app, g->n_req, gw);
-  uint32_t n_st = app_ranges(s->app, s->n_req, st);
+  auto table = [](const void *p, uint64_t bytes) { return Range{p, p ? bytes : 0u}; };
+  const uint64_t gn = g->n_req, gf = g->n_frags, sn = s->n_req, sf = s->n_frames;
+  const Range g_rx{g->ring.base, (uint64_t)g->ring.n_slots * g->ring.slot_size};
+  const Range s_rx{s->rx.base, (uint64_t)s->rx.n_slots * s->rx.slot_size};
   const Range s_tx{s->tx.base, (uint64_t)s->tx.n_slots * s->tx.slot_size};
-  st[n_st++] = s_tx;
-  st[n_st++] = Range{s->rx.base, (uint64_t)s->rx.n_slots * s->rx.slot_size};
-  bool apart = !ranges_overlap(s_tx.p, s_tx.n, g->ring.base, (uint64_t)g->ring.n_slots * g->ring.slot_size);
+  const Range s_offs = table(s->offsets_out, (sn + 1) * 8);
+  Range gw[SG_MAX_TENSORS + 1], st[SG_MAX_TENSORS + 10];
+  uint32_t n_gw = app_ranges(g->app, g->n_req, gw);
+  gw[n_gw++] = table(g->offsets_out, (gn + 1) * 8);
+  uint32_t n_st = app_ranges(s->app, s->n_req, st);
+  const Range s_more[] = {s_tx, s_rx, s_offs, table(s->tx_slot, sf * 4), table(s->hdr_src_slot, sf * 4),
+                          table(s->hdr_src_req, sn * 4), table(s->resp_first, (sn + 1) * 4),
+                          table(s->hdr_templates, sn * 64), table(s->req_token, sn * 8), table(s->counts, 16)};
+  for (const Range &r : s_more) st[n_st++] = r;
+  const Range g_reads[] = {g_rx, table(g->frag_slot, gf * 4), table(g->frag_len, gf * 4), table(g->req_first, (gn + 1) * 4),
+                           table(g->counts, 16)};
+  auto meet = [](const Range &x, const Range &y) { return x.n && y.n && ranges_overlap(x.p, x.n, y.p, y.n); };
+  bool apart = true;
   for (uint32_t i = 0; i < n_gw; i++)
-    for (uint32_t j = 0; j < n_st; j++) apart = apart && !ranges_overlap(gw[i].p, gw[i].n, st[j].p, st[j].n);
+    for (uint32_t j = 0; j < n_st; j++) apart = apart && !meet(gw[i], st[j]);
+  for (const Range &r : g_reads) apart = apart && !meet(s_tx, r) && !meet(s_offs, r);
   // Both halves are looked at before either is launched: a call the host refuses launches nothing.
   // A half that cannot share a launch leaves no trace; both are then made as calls of their own.
   ShuntHalf h;

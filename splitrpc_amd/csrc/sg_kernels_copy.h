@@ -853,9 +853,10 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
   uint32_t item = SPLIT ? w / pieces : w;
   const uint32_t piece = SPLIT ? w - item * pieces : 0;
   if (FUSED && a.rule.per_launch != a.rule.per_req) {
-    // the short remainder frame of every response is k_scatter_small's (a launch of its own: with
-    // both kinds of wavefront in one kernel, in turns or one kind after the other, the full frames
-    // lost more than the second launch costs): this launch counts the other frames only
+    // the short remainder frame of every response is scatter_small_wave's -- in a launch of its own
+    // behind this one, or in workgroups in front of these (k_shunt_any; dealt in among the others there,
+    // every 5th to 15th workgroup of eight, they cost 131072 responses 270 - 284 us per pass instead of
+    // 267): this body counts the other frames only
     const uint32_t pl = a.rule.per_launch;
     if (item >= n_req * pl) return;
     const uint32_t rr = (uint32_t)(((uint64_t)item * a.rule.lmul) >> a.rule.lshift);

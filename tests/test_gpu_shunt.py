@@ -185,6 +185,22 @@ def test_every_shape_shares_a_launch(sizes, n_req):
     ctx.close()
 
 
+def test_halves_that_write_the_same_table_run_in_order():
+    """One offsets table for both halves: the scatter's offsets are what it holds afterwards."""
+    w = synth.make_custom([4200] * 300, [3000] * 300, seed=79)
+    ctx = SgContext(0)
+    dw = DeviceWorkload(w)
+    ga, sa = _args(ctx, dw, w, None, 0, dw.req_offsets, dw.req_offsets)
+    ctx.set_cursor(0, 0)
+    ctx.set_cursor(1, 0)
+    ctx.set_profiling(True)
+    ctx.shunt_batch_raw(ga, sa)
+    _, toffs, _ = expected_scatter(w, None, resp_cap=dw.resp_app.cap)
+    assert np.array_equal(dw.req_offsets.cpu().numpy().view(np.uint64), toffs)
+    assert ctx.kernel_time(1)[1] == 1 and ctx.kernel_time(2)[1] == 1
+    ctx.close()
+
+
 def test_refusals_come_through_either_half():
     w = synth.make_custom([4200] * 6, [3000] * 6, seed=75)
     ctx = SgContext(0)
