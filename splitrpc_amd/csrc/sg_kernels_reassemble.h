@@ -52,7 +52,7 @@ namespace {
 //   to the table, records from a ring:
 //     insert / flag / scan / emit          23.2 / 5.5 / 4.9 / 8.4    30.1 / 9.7 / 4.7 / 13.0
 //   this form: insert / flag / emit        11.3 / 4.9 / 6.6          14.6 / 4.8 / 7.7
-//   64 arrivals in one launch              8.6 -> 5.4
+//   64 arrivals in one launch              8.6 -> 5.4, and 3.8 where the counts stay on the device
 // (a launch that does nothing shows as 2 to 4 us there).  Workgroups of 512 threads: 11.9 / 5.2 / 6.0
 // and 14.0 / 5.1 / 9.4; of 1024: 12.2 / 5.2 / 5.8 and 20.5 / 6.8 / 10.8.  The ring of free records
 // cost a returning addition per workgroup to one word, 35 to 70 ns each and one after the other, and
