@@ -527,7 +527,6 @@ struct ShuntHalf {
   // launch of its own would advance it itself
   uint64_t *cursor[2] = {nullptr, nullptr};
   bool self[2] = {false, false};
-  FinishArgs fin[2];
 };
 constexpr int kNoShare = 1;  // the call needs kernels of its own
 
@@ -948,7 +947,8 @@ static int gather_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const s
     if (n_items >= (1u << 27)) return fail(c, SG_E_INVAL, "%u fragments in one call: the limit is 2^27 - 1", n_items);
     if (a->fixed_req_size > 0xffffffffull || (packed ? a->fixed_req_size > app.cap : a->fixed_req_size > max_req_bytes))
       return fail(c, SG_E_INVAL, "request size %llu does not fit its destination", (unsigned long long)a->fixed_req_size);
-    GatherRuleArgs ga;
+    GatherRuleArgs own;
+    GatherRuleArgs &ga = half ? half->sh.g : own;  // a shared launch's are built where it takes them from
     memset(&ga, 0, sizeof ga);
     ga.ring = static_cast<const uint8_t *>(a->ring.base);
     ga.frag_slot = a->frag_slot;
@@ -1003,7 +1003,6 @@ static int gather_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const s
               ((((uintptr_t)a->ring.base | a->ring.slot_size) & 15u) ? 0u : kOptHdrChunk);
     if (half) {
       if (a->slot_state) return kNoShare;
-      half->sh.g = ga;
       const uint32_t lng = ga.pieces > 1 ? 1u : 0u;
       if (small_all) {
         const uint32_t per_group = kWave / small_all * kWavesPerBlock;
@@ -1015,7 +1014,6 @@ static int gather_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const s
       half->g_grid = grid;
       half->cursor[0] = packed ? sc.cursor[0] : nullptr;
       half->self[0] = self_advance;
-      half->fin[0] = finish_args(sc, half->cursor[0], a->fixed_req_size, app.cap, a->n_req, a->counts, nullptr, 0, 0, false);
       return SG_OK;
     }
     if (self_advance) ga.call_seq = ++*sc.call_seq;
@@ -1147,7 +1145,8 @@ static int scatter_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const 
     const uint32_t n_items = (uint32_t)(per * a->n_req);
     if (app.n_tensors == 0 ? a->fixed_resp_size > app.cap : a->fixed_resp_size > max_req_bytes)
       return fail(c, SG_E_INVAL, "response size %llu does not fit its source", (unsigned long long)a->fixed_resp_size);
-    ScatterArgs sa;
+    ScatterArgs own;
+    ScatterArgs &sa = half ? half->sh.s : own;
     memset(&sa, 0, sizeof sa);
     sa.hdr_src_slot = a->hdr_src_slot;
     sa.hdr_templates = a->hdr_templates;
@@ -1212,12 +1211,10 @@ static int scatter_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const 
         half->s_small_grid = ((small_all ? n_items : a->n_req) + per_group - 1) / per_group;
       }
       if (!small_all) geometry((uint64_t)a->n_req * sa.rule.per_launch * sa.pieces, !(a->flags & SG_F_NO_XCD_REMAP), &half->s_grid, &sa.remap);
-      half->sh.s = sa;
       half->sh.s_long = !small_all && sa.pieces > 1;
       half->full_csum = full_csum;
       half->cursor[1] = packed ? sc.cursor[1] : nullptr;
       half->self[1] = self_advance;
-      half->fin[1] = finish_args(sc, half->cursor[1], a->fixed_resp_size, app.cap, a->n_req, a->counts, nullptr, 0, 1, false);
       return SG_OK;
     }
     if (self_advance) sa.rule.call_seq = ++*sc.call_seq;
@@ -1359,10 +1356,52 @@ int sg_hip_scatter_batch(sg_hip_ctx *c, const sg_scatter_args *a)
 
 // ---- both directions in one launch ---------------------------------------------
 
-static bool ranges_overlap(const void *a, uint64_t an, const void *b, uint64_t bn)
+// Memory of a call: [at, end), empty for a null pointer.
+struct Range {
+  uintptr_t at, end;
+};
+static Range range(const void *p, uint64_t bytes) { return Range{(uintptr_t)p, (uintptr_t)p + (p ? bytes : 0u)}; }
+static bool meet(const Range &x, const Range &y) { return x.at < y.end && y.at < x.end && x.at != x.end && y.at != y.end; }
+
+// Application memory is an arena or, tensor-major, n_req rows per tensor.
+static uint32_t app_ranges(const sg_app_desc &app, uint32_t n_req, Range *out)
 {
-  const uintptr_t a0 = (uintptr_t)a, b0 = (uintptr_t)b;
-  return a0 < b0 + bn && b0 < a0 + an;
+  if (app.n_tensors == 0) {
+    out[0] = range(app.arena, app.arena_cap << (app.arena_mirrored ? 1 : 0));
+    return 1;
+  }
+  uint32_t k = 0;
+  for (; k < app.n_tensors && k < SG_MAX_TENSORS; k++) out[k] = range(app.tensor_base[k], app.tensor_size[k] * n_req);
+  return k;
+}
+
+// What the gather writes (requests, offsets) against everything the scatter touches (responses, the
+// ring its headers come from, TX slots, tables), and what the scatter writes (TX slots, offsets)
+// against what the gather reads: halves that touch each other's memory run one after the other.
+// (25 ns of the calling thread; 37 with every pair gone through whatever the ones before it said.)
+static bool halves_apart(const sg_gather_args *g, const sg_scatter_args *s)
+{
+  const uint64_t gn = g->n_req, gf = g->n_frags, sn = s->n_req, sf = s->n_frames;
+  const Range tx = range(s->tx.base, (uint64_t)s->tx.n_slots * s->tx.slot_size);
+  const Range s_offs = range(s->offsets_out, (sn + 1) * 8);
+  const Range g_reads[] = {range(g->ring.base, (uint64_t)g->ring.n_slots * g->ring.slot_size), range(g->frag_slot, gf * 4),
+                           range(g->frag_len, gf * 4), range(g->req_first, (gn + 1) * 4), range(g->counts, 16)};
+  for (const Range &r : g_reads)
+    if (meet(tx, r) || meet(s_offs, r)) return false;
+  Range resp[SG_MAX_TENSORS], req[SG_MAX_TENSORS + 1];
+  const uint32_t n_resp = app_ranges(s->app, s->n_req, resp);
+  uint32_t n_req = app_ranges(g->app, g->n_req, req);
+  req[n_req++] = range(g->offsets_out, (gn + 1) * 8);
+  const Range s_all[] = {tx, s_offs, range(s->rx.base, (uint64_t)s->rx.n_slots * s->rx.slot_size), range(s->tx_slot, sf * 4),
+                         range(s->hdr_src_slot, sf * 4), range(s->hdr_src_req, sn * 4), range(s->resp_first, (sn + 1) * 4),
+                         range(s->hdr_templates, sn * 64), range(s->req_token, sn * 8), range(s->counts, 16)};
+  for (uint32_t k = 0; k < n_req; k++) {
+    for (const Range &r : s_all)
+      if (meet(req[k], r)) return false;
+    for (uint32_t j = 0; j < n_resp; j++)
+      if (meet(req[k], resp[j])) return false;
+  }
+  return true;
 }
 
 int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_args *s)
@@ -1370,40 +1409,6 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
   if (!c || !g || !s) return fail(c, SG_E_INVAL, "null argument");
   DeviceGuard guard(c->device);
   const uint32_t async = g->flags & s->flags & SG_F_ASYNC;
-  // What the gather writes (requests, offsets) against everything the scatter touches (responses, the
-  // ring its headers come from, TX slots, tables), and what the scatter writes (TX slots, offsets)
-  // against what the gather reads: halves that touch each other's memory run one after the other.
-  // Application memory is an arena or, tensor-major, n_req rows per tensor.
-  struct Range { const void *p; uint64_t n; };
-  auto app_ranges = [](const sg_app_desc &app, uint32_t n_req, Range *out) {
-    uint32_t k = 0;
-    if (app.n_tensors == 0) out[k++] = Range{app.arena, app.arena_cap * (app.arena_mirrored ? 2u : 1u)};
-    else
-      for (uint32_t t = 0; t < app.n_tensors && t < SG_MAX_TENSORS; t++)
-        out[k++] = Range{app.tensor_base[t], app.tensor_size[t] * n_req};
-    return k;
-  };
-  auto table = [](const void *p, uint64_t bytes) { return Range{p, p ? bytes : 0u}; };
-  const uint64_t gn = g->n_req, gf = g->n_frags, sn = s->n_req, sf = s->n_frames;
-  const Range g_rx{g->ring.base, (uint64_t)g->ring.n_slots * g->ring.slot_size};
-  const Range s_rx{s->rx.base, (uint64_t)s->rx.n_slots * s->rx.slot_size};
-  const Range s_tx{s->tx.base, (uint64_t)s->tx.n_slots * s->tx.slot_size};
-  const Range s_offs = table(s->offsets_out, (sn + 1) * 8);
-  Range gw[SG_MAX_TENSORS + 1], st[SG_MAX_TENSORS + 10];
-  uint32_t n_gw = app_ranges(g->app, g->n_req, gw);
-  gw[n_gw++] = table(g->offsets_out, (gn + 1) * 8);
-  uint32_t n_st = app_ranges(s->app, s->n_req, st);
-  const Range s_more[] = {s_tx, s_rx, s_offs, table(s->tx_slot, sf * 4), table(s->hdr_src_slot, sf * 4),
-                          table(s->hdr_src_req, sn * 4), table(s->resp_first, (sn + 1) * 4),
-                          table(s->hdr_templates, sn * 64), table(s->req_token, sn * 8), table(s->counts, 16)};
-  for (const Range &r : s_more) st[n_st++] = r;
-  const Range g_reads[] = {g_rx, table(g->frag_slot, gf * 4), table(g->frag_len, gf * 4), table(g->req_first, (gn + 1) * 4),
-                           table(g->counts, 16)};
-  auto meet = [](const Range &x, const Range &y) { return x.n && y.n && ranges_overlap(x.p, x.n, y.p, y.n); };
-  bool apart = true;
-  for (uint32_t i = 0; i < n_gw; i++)
-    for (uint32_t j = 0; j < n_st; j++) apart = apart && !meet(gw[i], st[j]);
-  for (const Range &r : g_reads) apart = apart && !meet(s_tx, r) && !meet(s_offs, r);
   // Both halves are looked at before either is launched: a call the host refuses launches nothing.
   // A half that cannot share a launch leaves no trace; both are then made as calls of their own.
   ShuntHalf h;
@@ -1411,7 +1416,7 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
   if (rg < 0) return rg;
   const int rs = scatter_impl(c, c->sc, c->stream, s, &h);
   if (rs < 0) return rs;
-  if (apart && rg == SG_OK && rs == SG_OK) {
+  if (rg == SG_OK && rs == SG_OK && halves_apart(g, s)) {
     ShuntArgs &sh = h.sh;
     // the kernel advances the cursors itself where each half's own would; a workgroup for either
     // direction behind it does otherwise
@@ -1457,8 +1462,9 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
       uint32_t n = 0;
       for (int k = 0; k < 2; k++) {
         if (!h.cursor[k]) continue;
-        h.fin[k].clamp = h.self[k] ? 1u : 0u;  // as in the call of its own
-        p.h[n++] = h.fin[k];
+        p.h[n] = k == 0 ? finish_args(c->sc, h.cursor[0], g->fixed_req_size, g->app.arena_cap, g->n_req, g->counts, nullptr, 0, 0, false)
+                        : finish_args(c->sc, h.cursor[1], s->fixed_resp_size, s->app.arena_cap, s->n_req, s->counts, nullptr, 0, 1, false);
+        p.h[n++].clamp = h.self[k] ? 1u : 0u;  // as in the call of its own
       }
       if (n == 1) p.h[1] = p.h[0];
       k_finish<<<n, kBlock, 0, st>>>(p);
