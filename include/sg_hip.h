@@ -489,10 +489,12 @@ int sg_hip_gather_batch_static(int device_id, void *stream, const sg_gather_args
  * Synchronous unless SG_F_ASYNC is set; then counts_host_out is not written and
  * the counts are where counts_out says.  counts_host_out (4 words, or NULL):
  * requests completed, their fragments, arrivals dropped, requests still in
- * flight.  The first call on a context allocates the request table and the
- * its records (32 KiB per request of max_reqs; less where the device has no
- * room for that): make it, or
- * sg_hip_reassemble_reset, before recording calls into a graph. */
+ * flight.  The first call on a context allocates the request table with its
+ * records: 8 KiB per request of max_reqs (rounded up to a power of two), and
+ * two or four times that, which makes it a little faster, where the room
+ * beyond is at most a 64th of the device's free memory.  It holds max_reqs
+ * requests either way.  Make that call, or sg_hip_reassemble_reset, before
+ * recording calls into a graph. */
 int sg_hip_reassemble(sg_hip_ctx *ctx, const sg_reassemble_args *args, uint32_t *counts_host_out);
 
 /* Drops every request in flight (and allocates the state on first use). */

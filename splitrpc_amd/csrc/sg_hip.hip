@@ -128,7 +128,7 @@ struct sg_hip_ctx {
   uint64_t prof_n[6] = {0, 0, 0, 0, 0, 0};
   // reassembly scratch, allocated by the first sg_hip_reassemble call
   void *ra_mem = nullptr;
-  uint32_t ra_cells = 0;    // cells of the request table (power of two >= 4 * max_reqs)
+  uint32_t ra_cells = 0;    // cells of the request table: 4, 2 or 1 per request of max_reqs
   uint32_t *h_counts = nullptr;  // pinned: requests, fragments, dropped, in flight (written by the reassembly's kernels themselves)
   char err[512] = {0};
 };
@@ -515,6 +515,23 @@ static void launch_gather_rule(hipStream_t st, const GatherRuleArgs &ga, uint32_
   } else {
     if (ga.pieces > 1) k_gather_rule<true, 0, ADV><<<grid, kBlock, 0, st>>>(ga);
     else k_gather_rule<false, 0, ADV><<<grid, kBlock, 0, st>>>(ga);
+  }
+}
+
+// The reassembly's kernels.  SPILL: the table has fewer than four cells per request.
+template <bool SPILL>
+static void ra_launch(hipStream_t st, const RaArgs &r, uint32_t n_arrivals)
+{
+  if (n_arrivals <= (uint32_t)kRaSmallBurst) {
+    k_ra_burst<kRaSmallBurst, SPILL><<<1, kRaSmallBurst, 0, st>>>(r);
+  } else if (n_arrivals <= (uint32_t)kRaBurst) {
+    // a NIC burst (an empty one still leaves its counts): one workgroup, one launch
+    k_ra_burst<kRaBurst, SPILL><<<1, kRaBurst, 0, st>>>(r);
+  } else {
+    const uint32_t grid = (n_arrivals + kRaBlock - 1) / kRaBlock;
+    k_ra_insert<kRaBlock, SPILL><<<grid, kRaBlock, 0, st>>>(r);
+    k_ra_flag<kRaBlock><<<grid, kRaBlock, 0, st>>>(r);
+    k_ra_emit<kRaBlock><<<grid, kRaBlock, 0, st>>>(r);
   }
 }
 
@@ -1609,6 +1626,13 @@ uint32_t pow2_at_least(uint64_t v)
   return p;
 }
 
+// Cells of the request table for requests of which `of` may be in flight, `each` for every one.
+uint64_t ra_cells_for(uint32_t of, uint32_t each)
+{
+  const uint64_t cells = (uint64_t)each * pow2_at_least(of);
+  return cells < 2 * kRaBucket ? 2 * kRaBucket : cells;
+}
+
 // Carves the reassembly state out of c->ra_mem (allocating it first where needed).
 int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
 {
@@ -1621,23 +1645,28 @@ int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
       HIP_TRY(c, hipHostMalloc((void **)&c->h_counts, 4 * sizeof(uint32_t), hipHostMallocDefault));
       memset(c->h_counts, 0, 4 * sizeof(uint32_t));
     }
-    // Four cells for every request that may be in flight: a bucket of 32 then holds 8 on average and
-    // never fills up.  Where the device has no room for that many records (32 KiB per request), fewer:
-    // a bucket may then be full before max_reqs are in flight, which refuses the call that finds it so.
-    const uint32_t least = pow2_at_least(c->max_reqs);
-    uint32_t cells = pow2_at_least(4ull * c->max_reqs < 2 * kRaBucket ? 2 * kRaBucket : 4ull * c->max_reqs);
+    const uint64_t least = ra_cells_for(c->max_reqs, 1);
+    auto bytes = [&](uint64_t cells) {
+      return cells * (SG_MAX_BI_SIZE * 8 + 8 + 8 + 3 * 4) + cells / kRaBucket * 4 + kRaWords * 4 + (uint64_t)n_max * (8 + 4) +
+             n_blk * 2 * 8 + 256;
+    };
+    // Four cells per request that may be in flight where the room beyond one cell each is at most a
+    // 64th of what the device has free (3 GiB for 131072 requests); else two, else one.
+    size_t avail = 0, total = 0;
+    HIP_TRY(c, hipMemGetInfo(&avail, &total));
+    uint64_t cells = ra_cells_for(c->max_reqs, 4);
+    while (cells > least && bytes(cells) - bytes(least) > avail / 64) cells >>= 1;
     for (;;) {
-      const size_t bytes = (size_t)cells * (SG_MAX_BI_SIZE * 8 + 8 + 8 + 3 * 4) + kRaWords * 4 + (size_t)n_max * (8 + 4) +
-                           n_blk * 2 * 8 + 256;
-      const hipError_t e = hipMalloc(&c->ra_mem, bytes);
+      const hipError_t e = hipMalloc(&c->ra_mem, bytes(cells));
       if (e == hipSuccess) break;
       c->ra_mem = nullptr;
       (void)hipGetLastError();
-      if (e != hipErrorOutOfMemory || cells <= least || cells <= 2 * kRaBucket)
-        return fail(c, SG_E_NOMEM, "request table of %zu bytes: %s", bytes, hipGetErrorString(e));
+      if (e != hipErrorOutOfMemory || cells <= least)
+        return fail(c, e == hipErrorOutOfMemory ? SG_E_NOMEM : SG_E_HIP, "request table of %zu bytes: %s", (size_t)bytes(cells),
+                    hipGetErrorString(e));
       cells >>= 1;
     }
-    c->ra_cells = cells;
+    c->ra_cells = (uint32_t)cells;
     *fresh = true;
   }
   const uint32_t cells = c->ra_cells;
@@ -1653,7 +1682,9 @@ int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
   r->last = reinterpret_cast<uint32_t *>(m); m += (size_t)cells * 4;
   r->seen = reinterpret_cast<uint32_t *>(m); m += (size_t)cells * 4;
   r->words = reinterpret_cast<uint32_t *>(m); m += kRaWords * 4;
+  r->reach = reinterpret_cast<uint32_t *>(m); m += (size_t)cells / kRaBucket * 4;
   r->arr_cell = reinterpret_cast<uint32_t *>(m);
+  r->cells = cells;
   r->bmask = cells / kRaBucket - 1;
   r->pool = pow2_at_least(c->max_reqs);
   r->counts_host = c->h_counts;
@@ -1665,7 +1696,7 @@ int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
 void ra_launch_reset(sg_hip_ctx *c, const RaArgs &r)
 {
   const size_t items = (size_t)c->ra_cells * (SG_MAX_BI_SIZE / 2);  // two entries per thread: more than there are cells
-  k_ra_reset<<<(uint32_t)((items + 255) / 256), 256, 0, c->stream>>>(r, c->ra_cells);
+  k_ra_reset<<<(uint32_t)((items + 255) / 256), 256, 0, c->stream>>>(r);
 }
 
 }  // namespace
@@ -1693,7 +1724,7 @@ int sg_hip_reassemble_evict(sg_hip_ctx *c, uint32_t max_age_calls, uint32_t *n_e
   int rc = ra_state(c, &r, &fresh);
   if (rc != SG_OK) return rc;
   k_zero_words<<<1, kBlock, 0, c->stream>>>(r.words + kRaEvicted, 1);
-  k_ra_evict<<<(c->ra_cells + kWavesPerBlock - 1) / kWavesPerBlock, kBlock, 0, c->stream>>>(r, c->ra_cells, max_age_calls);
+  k_ra_evict<<<(c->ra_cells + kWavesPerBlock - 1) / kWavesPerBlock, kBlock, 0, c->stream>>>(r, max_age_calls);
   rc = finish(c, 0);
   if (rc != SG_OK) return rc;
   uint32_t n = 0;
@@ -1740,17 +1771,8 @@ int sg_hip_reassemble(sg_hip_ctx *c, const sg_reassemble_args *a, uint32_t *coun
 
   rc = prof_begin(c, 5);
   if (rc != SG_OK) return rc;
-  if (a->n_arrivals <= (uint32_t)kRaSmallBurst) {
-    k_ra_burst<kRaSmallBurst><<<1, kRaSmallBurst, 0, c->stream>>>(r);
-  } else if (a->n_arrivals <= (uint32_t)kRaBurst) {
-    // a NIC burst (an empty one still leaves its counts): one workgroup, one launch
-    k_ra_burst<kRaBurst><<<1, kRaBurst, 0, c->stream>>>(r);
-  } else {
-    const uint32_t grid = (a->n_arrivals + kRaBlock - 1) / kRaBlock;
-    k_ra_insert<kRaBlock><<<grid, kRaBlock, 0, c->stream>>>(r);
-    k_ra_flag<kRaBlock><<<grid, kRaBlock, 0, c->stream>>>(r);
-    k_ra_emit<kRaBlock><<<grid, kRaBlock, 0, c->stream>>>(r);
-  }
+  if (c->ra_cells < ra_cells_for(c->max_reqs, 4)) ra_launch<true>(c->stream, r, a->n_arrivals);
+  else ra_launch<false>(c->stream, r, a->n_arrivals);
   rc = prof_end(c);
   if (rc != SG_OK) return rc;
   rc = finish(c, a->flags);

@@ -21,7 +21,11 @@ namespace {
 //   request table   token -> cell, open addressing in buckets of kRaBucket
 //                   cells: a lookup reads the whole bucket, so emptying a cell
 //                   (a completed request) never hides another request, and a
-//                   new token claims an empty cell by atomicCAS
+//                   new token claims an empty cell by atomicCAS.  Four cells per
+//                   request that may be in flight, and a token belongs to one
+//                   bucket; or, to save memory, two or one (SPILL), and a full
+//                   bucket sends its tokens on to others and keeps count of how
+//                   far (`reach`)
 //   records         every cell has a record of its own: SG_MAX_BI_SIZE entries
 //                   {slot, length} indexed by sequence number (p2p_bufs of the
 //                   reference's rr).  The cell a token is found in says where
@@ -56,10 +60,10 @@ namespace {
 // (a launch that does nothing shows as 2 to 4 us there).  Workgroups of 512 threads: 11.9 / 5.2 / 6.0
 // and 14.0 / 5.1 / 9.4; of 1024: 12.2 / 5.2 / 5.8 and 20.5 / 6.8 / 10.8.  The ring of free records
 // cost a returning addition per workgroup to one word, 35 to 70 ns each and one after the other, and
-// two dependent reads per new request; a record per cell takes four times the room.
+// two dependent reads per new request.
 
 constexpr uint32_t kRaBucket = 32;
-static_assert(kRaBucket == 32, "ra_find_cell keeps one bit per cell and takes a token's first cell from the top five bits of its hash");
+static_assert(kRaBucket == 32, "ra_look keeps one bit per cell; a token's first cell is the top five bits of its hash");
 constexpr uint32_t kRaNoCell = 0x7fffffffu;
 // beside the cell of an arrival: its thread is the one that went to the table for the token
 constexpr uint32_t kRaOwner = 0x80000000u;
@@ -77,11 +81,12 @@ struct RaArgs {
   const uint32_t *arrivals;
   const uint32_t *len_nic;
   uint64_t req_size;  // REF64 readiness: bytes == req_size; BL58: fragments == num_frags
-  uint32_t bmask;     // buckets - 1
+  uint32_t cells, bmask;  // cells; buckets - 1
   uint32_t pool;      // requests that may be in flight
   uint32_t max_req, max_frag;  // room in the output tables
   // request table: cells
   unsigned long long *keys;
+  uint32_t *reach;           // per bucket: how many buckets further a token whose first bucket it is may sit
   unsigned long long *acc;   // fragments so far << 40 | payload bytes so far: one atomic addition per workgroup and token
   uint32_t *last;            // position in this call of the token's latest arrival; zero between calls
   uint32_t *want, *seen;     // fragments of the request; epoch of the latest call that brought one
@@ -147,9 +152,30 @@ __device__ __forceinline__ unsigned long long ra_key(const unsigned long long *p
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Find or claim the cell of `token`.  The whole bucket is read first, all of it asked for at once:
-// the request may sit anywhere in it (cells empty as requests complete).  Only then
-// is an empty cell claimed.  Every token walks the bucket in an order of its
+// The cells of a bucket that hold `token`, and those that are empty, a bit each.
+struct RaSeen {
+  uint32_t found, empty;
+};
+__device__ __forceinline__ RaSeen ra_look(const RaArgs &a, uint32_t b, unsigned long long token)
+{
+  // Ordinary 16-byte loads, two keys each, all of them asked for at once.  While arrivals are being
+  // filed a key only ever goes from empty to a token, so all a load that is behind the times can show
+  // is an empty cell that has just been taken -- and a claim goes through atomicCAS, which then
+  // returns the taker (this thread's own token included).
+  const ulonglong2 *kp = reinterpret_cast<const ulonglong2 *>(a.keys + b);
+  ulonglong2 v[kRaBucket / 2];
+#pragma unroll
+  for (uint32_t j = 0; j < kRaBucket / 2; j++) v[j] = kp[j];
+  RaSeen s = {0u, 0u};
+#pragma unroll
+  for (uint32_t j = 0; j < kRaBucket / 2; j++) {
+    s.found |= (v[j].x == token ? 1u << (2 * j) : 0u) | (v[j].y == token ? 2u << (2 * j) : 0u);
+    s.empty |= (v[j].x == 0ull ? 1u << (2 * j) : 0u) | (v[j].y == 0ull ? 2u << (2 * j) : 0u);
+  }
+  return s;
+}
+
+// Claims a cell of a bucket that showed empty ones.  Every token walks a bucket in an order of its
 // own -- cyclically from a cell its hash picks -- starting at the first cell of
 // that order it has seen empty and trying every empty cell on the way; cells
 // before that one in the order were taken when they were read and stay taken
@@ -158,27 +184,9 @@ __device__ __forceinline__ unsigned long long ra_key(const unsigned long long *p
 // order for all tokens -- lowest cell first -- the new requests of a burst that
 // share a bucket queued up on its lowest empty cells, one failed
 // compare-and-swap round trip after the other.)
-__device__ __forceinline__ uint32_t ra_find_cell(const RaArgs &a, unsigned long long token, uint32_t hash, bool *claimed)
+__device__ __forceinline__ uint32_t ra_claim(const RaArgs &a, uint32_t b, unsigned long long token, uint32_t start, uint32_t empty,
+                                             bool *claimed)
 {
-  const uint32_t b = (hash & a.bmask) * kRaBucket;
-  const uint32_t start = hash >> 27;  // the top five bits: the bucket takes the low ones
-  *claimed = false;
-  // Ordinary 16-byte loads, two keys each.  While arrivals are being filed a key only ever goes
-  // from empty to a token, so all a load that is behind the times can show is an empty cell that
-  // has just been taken -- and the claim below goes through atomicCAS, which then returns the
-  // taker (this thread's own token included).
-  const ulonglong2 *kp = reinterpret_cast<const ulonglong2 *>(a.keys + b);
-  ulonglong2 v[kRaBucket / 2];
-#pragma unroll
-  for (uint32_t j = 0; j < kRaBucket / 2; j++) v[j] = kp[j];
-  uint32_t found = 0, empty = 0;  // a bit per cell
-#pragma unroll
-  for (uint32_t j = 0; j < kRaBucket / 2; j++) {
-    found |= (v[j].x == token ? 1u << (2 * j) : 0u) | (v[j].y == token ? 2u << (2 * j) : 0u);
-    empty |= (v[j].x == 0ull ? 1u << (2 * j) : 0u) | (v[j].y == 0ull ? 2u << (2 * j) : 0u);
-  }
-  if (found) return b + (uint32_t)__ffs((int)found) - 1;
-  if (!empty) return kRaNoCell;
   // place in this token's order of the first cell seen empty
   const uint32_t turned = start ? (empty >> start) | (empty << (32u - start)) : empty;
   const uint32_t first_rank = (uint32_t)__ffs((int)turned) - 1;
@@ -195,7 +203,61 @@ __device__ __forceinline__ uint32_t ra_find_cell(const RaArgs &a, unsigned long 
     }
     if (k == token) return b + j;
   }
-  return kRaNoCell;  // bucket full
+  return kRaNoCell;  // taken by others meanwhile
+}
+
+// Find or claim the cell of `token`.
+//
+// SPILL: every token has an order of buckets -- its first, then on by an odd stride of its own, which
+// comes past all of them -- and sits in the first of them that was not full when it came.  It is looked
+// for as far as any token has gone from its first bucket (mostly nowhere: `reach`), and only then
+// claimed, in the first bucket that shows an empty cell.  Buckets before that one were full when they
+// were read and stay so while arrivals are being filed, so here too all who bring the same new token
+// meet.  `full`: every cell was taken before this call, nothing is to be claimed.  65536 interleaved
+// requests of two fragments into 131072 cells take 56 us (43 us with four cells each), 98304 take 107
+// (57); the last per mille of a table looks through many buckets, at most kRaFar.  Bursts of 64 take
+// 8.1 us (6.8): a table that need not does without.
+constexpr uint32_t kRaFar = 1023;
+template <bool SPILL>
+__device__ __forceinline__ uint32_t ra_find_cell(const RaArgs &a, unsigned long long token, uint32_t hash, bool full, bool *claimed)
+{
+  const uint32_t first = hash & a.bmask;
+  const uint32_t start = hash >> 27;  // the top five bits: the bucket takes the low ones
+  *claimed = false;
+  if (!SPILL) {
+    const uint32_t b = first * kRaBucket;
+    const RaSeen s = ra_look(a, b, token);
+    if (s.found) return b + (uint32_t)__ffs((int)s.found) - 1;
+    return s.empty ? ra_claim(a, b, token, start, s.empty, claimed) : kRaNoCell;
+  }
+  const uint32_t stride = (hash >> 13) | 1u;
+  const uint32_t reach = a.reach[first];
+  const uint32_t far = a.bmask < kRaFar ? a.bmask : kRaFar;
+  uint32_t at = ~0u, empty = 0;  // the first bucket of the order with empty cells
+  uint32_t k = 0;
+#pragma unroll 1
+  for (;;) {
+    const uint32_t b = ((first + k * stride) & a.bmask) * kRaBucket;
+    const RaSeen s = ra_look(a, b, token);
+    if (s.found) return b + (uint32_t)__ffs((int)s.found) - 1;
+    if (at == ~0u && s.empty) {
+      at = k;
+      empty = s.empty;
+    }
+    if (k < far && (k < reach || (at == ~0u && !full))) {
+      k++;
+      continue;
+    }
+    if (at == ~0u) return kRaNoCell;
+    const uint32_t c = ra_claim(a, ((first + at * stride) & a.bmask) * kRaBucket, token, start, empty, claimed);
+    if (c != kRaNoCell) {
+      if (*claimed && at) atomicMax(&a.reach[first], at);  // for later calls
+      return c;
+    }
+    k = at + 1;  // its empty cells went to others meanwhile: on to the next
+    at = ~0u;
+    if (k > far) return kRaNoCell;
+  }
 }
 
 // The distinct tokens among a workgroup's arrivals, open addressing in LDS, twice as many entries
@@ -344,7 +406,7 @@ __device__ __forceinline__ unsigned long long ra_count_new(bool claimed, bool lo
   return t;
 }
 
-template <int B>
+template <int B, bool SPILL>
 __global__ __launch_bounds__(B) void k_ra_insert(RaArgs a)
 {
   __shared__ RaLds<B> l;
@@ -355,6 +417,7 @@ __global__ __launch_bounds__(B) void k_ra_insert(RaArgs a)
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const bool in_range = i < n;
   const uint32_t epoch = sload(a.words + kRaEpoch);  // advanced by k_ra_emit, two kernels behind
+  const bool full = SPILL && sload(a.words + kRaInFlight) >= a.cells;
   const RaMine m = ra_read(a, i, in_range);
   ra_lds_clear(l);
   __syncthreads();
@@ -363,7 +426,7 @@ __global__ __launch_bounds__(B) void k_ra_insert(RaArgs a)
   const uint32_t e = ra_group<B>(l, m, hash, lane, &owner);
   __syncthreads();
   if (owner) {
-    const uint32_t c = ra_find_cell(a, m.token, hash, &claimed);
+    const uint32_t c = ra_find_cell<SPILL>(a, m.token, hash, full, &claimed);
     l.cell[e] = c;
     if (c != kRaNoCell) {
       atomicAdd(&a.acc[c], l.acc[e]);
@@ -371,7 +434,7 @@ __global__ __launch_bounds__(B) void k_ra_insert(RaArgs a)
       a.seen[c] = epoch;
       if (!a.ref64) a.want[c] = m.want;  // every fragment of a request says the same
     } else {
-      refuse(a.status, a.status_flag, kStPoolFull);  // bucket full
+      refuse(a.status, a.status_flag, kStPoolFull);
     }
   }
   __syncthreads();
@@ -589,7 +652,7 @@ __global__ __launch_bounds__(B) void k_ra_emit(RaArgs a)
 // A burst that one workgroup takes, which is what a NIC delivers: the three steps in ONE kernel.
 // Nothing else touches the table meanwhile, so the owner of a token works on its cell with
 // ordinary loads and stores and hands the new total to the token's other arrivals through LDS.
-template <int B>
+template <int B, bool SPILL>
 __global__ __launch_bounds__(B) void k_ra_burst(RaArgs a)
 {
   __shared__ RaLds<B> l;
@@ -600,6 +663,7 @@ __global__ __launch_bounds__(B) void k_ra_burst(RaArgs a)
   const uint32_t lane = i & (kWave - 1);
   const bool in_range = i < n;
   const uint32_t epoch = a.words[kRaEpoch];
+  const bool full = SPILL && a.words[kRaInFlight] >= a.cells;
   const RaMine m = ra_read(a, i, in_range);
   ra_lds_clear(l);
   __syncthreads();
@@ -608,7 +672,7 @@ __global__ __launch_bounds__(B) void k_ra_burst(RaArgs a)
   const uint32_t e = ra_group<B>(l, m, hash, lane, &owner);
   __syncthreads();
   if (owner) {
-    const uint32_t c = ra_find_cell(a, m.token, hash, &claimed);
+    const uint32_t c = ra_find_cell<SPILL>(a, m.token, hash, full, &claimed);
     l.cell[e] = c;
     if (c != kRaNoCell) {
       const unsigned long long acc = (claimed ? 0ull : a.acc[c]) + l.acc[e];  // an empty cell's total is zero
@@ -616,7 +680,7 @@ __global__ __launch_bounds__(B) void k_ra_burst(RaArgs a)
       l.acc[e] = acc;
       a.seen[c] = epoch;
     } else {
-      refuse(a.status, a.status_flag, kStPoolFull);  // bucket full
+      refuse(a.status, a.status_flag, kStPoolFull);
     }
   }
   __syncthreads();
@@ -640,16 +704,17 @@ __global__ __launch_bounds__(B) void k_ra_burst(RaArgs a)
 }
 
 // Empties the table: every cell, every record.
-__global__ __launch_bounds__(256) void k_ra_reset(RaArgs a, uint32_t cells)
+__global__ __launch_bounds__(256) void k_ra_reset(RaArgs a)
 {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < cells) {
+  if (i < a.cells) {
     a.keys[i] = 0;
     a.acc[i] = 0;
     a.last[i] = a.want[i] = a.seen[i] = 0;
+    if (i <= a.bmask) a.reach[i] = 0;
   }
   // two entries per thread
-  if (2 * i < (size_t)cells * SG_MAX_BI_SIZE) reinterpret_cast<u32x4 *>(a.tab)[i] = (u32x4){0u, 0u, 0u, 0u};
+  if (2 * i < (size_t)a.cells * SG_MAX_BI_SIZE) reinterpret_cast<u32x4 *>(a.tab)[i] = (u32x4){0u, 0u, 0u, 0u};
   if (i < kRaWords) a.words[i] = 0;
 }
 
@@ -657,11 +722,11 @@ __global__ __launch_bounds__(256) void k_ra_reset(RaArgs a, uint32_t cells)
 // (a lost fragment parks its request for good in the reference,
 // src/p2p_rpc_rr_pool_ng.h:57-64; here the caller can clear such requests out).
 // One wavefront per cell.
-__global__ __launch_bounds__(256) void k_ra_evict(RaArgs a, uint32_t cells, uint32_t max_age)
+__global__ __launch_bounds__(256) void k_ra_evict(RaArgs a, uint32_t max_age)
 {
   const uint32_t c = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
   const uint32_t lane = threadIdx.x & (kWave - 1);
-  if (c >= cells) return;
+  if (c >= a.cells) return;
   if (a.keys[c] == 0ull) return;
   if (a.words[kRaEpoch] - a.seen[c] <= max_age) return;
   unsigned long long *t = a.tab + (size_t)c * SG_MAX_BI_SIZE;
