@@ -129,6 +129,7 @@ struct sg_hip_ctx {
   // reassembly scratch, allocated by the first sg_hip_reassemble call
   void *ra_mem = nullptr;
   uint32_t ra_cells = 0;    // cells of the request table: 4, 2 or 1 per request of max_reqs
+  bool ra_clean = false;    // the table has been emptied since it was allocated
   uint32_t *h_counts = nullptr;  // pinned: requests, fragments, dropped, in flight (written by the reassembly's kernels themselves)
   char err[512] = {0};
 };
@@ -1634,11 +1635,10 @@ uint64_t ra_cells_for(uint32_t of, uint32_t each)
 }
 
 // Carves the reassembly state out of c->ra_mem (allocating it first where needed).
-int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
+int ra_state(sg_hip_ctx *c, RaArgs *r)
 {
   const uint32_t n_max = c->max_frames;
   const size_t n_blk = ((size_t)n_max + kRaBlock - 1) / kRaBlock + 1;
-  *fresh = false;
   if (!c->ra_mem) {
     // the small allocation first: a context never holds the state without its pinned counts
     if (!c->h_counts) {
@@ -1667,7 +1667,6 @@ int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
       cells >>= 1;
     }
     c->ra_cells = (uint32_t)cells;
-    *fresh = true;
   }
   const uint32_t cells = c->ra_cells;
   memset(r, 0, sizeof *r);
@@ -1693,10 +1692,13 @@ int ra_state(sg_hip_ctx *c, RaArgs *r, bool *fresh)
   return SG_OK;
 }
 
-void ra_launch_reset(sg_hip_ctx *c, const RaArgs &r)
+int ra_launch_reset(sg_hip_ctx *c, const RaArgs &r)
 {
-  const size_t items = (size_t)c->ra_cells * (SG_MAX_BI_SIZE / 2);  // two entries per thread: more than there are cells
-  k_ra_reset<<<(uint32_t)((items + 255) / 256), 256, 0, c->stream>>>(r);
+  const uint64_t groups = ((uint64_t)c->ra_cells * (SG_MAX_BI_SIZE / 2) + 255) / 256;  // two entries per thread
+  k_ra_reset<<<(uint32_t)(groups < 65536 ? groups : 65536), 256, 0, c->stream>>>(r);
+  HIP_TRY(c, hipGetLastError());
+  c->ra_clean = true;
+  return SG_OK;
 }
 
 }  // namespace
@@ -1706,10 +1708,10 @@ int sg_hip_reassemble_reset(sg_hip_ctx *c)
   if (!c) return SG_E_INVAL;
   DeviceGuard g(c->device);
   RaArgs r;
-  bool fresh;
-  int rc = ra_state(c, &r, &fresh);
+  int rc = ra_state(c, &r);
   if (rc != SG_OK) return rc;
-  ra_launch_reset(c, r);
+  rc = ra_launch_reset(c, r);
+  if (rc != SG_OK) return rc;
   return finish(c, 0);
 }
 
@@ -1717,11 +1719,10 @@ int sg_hip_reassemble_evict(sg_hip_ctx *c, uint32_t max_age_calls, uint32_t *n_e
 {
   if (!c) return SG_E_INVAL;
   if (n_evicted_out) *n_evicted_out = 0;
-  if (!c->ra_mem) return SG_OK;  // nothing has come in yet
+  if (!c->ra_clean) return SG_OK;  // nothing has come in yet
   DeviceGuard g(c->device);
   RaArgs r;
-  bool fresh;
-  int rc = ra_state(c, &r, &fresh);
+  int rc = ra_state(c, &r);
   if (rc != SG_OK) return rc;
   k_zero_words<<<1, kBlock, 0, c->stream>>>(r.words + kRaEvicted, 1);
   k_ra_evict<<<(c->ra_cells + kWavesPerBlock - 1) / kWavesPerBlock, kBlock, 0, c->stream>>>(r, max_age_calls);
@@ -1746,10 +1747,9 @@ int sg_hip_reassemble(sg_hip_ctx *c, const sg_reassemble_args *a, uint32_t *coun
   DeviceGuard g(c->device);
 
   RaArgs r;
-  bool fresh;
-  rc = ra_state(c, &r, &fresh);
+  rc = ra_state(c, &r);
+  if (rc == SG_OK && !c->ra_clean) rc = ra_launch_reset(c, r);
   if (rc != SG_OK) return rc;
-  if (fresh) ra_launch_reset(c, r);
   r.ring = static_cast<const uint8_t *>(a->ring.base);
   r.n_slots = a->ring.n_slots;
   r.slot_size = a->ring.slot_size;

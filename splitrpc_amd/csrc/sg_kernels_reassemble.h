@@ -703,19 +703,20 @@ __global__ __launch_bounds__(B) void k_ra_burst(RaArgs a)
   });
 }
 
-// Empties the table: every cell, every record.
+// Empties the table: every cell, every record.  Any grid: the records of millions of requests are
+// more than a launch has threads for.
 __global__ __launch_bounds__(256) void k_ra_reset(RaArgs a)
 {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < a.cells) {
+  const size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+  for (size_t i = i0; i < a.cells; i += step) {
     a.keys[i] = 0;
     a.acc[i] = 0;
     a.last[i] = a.want[i] = a.seen[i] = 0;
     if (i <= a.bmask) a.reach[i] = 0;
   }
-  // two entries per thread
-  if (2 * i < (size_t)a.cells * SG_MAX_BI_SIZE) reinterpret_cast<u32x4 *>(a.tab)[i] = (u32x4){0u, 0u, 0u, 0u};
-  if (i < kRaWords) a.words[i] = 0;
+  // two entries at a time
+  for (size_t i = i0; 2 * i < (size_t)a.cells * SG_MAX_BI_SIZE; i += step) reinterpret_cast<u32x4 *>(a.tab)[i] = (u32x4){0u, 0u, 0u, 0u};
+  if (i0 < kRaWords) a.words[i0] = 0;
 }
 
 // Drops the requests no fragment has come in for during the last max_age calls

@@ -135,3 +135,23 @@ def test_a_table_of_a_cell_per_request(share):
     assert call(2 * few[::-1] + 1) == (600, 1200, 0)
     assert np.array_equal(st.fs[:1200].cpu().numpy().reshape(-1, 2), 2 * few[::-1, None] + np.arange(2))
     ctx.close()
+
+
+def test_a_table_of_more_records_than_a_launch_has_threads():
+    """Eight million requests: 2^32 pairs of entries to empty."""
+    max_reqs = 1 << 23
+    if torch.cuda.mem_get_info()[0] < 90 << 30:
+        pytest.skip("the table takes 64 GiB")
+    print("case table of 2^23 cells", flush=True)
+    ctx = SgContext(0, max_reqs=max_reqs, max_frames=4096)
+    t = _tokens(2000, 11)
+    st = Stream(t, 2, 4096, 4096)
+    slots = np.random.default_rng(12).permutation(4000)
+    for _ in range(2):
+        st.call(ctx, slots[:3000])
+        st.parked.clear()
+        ctx.reassemble_reset()
+    st.call(ctx, slots[:3100])
+    st.call(ctx, slots[3100:])
+    assert not st.parked
+    ctx.close()
