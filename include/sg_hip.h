@@ -489,7 +489,11 @@ int sg_hip_gather_batch_static(int device_id, void *stream, const sg_gather_args
  * Synchronous unless SG_F_ASYNC is set; then counts_host_out is not written and
  * the counts are where counts_out says.  counts_host_out (4 words, or NULL):
  * requests completed, their fragments, arrivals dropped, requests still in
- * flight.  The first call on a context allocates the request table with its
+ * flight; also where the call returns SG_E_DATA, which takes nothing back: what
+ * completed has been handed over.  More than max_reqs requests (rounded up to a
+ * power of two) left in flight by a call is SG_E_DATA, though none of them is
+ * lost unless the table itself is full: arrivals that find no cell count as
+ * dropped.  The first call on a context allocates the request table with its
  * records: 8 KiB per request of max_reqs (rounded up to a power of two), and
  * two or four times that, which makes it a little faster, where the room
  * beyond is at most a 64th of the device's free memory.  It holds max_reqs

@@ -1776,9 +1776,10 @@ int sg_hip_reassemble(sg_hip_ctx *c, const sg_reassemble_args *a, uint32_t *coun
   rc = prof_end(c);
   if (rc != SG_OK) return rc;
   rc = finish(c, a->flags);
-  if (rc != SG_OK || (a->flags & SG_F_ASYNC)) return rc;
-  if (counts_host_out) memcpy(counts_host_out, c->h_counts, 4 * sizeof(uint32_t));
-  return SG_OK;
+  // a call that refused something has handed over what completed all the same
+  if ((rc == SG_OK || rc == SG_E_DATA) && !(a->flags & SG_F_ASYNC) && counts_host_out)
+    memcpy(counts_host_out, c->h_counts, 4 * sizeof(uint32_t));
+  return rc;
 }
 
 }  // extern "C"

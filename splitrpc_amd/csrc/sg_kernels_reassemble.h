@@ -488,10 +488,11 @@ __device__ __forceinline__ void ra_close(const RaArgs &a, uint64_t tot, unsigned
 {
   const uint32_t n_req = overflow ? 0u : (uint32_t)(tot >> 32), n_frag = overflow ? 0u : (uint32_t)tot;
   const uint32_t claims = (uint32_t)(fresh >> 32), before = a.words[kRaInFlight];
-  if (claims && before + claims > a.pool) refuse(a.status, a.status_flag, kStPoolFull);
+  const uint32_t in_flight = before + claims - n_req;
+  // more than the context was made for are left (not dropped: every one has its cell)
+  if (claims && in_flight > a.pool) refuse(a.status, a.status_flag, kStPoolFull);
   // the output tables cannot take what completed: nothing is emitted, the requests stay parked
   if (overflow) refuse(a.status, a.status_flag, kStBadTable);
-  const uint32_t in_flight = before + claims - n_req;
   a.req_first[n_req] = n_frag;
   a.words[kRaInFlight] = in_flight;
   a.words[kRaEpoch] += 1;

@@ -1,10 +1,13 @@
 """The request table of the reassembly at its limits: as many requests in flight
 as the context was made for, a table of a cell per request, tokens that share a
 bucket, how much of the device it takes -- against requests collected in a dict."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
+from splitrpc_amd import capi
 from splitrpc_amd.engine import RingRef, SgContext, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -153,5 +156,35 @@ def test_a_table_of_more_records_than_a_launch_has_threads():
         ctx.reassemble_reset()
     st.call(ctx, slots[:3100])
     st.call(ctx, slots[3100:])
+    assert not st.parked
+    ctx.close()
+
+
+@pytest.mark.parametrize("max_reqs", [64, 1024], ids=["one-launch", "three-kernels"])
+def test_requests_beyond_those_a_context_was_made_for(max_reqs):
+    """A call may bring more requests than may be in flight if it completes enough of them; one that leaves more is
+    refused, reports what it has handed over, and keeps the others."""
+    full, part = max_reqs - 4, max_reqs // 2
+    print(f"case table beyond max_reqs={max_reqs}", flush=True)
+    ctx = SgContext(0, max_reqs=max_reqs, max_frames=8192)
+    st = Stream(_tokens(full + part, 13), 2, max_reqs, 8192)
+    rng = np.random.default_rng(14)
+    st.call(ctx, rng.permutation(np.concatenate([np.arange(2 * full), 2 * np.arange(full, full + part)])))
+    st.call(ctx, 2 * rng.permutation(np.arange(full, full + part)) + 1)
+    assert not st.parked
+    # twenty complete, one more than fit stays
+    st = Stream(_tokens(20 + max_reqs + 1, 15), 2, max_reqs, 8192)
+    slots = np.concatenate([np.arange(40), 2 * np.arange(20, 21 + max_reqs)]).astype(np.uint32)
+    arr = to_dev(slots, DEV)
+    counts = (C.c_uint32 * 4)()
+    torch.cuda.synchronize()
+    a = ctx.reassemble_args(st.rx, arr, len(slots), st.fs, st.fl, st.rf, st.tok, counts_out=st.counts)
+    assert ctx.lib.sg_hip_reassemble(ctx.h, C.byref(a), C.byref(counts)) == capi.SG_E_DATA
+    assert list(counts) == st.counts.cpu().tolist() == [20, 40, 0, max_reqs + 1]
+    assert np.array_equal(st.fs[:40].cpu().numpy(), np.arange(40))
+    st.parked = {r: {2 * r} for r in range(20, 21 + max_reqs)}
+    late = 2 * rng.permutation(np.arange(20, 21 + max_reqs)) + 1
+    st.call(ctx, late[:30])
+    st.call(ctx, late[30:])
     assert not st.parked
     ctx.close()
