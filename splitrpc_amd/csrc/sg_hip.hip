@@ -532,7 +532,12 @@ static void ra_launch(hipStream_t st, const RaArgs &r, uint32_t n_arrivals)
     const uint32_t grid = (n_arrivals + kRaBlock - 1) / kRaBlock;
     k_ra_insert<kRaBlock, SPILL><<<grid, kRaBlock, 0, st>>>(r);
     k_ra_flag<kRaBlock><<<grid, kRaBlock, 0, st>>>(r);
-    k_ra_emit<kRaBlock><<<grid, kRaBlock, 0, st>>>(r);
+    if (grid <= kRaSumBlocks) {
+      k_ra_emit<kRaBlock, false><<<grid, kRaBlock, 0, st>>>(r);
+    } else {
+      k_ra_scan<kRaScan, kRaBlock><<<1, kRaScan, 0, st>>>(r);
+      k_ra_emit<kRaBlock, true><<<grid, kRaBlock, 0, st>>>(r);
+    }
   }
 }
 

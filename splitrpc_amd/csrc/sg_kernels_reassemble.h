@@ -42,7 +42,8 @@ namespace {
 //   k_ra_emit    batch index of a request = number of requests completed before
 //                it in this call (completion order, the order of the rx-ready
 //                ring); a wavefront in which requests complete adds up the
-//                totals of the workgroups before its own, copies the records
+//                totals of the workgroups before its own (where they are many,
+//                k_ra_scan has), copies the records
 //                into the output tables, empties them and their cells; the
 //                first wavefront closes the call: counts, epoch
 // Nothing waits on another thread: every probe makes progress by itself.
@@ -70,6 +71,12 @@ constexpr uint32_t kRaOwner = 0x80000000u;
 constexpr int kRaBlock = 256;       // workgroup of the three kernels
 constexpr int kRaBurst = 1024;      // most arrivals that one workgroup takes in one launch
 constexpr int kRaSmallBurst = 256;  // most that a smaller one takes
+constexpr int kRaScan = 1024;       // workgroup of k_ra_scan
+// Most workgroups whose totals every wavefront of k_ra_emit that hands something over adds up by itself
+// (which grows with the square of the burst); those of more are scanned by a launch in between.  A call,
+// us, added up / scanned:  220672 arrivals  17.8 / 20.5   524288  118.7 / 119.1   1000000  657 / 640
+//                          1024000 of 512 each  46.3 / 43.1      4000000  1200 / 1215
+constexpr uint32_t kRaSumBlocks = 3072;
 // device words of the reassembly state
 enum { kRaEpoch = 0, kRaInFlight, kRaEvicted, kRaWords = 16 };
 
@@ -617,8 +624,43 @@ __device__ __forceinline__ void ra_sum_blocks(const unsigned long long *p, uint3
   *before = wave_sum_pairs(b);
 }
 
-// B: the workgroup size of this kernel and of the two before it (a total per workgroup).
-template <int B>
+// The totals of more workgroups than that are scanned once, by one workgroup of T threads: in place,
+// with the sums of all behind them.  (B: as for k_ra_emit.)
+template <int T, int B>
+__global__ __launch_bounds__(T) void k_ra_scan(RaArgs a)
+{
+  __shared__ uint64_t wave_tot[T / kWave];
+  constexpr uint32_t kEach = 4;
+  const uint32_t n_blocks = (ra_n(a) + B - 1) / B;
+  uint64_t run = 0, fresh = 0;
+  for (uint32_t b0 = 0; b0 < n_blocks; b0 += kEach * T) {
+    const uint32_t b = b0 + kEach * threadIdx.x;
+    uint64_t v[kEach], mine = 0, tot;
+#pragma unroll
+    for (uint32_t k = 0; k < kEach; k++) {
+      v[k] = b + k < n_blocks ? a.blk[b + k] : 0ull;
+      fresh += b + k < n_blocks ? a.blk_new[b + k] : 0ull;
+      mine += v[k];
+    }
+    uint64_t at = run + block_exclusive_scan<T>(mine, wave_tot, &tot);
+#pragma unroll
+    for (uint32_t k = 0; k < kEach; k++) {
+      if (b + k < n_blocks) a.blk[b + k] = at;
+      at += v[k];
+    }
+    run += tot;
+  }
+  uint64_t all;
+  (void)block_exclusive_scan<T>(fresh, wave_tot, &all);
+  if (threadIdx.x == 0) {
+    a.blk[n_blocks] = run;
+    a.blk_new[n_blocks] = all;
+  }
+}
+
+// B: the workgroup size of this kernel and of the two before it (a total per workgroup).  SCANNED:
+// k_ra_scan has been over the totals.
+template <int B, bool SCANNED>
 __global__ __launch_bounds__(B) void k_ra_emit(RaArgs a)
 {
   const uint32_t n = ra_n(a);
@@ -635,15 +677,21 @@ __global__ __launch_bounds__(B) void k_ra_emit(RaArgs a)
   }
   if (!__any(done != 0) && !closer) return;
   // What completed in the workgroups before this one, and in all of them: every wavefront that
-  // has something to hand over adds the few hundred totals up by itself.
+  // has something to hand over adds the totals up by itself where they are few.
   const uint32_t n_blocks = (n + B - 1) / B;
   ra_emit(a, cell, done, lane, [&](uint64_t *base) {
     uint64_t tot;
-    ra_sum_blocks(a.blk, n_blocks, blockIdx.x, lane, &tot, base);
+    if (SCANNED) {
+      *base = sload(a.blk + blockIdx.x);
+      tot = sload(a.blk + n_blocks);
+    } else {
+      ra_sum_blocks(a.blk, n_blocks, blockIdx.x, lane, &tot, base);
+    }
     const bool overflow = (uint32_t)(tot >> 32) > a.max_req || (uint32_t)tot > a.max_frag;
     if (closer) {
       uint64_t fresh, none;
-      ra_sum_blocks(a.blk_new, n_blocks, 0, lane, &fresh, &none);
+      if (SCANNED) fresh = sload(a.blk_new + n_blocks);
+      else ra_sum_blocks(a.blk_new, n_blocks, 0, lane, &fresh, &none);
       if (lane == 0) ra_close(a, tot, fresh, overflow);
     }
     return !overflow;

@@ -137,6 +137,12 @@ def test_a_table_of_a_cell_per_request(share):
         assert call(2 * few[lo:hi])[:2] == (0, 0)
     assert call(2 * few[::-1] + 1) == (600, 1200, 0)
     assert np.array_equal(st.fs[:1200].cpu().numpy().reshape(-1, 2), 2 * few[::-1, None] + np.arange(2))
+    # launches sized for all of the arrivals, with fewer of them there
+    arr = to_dev((2 * early).astype(np.uint32), DEV)
+    for k in (0, 700, n - 5):
+        dev = torch.tensor([k], dtype=torch.int32, device=DEV)
+        assert ctx.reassemble(st.rx, arr, n, st.fs, st.fl, st.rf, st.tok, n_arrivals_dev=dev) == (0, 0, k)
+        assert int(st.rf[0]) == 0 and ctx.reassemble_evict(0) == k
     ctx.close()
 
 
