@@ -290,6 +290,22 @@ bool self_advancing(const Scratch &sc, bool packed, const void *slot_state, uint
 //                      32000              28.5 -> 37.4     32000 / 32000          23.2 -> 26.2
 constexpr uint32_t kSelfScanReqs = 16384, kSelfScanItems = 16384;
 
+template <bool SELF>
+void launch_prep_as(hipStream_t st, const PrepArgs &p, uint32_t avg)
+{
+  if (avg <= 8) {
+    k_prep_group<16, SELF><<<(p.n_req + 4 * kWavesPerBlock - 1) / (4 * kWavesPerBlock), kBlock, 0, st>>>(p);
+  } else if (avg <= 16) {
+    k_prep_group<32, SELF><<<(p.n_req + 2 * kWavesPerBlock - 1) / (2 * kWavesPerBlock), kBlock, 0, st>>>(p);
+  } else if (avg <= 32) {
+    k_prep_wave<SELF><<<(p.n_req + kWavesPerBlock - 1) / kWavesPerBlock, kBlock, 0, st>>>(p);
+  } else if (avg <= 256) {
+    k_prep_block<256, SELF><<<p.n_req, 256, 0, st>>>(p);
+  } else {
+    k_prep_block<1024, SELF><<<p.n_req, 1024, 0, st>>>(p);
+  }
+}
+
 // Descriptor build: kernel shape by the average request, then the bump-ring
 // scan of the request totals where offsets are not plain multiples.
 int launch_prep(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const PrepArgs &args)
@@ -303,21 +319,12 @@ int launch_prep(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const PrepArgs
   const uint32_t per_part = avg <= 8 ? 4 * kWavesPerBlock : avg <= 16 ? 2 * kWavesPerBlock : 0;
   // Few requests (a response's size stands in a table) or few fragments (so does its length): the
   // descriptor kernel's workgroups add up what lies before them and no scan is launched.
-  p.self_scan = p.packed && !p.fixed_offsets && !p.counts &&
-                (p.mode == 1 ? p.sizes && p.n_req <= kSelfScanReqs : p.item_len && p.n_items <= kSelfScanItems);
-  if (tiled && per_part && !p.self_scan) p.part = sc.tile_tot;
-  if (avg <= 8) {
-    k_prep_group<16><<<(p.n_req + 4 * kWavesPerBlock - 1) / (4 * kWavesPerBlock), kBlock, 0, st>>>(p);
-  } else if (avg <= 16) {
-    k_prep_group<32><<<(p.n_req + 2 * kWavesPerBlock - 1) / (2 * kWavesPerBlock), kBlock, 0, st>>>(p);
-  } else if (avg <= 32) {
-    k_prep_wave<<<(p.n_req + kWavesPerBlock - 1) / kWavesPerBlock, kBlock, 0, st>>>(p);
-  } else if (avg <= 256) {
-    k_prep_block<256><<<p.n_req, 256, 0, st>>>(p);
-  } else {
-    k_prep_block<1024><<<p.n_req, 1024, 0, st>>>(p);
-  }
-  if (p.packed && !p.fixed_offsets && !p.self_scan) {
+  const bool self_scan = p.packed && !p.fixed_offsets && !p.counts &&
+                         (p.mode == 1 ? p.sizes && p.n_req <= kSelfScanReqs : p.item_len && p.n_items <= kSelfScanItems);
+  if (tiled && per_part && !self_scan) p.part = sc.tile_tot;
+  if (self_scan) launch_prep_as<true>(st, p, avg);
+  else launch_prep_as<false>(st, p, avg);
+  if (p.packed && !p.fixed_offsets && !self_scan) {
     if (p.n_req <= 2 * kScanTile || p.counts) {  // counts on the device: one workgroup walks whatever is there
       k_req_scan<<<1, kScanBlock, 0, st>>>(p);
     } else {

@@ -81,9 +81,6 @@ struct PrepArgs {
   // k_prep_group: where every workgroup leaves the sum of its requests' totals (for the tiled
   // scan of many requests, which then needs no launch of its own to total the tiles); or nullptr
   uint64_t *part;
-  // The sizes of the requests before a workgroup's own are few and stand in a table (response sizes,
-  // or lengths): every workgroup adds them up and writes its requests' offsets itself, no scan follows.
-  uint32_t self_scan;
   // What this pass leaves for a later call that wants to reuse its descriptors
   // (SG_F_REUSE_DESC): desc_tag = {gen, requests, items, slot size the lengths were held
   // against, arena base, arena capacity} (kTag*, eight 32-bit words).
@@ -149,9 +146,46 @@ __device__ __forceinline__ uint64_t block_exclusive_scan(uint64_t v, uint64_t *l
   return base + inc - v;
 }
 
-// Length and slot of item f of request r, which is its item i: raises status bits for what it
-// refuses.  In two steps, so that a caller with several items per lane has all of one step's loads
-// in flight together: what the tables say of item f ...
+// Length and slot of item i of a request, `s` what the slot table says: raises status bits for what it
+// refuses.  Where its length and its header's source come from is the caller's: read where they are
+// needed, or before.
+template <class Len, class Hdr>
+__device__ __forceinline__ void prep_item(const PrepArgs &a, uint32_t s, uint32_t i, uint64_t size, Len asked_len, Hdr asked_hdr,
+                                          uint32_t *slot, uint32_t *len, uint32_t *bad)
+{
+  uint32_t l = 0;
+  if (s >= a.n_slots) {
+    *bad |= kStBadSlot;
+    s = 0;
+  } else if (a.mode == 0) {
+    l = asked_len();
+    if (l > a.slot_size - a.hl) {
+      *bad |= kStBadLen;
+      l = 0;
+    }
+  } else {
+    // frame i carries min(remaining, mtu) (src/transport/dpdk_rx_tx.h:137-139)
+    const uint64_t taken = (uint64_t)i * a.mtu;
+    const uint64_t rem = taken < size ? size - taken : 0;
+    l = (uint32_t)(rem <= a.mtu ? rem : a.mtu);
+    if (a.hdr_src_slot && asked_hdr() >= a.rx_n_slots) *bad |= kStBadSlot;
+  }
+  *slot = s;
+  *len = l;
+}
+
+// Item f, read as it comes (one item per thread and pass).
+__device__ __forceinline__ void prep_item_at(const PrepArgs &a, uint32_t f, uint32_t i, uint64_t size, uint32_t *slot,
+                                             uint32_t *len, uint32_t *bad)
+{
+  const uint32_t s = a.item_slot[f];
+  prep_item(
+      a, s, i, size, [&] { return a.item_len ? a.item_len[f] : load32_any(a.ring + (size_t)s * a.slot_size + 54); },
+      [&] { return a.hdr_src_slot[f]; }, slot, len, bad);
+}
+
+// The same in two steps, so that a caller with several items per lane has all of one step's loads in
+// flight together: what the tables say of item f ...
 struct PrepItem {
   uint32_t slot, len, hdr;
 };
@@ -169,29 +203,6 @@ __device__ __forceinline__ PrepItem prep_ask(const PrepArgs &a, uint32_t f, bool
 __device__ __forceinline__ void prep_look(const PrepArgs &a, PrepItem &t, bool on)
 {
   if (on && a.mode == 0 && !a.item_len && t.slot < a.n_slots) t.len = load32_any(a.ring + (size_t)t.slot * a.slot_size + 54);
-}
-__device__ __forceinline__ void prep_item(const PrepArgs &a, const PrepItem &t, uint32_t i, uint64_t size, uint32_t *slot,
-                                          uint32_t *len, uint32_t *bad)
-{
-  uint32_t s = t.slot, l = 0;
-  if (s >= a.n_slots) {
-    *bad |= kStBadSlot;
-    s = 0;
-  } else if (a.mode == 0) {
-    l = t.len;
-    if (l > a.slot_size - a.hl) {
-      *bad |= kStBadLen;
-      l = 0;
-    }
-  } else {
-    // frame i carries min(remaining, mtu) (src/transport/dpdk_rx_tx.h:137-139)
-    const uint64_t taken = (uint64_t)i * a.mtu;
-    const uint64_t rem = taken < size ? size - taken : 0;
-    l = (uint32_t)(rem <= a.mtu ? rem : a.mtu);
-    if (a.hdr_src_slot && t.hdr >= a.rx_n_slots) *bad |= kStBadSlot;
-  }
-  *slot = s;
-  *len = l;
 }
 
 // Checks on one request's slice of the CSR table and on its total; returns the
@@ -257,7 +268,7 @@ __device__ __forceinline__ void prep_finish(const PrepArgs &a, uint32_t r, uint6
 }
 
 // Bytes of the requests before request r0, whose first item is f0, added up by a workgroup of
-// BLOCK threads out of the table the sizes come from (self_scan).  A size or length that is refused
+// BLOCK threads out of the table the sizes come from (SELF).  A size or length that is refused
 // counts as it stands: the batch then moves nothing.
 template <int BLOCK>
 __device__ __forceinline__ uint64_t prep_before(const PrepArgs &a, uint32_t r0, uint32_t f0, uint64_t *lds_wave_tot)
@@ -308,7 +319,7 @@ __device__ __forceinline__ uint64_t ring_at(const PrepArgs &a, uint64_t c0, uint
   return o >= a.cap ? o - a.cap : o;
 }
 
-// Offset of request r, `before` bytes behind the batch's first, by the thread that owns it (self_scan).
+// Offset of request r, `before` bytes behind the batch's first, by the thread that owns it (SELF).
 __device__ __forceinline__ void prep_offset(const PrepArgs &a, uint32_t r, uint64_t before, uint64_t total)
 {
   uint64_t c0 = *a.cursor;
@@ -324,9 +335,15 @@ __device__ __forceinline__ void prep_offset(const PrepArgs &a, uint32_t r, uint6
   }
 }
 
+// The k_prep_* kernels.  SELF: the sizes of the requests before a workgroup's own are few and stand in
+// a table (response sizes, or lengths); every workgroup adds them up and writes its requests' offsets
+// itself, and no scan follows.  (Instances of their own: chosen at run time it cost the others
+// registers -- the descriptor pass of 17000 responses of 300 frames 262 us instead of 219, of 20000 of
+// 20 frames 25.7 instead of 24.5.)
+
 // One workgroup of BLOCK threads per request: block-wide exclusive scan of the
 // fragment lengths, all header reads of a pass in flight together.
-template <int BLOCK>
+template <int BLOCK, bool SELF>
 __global__ __launch_bounds__(BLOCK) void k_prep_block(PrepArgs a)
 {
   __shared__ uint64_t wave_tot[BLOCK / kWave];
@@ -340,9 +357,7 @@ __global__ __launch_bounds__(BLOCK) void k_prep_block(PrepArgs a)
   for (uint32_t base = f0; base < f1; base += BLOCK) {
     const uint32_t f = base + threadIdx.x;
     uint32_t len = 0, slot = 0;
-    PrepItem t = prep_ask(a, f, f < f1);
-    prep_look(a, t, f < f1);
-    if (f < f1) prep_item(a, t, f - f0, size, &slot, &len, &bad);
+    if (f < f1) prep_item_at(a, f, f - f0, size, &slot, &len, &bad);
     uint64_t tot;
     const uint64_t ex = block_exclusive_scan<BLOCK>(len, wave_tot, &tot);
     if (f < f1) {
@@ -355,13 +370,14 @@ __global__ __launch_bounds__(BLOCK) void k_prep_block(PrepArgs a)
   bad = wave_or(bad);
   if ((threadIdx.x & (kWave - 1)) == 0 && bad) refuse(a.status, a.status_flag, bad);
   if (threadIdx.x == 0) prep_finish(a, r, carry, 0);
-  if (a.self_scan) {
+  if (SELF) {
     const uint64_t before = prep_before<BLOCK>(a, r, f0, wave_tot);
     if (threadIdx.x == 0) prep_offset(a, r, before, carry);
   }
 }
 
 // One wavefront per request (requests of at most a few dozen fragments).
+template <bool SELF>
 __global__ __launch_bounds__(kBlock) void k_prep_wave(PrepArgs a)
 {
   __shared__ uint64_t wave_tot[kWavesPerBlock], req_tot[kWavesPerBlock];
@@ -369,7 +385,7 @@ __global__ __launch_bounds__(kBlock) void k_prep_wave(PrepArgs a)
   const uint32_t r0 = blockIdx.x * kWavesPerBlock, wv = threadIdx.x / kWave;
   const uint32_t r = r0 + wv;
   const bool live = r < a.n_req;
-  if (r0 >= a.n_req || (!live && !a.self_scan)) return;  // (with self_scan the whole workgroup has barriers to come to)
+  if (r0 >= a.n_req || (!live && !SELF)) return;  // (with SELF the whole workgroup has barriers to come to)
   const uint32_t lane = threadIdx.x & (kWave - 1);
   uint32_t f0 = 0, f1 = 0, bad = 0;
   uint64_t size = 0;
@@ -378,9 +394,7 @@ __global__ __launch_bounds__(kBlock) void k_prep_wave(PrepArgs a)
   for (uint32_t base = f0; base < f1; base += kWave) {
     const uint32_t f = base + lane;
     uint32_t len = 0, slot = 0;
-    PrepItem t = prep_ask(a, f, f < f1);
-    prep_look(a, t, f < f1);
-    if (f < f1) prep_item(a, t, f - f0, size, &slot, &len, &bad);
+    if (f < f1) prep_item_at(a, f, f - f0, size, &slot, &len, &bad);
     uint64_t tot;
     const uint64_t ex = block_exclusive_scan<kWave>(len, nullptr, &tot);
     if (f < f1) {
@@ -391,7 +405,7 @@ __global__ __launch_bounds__(kBlock) void k_prep_wave(PrepArgs a)
   }
   bad = wave_or(bad);
   if (live && lane == 0) prep_finish(a, r, carry, bad);
-  if (a.self_scan) {
+  if (SELF) {
     if (lane == 0) req_tot[wv] = carry;
     uint64_t before = prep_before<kBlock>(a, r0, a.first[r0], wave_tot);  // its barrier also stands behind req_tot
     if (live && lane == 0) {
@@ -408,7 +422,7 @@ __global__ __launch_bounds__(kBlock) void k_prep_wave(PrepArgs a)
 // keeps stepping while any of its groups has fragments left.
 // (Held to the scalar registers of eight wavefronts per SIMD instead of seven: 32768 requests 10.2 ->
 // 12.7 us, the arguments are then fetched again and again.)
-template <int L>
+template <int L, bool SELF>
 __global__ __launch_bounds__(kBlock) void k_prep_group(PrepArgs a)
 {
   constexpr uint32_t G = kWave / L;
@@ -436,7 +450,7 @@ __global__ __launch_bounds__(kBlock) void k_prep_group(PrepArgs a)
       const uint32_t f = base0 + k * L + gl;
       if (!__any(base0 + k * L < f1)) break;
       uint32_t len = 0, slot = 0;
-      if (f < f1) prep_item(a, t[k], f - f0, size, &slot, &len, &bad);
+      if (f < f1) prep_item(a, t[k].slot, f - f0, size, [&] { return t[k].len; }, [&] { return t[k].hdr; }, &slot, &len, &bad);
       // inclusive scan over the group's lanes
       uint32_t inc = len;
 #pragma unroll
@@ -454,7 +468,7 @@ __global__ __launch_bounds__(kBlock) void k_prep_group(PrepArgs a)
 #pragma unroll
   for (int m = L / 2; m >= 1; m >>= 1) bad |= __shfl_xor(bad, m, L);
   if (live && gl == 0) prep_finish(a, r, carry, bad);
-  if (a.self_scan) {
+  if (SELF) {
     const uint32_t r0 = blockIdx.x * kWavesPerBlock * G, mine = threadIdx.x / L;
     if (gl == 0) group_tot[mine] = carry;
     uint64_t before = prep_before<kBlock>(a, r0, a.first[r0], wave_tot);  // its barrier also stands behind group_tot
