@@ -279,16 +279,22 @@ bool self_advancing(const Scratch &sc, bool packed, const void *slot_state, uint
 }
 
 
-// Most requests (sizes in a table) and most fragments (lengths in a table) of which every workgroup
-// of the descriptor pass adds up those before its own, instead of a scan behind it.  Whole call,
-// scan -> this, us:     requests          scatter          requests / fragments   gather
-//                       1000              12.7 ->  9.0     1000 / 1000            11.2 ->  8.8
-//                       4000              13.7 -> 10.7     4000 / 7601            14.6 -> 11.6
-//                       8000              18.9 -> 12.2     2500 / 13722           18.2 -> 16.6
-//                      16000              20.0 -> 18.9     16000 / 16000          17.3 -> 14.8
-//                      24000              24.2 -> 27.2     24000 / 24000          20.0 -> 19.5
-//                      32000              28.5 -> 37.4     32000 / 32000          23.2 -> 26.2
-constexpr uint32_t kSelfScanReqs = 16384, kSelfScanItems = 16384;
+// Most requests of which every workgroup of the descriptor pass adds up the sizes before its own,
+// instead of a scan behind it, where the sizes stand in a table of their own (responses).  By the
+// average number of frames, which decides how many requests a workgroup has (16, 8, 4, 1), and with it
+// how often the table is read.  Whole call, us, scan -> this, on either side of the line:
+//   frames   1   8000  19.0 ->  12.4   12000  15.6 ->  15.4   16000  17.6 ->  18.9
+//           12   8000  53.0 ->  46.9   12000  67.3 ->  68.7   16000  87.2 ->  91.0
+//           32   8000 115.9 -> 110.8   12000 165.4 -> 163.9   16000 214.9 -> 218.7
+//           70   4000 123.9 -> 122.7    6000 182.9 -> 181.6    8000 239.0 -> 241.7
+//          300    500  71.2 ->  70.1    1000 134.0 -> 135.4    2000 257.7 -> 264.4
+uint32_t self_scan_reqs(uint32_t avg) { return avg <= 8 ? 12288 : avg <= 16 ? 10240 : avg <= 32 ? 12288 : avg <= 256 ? 6144 : 640; }
+// Most fragments, where the lengths do (requests): what a workgroup reads then grows with the fragments
+// before its own whatever their number per request.
+//   requests of 1   8000  17.0 -> 10.1   16000  14.4 -> 14.5   20000  16.0 -> 17.0
+//              12    500  11.2 ->  9.1    1360  14.3 -> 13.8    2000  16.5 -> 17.2
+//              70    200  13.4 -> 12.0     230  14.1 -> 13.0     400  17.5 -> 18.3
+constexpr uint32_t kSelfScanItems = 16384;
 
 template <bool SELF>
 void launch_prep_as(hipStream_t st, const PrepArgs &p, uint32_t avg)
@@ -320,7 +326,7 @@ int launch_prep(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const PrepArgs
   // Few requests (a response's size stands in a table) or few fragments (so does its length): the
   // descriptor kernel's workgroups add up what lies before them and no scan is launched.
   const bool self_scan = p.packed && !p.fixed_offsets && !p.counts &&
-                         (p.mode == 1 ? p.sizes && p.n_req <= kSelfScanReqs : p.item_len && p.n_items <= kSelfScanItems);
+                         (p.mode == 1 ? p.sizes && p.n_req <= self_scan_reqs(avg) : p.item_len && p.n_items <= kSelfScanItems);
   if (tiled && per_part && !self_scan) p.part = sc.tile_tot;
   if (self_scan) launch_prep_as<true>(st, p, avg);
   else launch_prep_as<false>(st, p, avg);

@@ -26,7 +26,7 @@ def _sizes(n, frags, seed):
 
 
 # (requests, fragments of each on average): 16, 32 and 64 lanes per request, workgroups of 256 and 1024; one request;
-# 16384 and one more of requests (scatter) and of fragments (gather)
+# 16384 fragments (gather) and one more
 SHAPES = [(1, 3), (15, 2), (17, 2), (130, 6), (61, 12), (9, 24), (5, 60), (7, 400), (16384, 1), (16385, 1), (700, 23), (1000, 17)]
 
 
@@ -61,4 +61,31 @@ def test_offsets_of_a_batch_with_tables(n_req, frags):
         assert np.array_equal(got, exp_tx), first_diff(got, exp_tx)
         assert np.array_equal(dw.resp_offsets.cpu().numpy().view(np.uint64), toffs)
         assert ctx.get_cursor(1) == tcur
+    ctx.close()
+
+
+# frames of each response, and how many of those are still added up (the descriptor kernels of 16, 32 and 64 lanes per
+# request, workgroups of 256 and of 1024 threads)
+LINES = [(1, 12288), (8, 12288), (9, 10240), (16, 10240), (17, 12288), (32, 12288), (33, 6144), (40, 6144), (257, 640)]
+
+
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("frames,line", LINES)
+def test_responses_on_both_sides_of_the_line(frames, line, over):
+    n = line + over
+    resp = np.full(n, 16 * frames - 3)
+    resp[::2] -= 5
+    w = synth.make_custom(np.full(n, 8), resp, mtu=16, slot_size=96, seed=frames)
+    print(f"case offsets frames={frames} n={n}", flush=True)
+    ctx = SgContext(0, max_reqs=n, max_frames=w.n_resp_frames)
+    dw = DeviceWorkload(w, arena_slack=1001)
+    rcap = dw.resp_app.cap
+    tcur = rcap - 5
+    ctx.set_cursor(1, tcur)
+    dw.scatter(ctx, fixed=False)
+    exp_tx, toffs, tcur = expected_scatter(w, None, resp_cap=rcap, cursor=tcur)
+    got = dw.tx_ring.cpu().numpy()
+    assert np.array_equal(got, exp_tx), first_diff(got, exp_tx)
+    assert np.array_equal(dw.resp_offsets.cpu().numpy().view(np.uint64), toffs)
+    assert ctx.get_cursor(1) == tcur
     ctx.close()
