@@ -407,7 +407,10 @@ int sg_hip_scatter_batch(sg_hip_ctx *ctx, const sg_scatter_args *args);
  * full UDP checksum excepted): on one stream the second of two launches waits
  * until the first has drained the chip.  Any other pair of calls is made as two
  * calls, gather first.  Synchronous unless both argument blocks carry
- * SG_F_ASYNC. */
+ * SG_F_ASYNC.  What the host refuses in either half launches neither.  What the
+ * device refuses in the gather (SG_E_DATA) leaves the scatter undone only where
+ * the pair is made as two synchronous calls: in a shared launch both halves
+ * have run, the refused fragments alone are skipped, both cursors are advanced. */
 int sg_hip_shunt_batch(sg_hip_ctx *ctx, const sg_gather_args *gather, const sg_scatter_args *scatter);
 
 /* Fragment tables the device reads where the receive thread writes them.

@@ -231,6 +231,39 @@ def test_refusals_come_through_either_half():
     ctx.close()
 
 
+@pytest.mark.parametrize("n_req", [6, 3000], ids=["small", "large"])
+@pytest.mark.parametrize("shared", [True, False], ids=["one-launch", "two-calls"])
+def test_what_a_refused_gather_leaves_of_the_scatter(shared, n_req):
+    """In a shared launch of any size the scatter has run and both cursors are on; a pair made as two synchronous calls
+    ends with the gather."""
+    from splitrpc_amd.engine import to_dev
+    w = synth.make_custom([4200] * n_req, [3000] * n_req, seed=80)
+    ctx = SgContext(0)
+    dw = DeviceWorkload(w, arena_slack=64)
+    # (one offsets table for both halves keeps them apart)
+    ga, sa = _args(ctx, dw, w, None, 0, dw.req_offsets, dw.resp_offsets if shared else dw.req_offsets)
+    rcap = sa.app.arena_cap = dw.resp_app.cap - 100  # the responses do not fill it evenly
+    bad = w.frag_slot.copy()
+    bad[4] = w.n_slots + 3
+    bad_dev = to_dev(bad, DEV)
+    ga.frag_slot = bad_dev.data_ptr()
+    ctx.set_cursor(0, 0)
+    ctx.set_cursor(1, 0)
+    torch.cuda.synchronize()
+    with pytest.raises(Exception) as e:
+        ctx.shunt_batch_raw(ga, sa)
+    assert e.value.code == capi.SG_E_DATA
+    exp, _, ecur = expected_gather(w, arena_cap=dw.req_app.cap)
+    exp = exp.copy()
+    exp[4 * 1400:5 * 1400] = 0  # the fragment that is not there (4200 = 3 * 1400)
+    assert np.array_equal(dw.req_arena.cpu().numpy(), exp) and ctx.get_cursor(0) == ecur
+    exp_tx, _, tcur = expected_scatter(w, None, resp_cap=rcap)
+    assert ecur and tcur
+    assert np.array_equal(dw.tx_ring.cpu().numpy(), exp_tx if shared else w.tx_ring_init)
+    assert ctx.get_cursor(1) == (tcur if shared else 0)
+    ctx.close()
+
+
 def test_shunt_calls_recorded_into_a_graph_continue_both_rings():
     """Three calls of one launch each in one graph; every replay continues both
     bump rings where the last one stopped, with eager work in between."""
