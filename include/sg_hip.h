@@ -404,7 +404,7 @@ int sg_hip_scatter_batch(sg_hip_ctx *ctx, const sg_scatter_args *args);
  * keeps a slot ring, and neither touches the other's memory (the TX ring apart
  * from the RX ring, the response buffers apart from the request buffers), both
  * travel in ONE launch, of any size (an mtu of more than 14111 bytes with the
- * full UDP checksum excepted): on one stream the second of two launches waits
+ * full UDP checksum, and more wavefronts than a launch takes, 2^26, excepted): on one stream the second of two launches waits
  * until the first has drained the chip.  Any other pair of calls is made as two
  * calls, gather first.  Synchronous unless both argument blocks carry
  * SG_F_ASYNC.  What the host refuses in either half launches neither.  What the

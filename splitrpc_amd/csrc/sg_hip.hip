@@ -1452,7 +1452,8 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
   if (rg < 0) return rg;
   const int rs = scatter_impl(c, c->sc, c->stream, s, &h);
   if (rs < 0) return rs;
-  if (rg == SG_OK && rs == SG_OK && halves_apart(g, s)) {
+  constexpr uint64_t kMostGroups = 0xffffffffu / kBlock;  // a launch's threads are counted in 32 bits
+  if (rg == SG_OK && rs == SG_OK && (uint64_t)h.s_small_grid + h.s_grid + h.g_grid <= kMostGroups && halves_apart(g, s)) {
     ShuntArgs &sh = h.sh;
     // the kernel advances the cursors itself where each half's own would; a workgroup for either
     // direction behind it does otherwise

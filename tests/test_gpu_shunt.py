@@ -264,6 +264,40 @@ def test_what_a_refused_gather_leaves_of_the_scatter(shared, n_req):
     ctx.close()
 
 
+@pytest.mark.parametrize("n_req", [500, 1150000], ids=["one-launch", "two-launches"])
+def test_more_wavefronts_than_a_launch_takes(n_req):
+    """Either half within what a launch takes (30 wavefronts per fragment by its mtu), both together not: two launches.
+    Every request comes from one slot, every response goes to one."""
+    mtu, slot, size = 60000, 60064, 16
+    w = synth.make_custom([size], [size], mtu=mtu, slot_size=slot, seed=81)
+    print(f"case shunt many wavefronts n_req={n_req}", flush=True)
+    ctx = SgContext(0, max_reqs=n_req, max_frames=n_req)
+    dw = DeviceWorkload(w)
+    i32 = lambda t: t.to(torch.int32).to(DEV)
+    zero, one = i32(torch.zeros(n_req)), i32(torch.arange(n_req + 1))
+    frag, tx = zero + int(w.frag_slot[0]), zero + int(w.tx_slot[0])
+    cap = n_req * size + 100
+    arena = torch.zeros(cap, dtype=torch.uint8, device=DEV)
+    resp = dw.resp_arena[:size].repeat(n_req + 1)
+    flags = capi.F_NO_SMALL
+    ga = ctx.gather_args(dw.rx, frag, None, one, n_req, n_req, AppRef(arena=arena, cap=cap), None,
+                         flags=flags | capi.F_RULE_FRAGS, fixed_req_size=size, mtu=mtu)
+    sa = ctx.scatter_args(dw.rx, dw.tx, tx, zero + int(w.hdr_src_slot[0]), one, None, size, n_req, n_req, mtu,
+                          AppRef(arena=resp, cap=(n_req + 1) * size), None, w.flags | flags)
+    ctx.set_cursor(0, 0)
+    ctx.set_cursor(1, 0)
+    ctx.set_profiling(True)
+    torch.cuda.synchronize()
+    ctx.shunt_batch_raw(ga, sa)
+    assert bool((arena[:n_req * size].view(n_req, size) == torch.from_numpy(w.req_payload).to(DEV)).all())
+    assert not bool(arena[n_req * size:].any())
+    exp_tx, _, _ = expected_scatter(w, None, resp_cap=dw.resp_app.cap)
+    assert np.array_equal(dw.tx_ring.cpu().numpy(), exp_tx)
+    assert ctx.get_cursor(0) == n_req * size and ctx.get_cursor(1) == n_req * size
+    assert ctx.kernel_time(1)[1] == 1 and ctx.kernel_time(2)[1] == (0 if n_req < 1000 else 1)
+    ctx.close()
+
+
 def test_shunt_calls_recorded_into_a_graph_continue_both_rings():
     """Three calls of one launch each in one graph; every replay continues both
     bump rings where the last one stopped, with eager work in between."""
