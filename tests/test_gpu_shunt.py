@@ -4,7 +4,7 @@ gather followed by its scatter, bit for bit, through the C ABI: arenas, TX
 ring, offsets and both bump-ring cursors, over calls in a row and over graph
 replays.  Pairs of calls that cannot share a launch (sizes that differ, an
 echo answered in place) must come out the same through the two-call path the
-entry point then takes, and so must tensors and larger calls either way."""
+entry point then takes; the launches are counted."""
 import numpy as np
 import pytest
 import torch
@@ -83,48 +83,64 @@ def test_one_launch_moves_what_two_calls_move(name, profile):
     ctx.close()
 
 
-APART = {
-    # (workload, what it is about)
-    "jumbo": lambda: synth.make_workload(5, 1),                     # frames of several wavefronts
-    "short-frames-16-lanes": lambda: synth.make_custom([300] * 50, [300] * 50, seed=78),  # short frames, 16 lanes each
-    "bert": lambda: synth.make_workload(3, 20),                     # tensors; short last fragments
-    "mixed-echo": lambda: synth.make_workload(4, 50),               # variable sizes, answered in place
-    "sizes-differ": lambda: synth.make_custom([4200] * 12, [100 + 333 * k for k in range(12)], seed=74),
+# (workload, whether its two calls share a launch; if not, how many descriptor passes they make)
+PAIRS = {
+    "jumbo": (lambda: synth.make_workload(5, 1), True),                     # frames of several wavefronts
+    "short-frames-16-lanes": (lambda: synth.make_custom([300] * 50, [300] * 50, seed=78), True),
+    "bert": (lambda: synth.make_workload(3, 20), True),                     # tensors; short last fragments
+    "tensors-in": (lambda: synth.make_custom([4200] * 40, [3000] * 40, seed=82, in_tensor_sizes=[1500, 2700]), True),
+    "tensors-out": (lambda: synth.make_custom([4200] * 40, [3000] * 40, seed=83, out_tensor_sizes=[2000, 1000]), True),
     # more wavefronts than the chip holds at once
-    "lenet-4096": lambda: synth.make_workload(1, 4096),
-    "two-frames-3000": lambda: synth.make_custom([4200] * 3000, [2800] * 3000, seed=77, flags=synth.F_UDP_CSUM_PSEUDO),
+    "lenet-4096": (lambda: synth.make_workload(1, 4096), True),
+    "two-frames-3000": (lambda: synth.make_custom([4200] * 3000, [2800] * 3000, seed=77, flags=synth.F_UDP_CSUM_PSEUDO), True),
+    # more than advance their cursor themselves: both halves, the gather's alone, the scatter's alone
+    "wavefronts-70000": (lambda: synth.make_custom([1000] * 70000, [1000] * 70000, slot_size=1536, seed=84), True),
+    "gather-of-75000": (lambda: synth.make_custom([4200] * 25000, [40] * 25000, slot_size=1536, seed=85), True),
+    "scatter-of-75000": (lambda: synth.make_custom([40] * 25000, [4200] * 25000, slot_size=1536, seed=86), True),
+    "mixed-echo": (lambda: synth.make_workload(4, 50), 2),                  # variable sizes, answered in place
+    "sizes-differ": (lambda: synth.make_custom([4200] * 12, [100 + 333 * k for k in range(12)], seed=74), 1),
 }
 
 
-@pytest.mark.parametrize("name", list(APART))
-def test_pairs_that_cannot_share_a_launch_take_two(name):
-    w = APART[name]()
-    print(f"case shunt apart {name} n_req={w.n_req} frags={w.n_frags} frames={w.n_resp_frames}", flush=True)
-    ctx = SgContext(0, max_reqs=8192, max_frames=1 << 17)
-    dw = DeviceWorkload(w)
+@pytest.mark.parametrize("name", list(PAIRS))
+def test_pairs_come_out_the_same_in_one_launch_or_two(name):
+    w, shares = PAIRS[name][0](), PAIRS[name][1]
+    print(f"case shunt pair {name} n_req={w.n_req} frags={w.n_frags} frames={w.n_resp_frames}", flush=True)
+    ctx = SgContext(0, max_reqs=1 << 17, max_frames=1 << 17)
+    dw = DeviceWorkload(w, arena_slack=0 if w.tx_in_place else 72)
     one_size = bool((w.req_sizes == w.req_sizes[0]).all())
     ga, sa = _args(ctx, dw, w, None, 0, dw.req_offsets, dw.resp_offsets, rule=one_size)
+    rcap = 0 if w.out_tensor_sizes else dw.resp_app.cap
+    if rcap and w.n_req > 1 and not w.tx_in_place:
+        rcap = sa.app.arena_cap = rcap - 8  # a pass does not end where it began
     ctx.set_cursor(0, 0)
     ctx.set_cursor(1, 0)
+    ctx.set_profiling(True)
     ctx.shunt_batch_raw(ga, sa)
+    if shares is True:
+        assert [ctx.kernel_time(k)[1] for k in range(3)] == [0, 1, 0]
+    else:
+        assert [ctx.kernel_time(k)[1] for k in range(3)] == [shares, 1, 1]
     if w.in_tensor_sizes:
         exp, _, _ = expected_gather(w)
         for t, e in zip(dw.in_tensors, exp):
             assert np.array_equal(t.cpu().numpy(), e)
-        gathered = None
+        gathered, ecur = None, 0
     else:
         exp, eoffs, ecur = expected_gather(w, arena_cap=dw.req_app.cap)
         got = dw.req_arena.cpu().numpy()
         assert np.array_equal(got, exp), first_diff(got, exp)
         assert np.array_equal(dw.req_offsets.cpu().numpy().view(np.uint64), eoffs)
-        assert ctx.get_cursor(0) == ecur
         gathered = exp
-    exp_tx, toffs, tcur = expected_scatter(w, gathered, resp_cap=dw.resp_app.cap if not w.out_tensor_sizes else None)
+    assert ctx.get_cursor(0) == ecur
+    exp_tx, toffs, tcur = expected_scatter(w, gathered, resp_cap=rcap or None)
     got = dw.tx_ring.cpu().numpy()
     assert np.array_equal(got, exp_tx), first_diff(got, exp_tx)
-    if dw.resp_offsets is not None:
+    if w.out_tensor_sizes:
+        tcur = 0
+    else:
         assert np.array_equal(dw.resp_offsets.cpu().numpy().view(np.uint64), toffs)
-        assert ctx.get_cursor(1) == tcur
+    assert ctx.get_cursor(1) == tcur
     ctx.close()
 
 
