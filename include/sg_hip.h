@@ -96,9 +96,10 @@ extern "C" {
 #define SG_F_TAIL_KERNEL (1u << 21)    /* the opposite: always the kernel behind the call (for experiments) */
 #define SG_F_SMALL_GROUPS (1u << 22)   /* sg_hip_reassemble: the call is meant to run BESIDE a long copy
                                           kernel of another stream (another receive queue's gather, or
-                                          this queue's previous burst).  Its kernels come in workgroups of
-                                          256 threads, which find room on a chip that such a kernel keeps
-                                          full, with or without this flag: accepted, and without effect. */
+                                          this queue's previous burst).  Accepted, and without effect: its
+                                          kernels come in workgroups of 256 threads anyway, which find room on
+                                          a chip that such a kernel keeps full -- but for bursts of 257 to
+                                          1024 arrivals, which are one workgroup of 1024. */
 
 /* States of an application slot (APP_RR_STATUS, src/p2p_rpc_app_ctx.h:22). */
 #define SG_SLOT_FREE 0u
