@@ -270,7 +270,9 @@ const uint64_t *plain_cursor(const Scratch &sc, int which)
 // call on a stream each): 16 requests of 602112 bytes 13.0 -> 8.9 us, eight such batches in one
 // call 31.6 -> 30.7 us, 32 batches 105.9 -> 105.3 us; 8192 requests of 3136 bytes 18.1 -> 16.0 us,
 // 65536 of them 89.8 -> 90.4 us; 256 requests of 1.5 MB in 8800-byte fragments 233.5 -> 235.6 us.
-// A call that publishes slot states has the kernel behind it anyway.
+// A call that publishes slot states has the kernel behind it anyway.  (The line was drawn with a stream
+// per direction, which hides most of the kernel behind.  It has not been drawn again for a launch of
+// both directions on one stream, which does not.)
 constexpr uint64_t kSelfAdvanceMaxWaves = 65536;
 bool self_advancing(const Scratch &sc, bool packed, const void *slot_state, uint64_t waves, uint32_t flags)
 {
@@ -461,7 +463,8 @@ static uint32_t small_lanes(uint64_t bytes, bool eight = true)
 
 // Remainder fragments get wavefronts of their own kind when they are a good share of the
 // call's wavefronts -- and, where that takes a launch of its own (scatter), when the call is
-// large enough to hide one more launch.
+// large enough to hide one more launch.  (A scatter in a launch of both directions goes by the same
+// line, measured with a launch of its own.)
 static bool small_last_pays(uint64_t per_req, uint32_t n_req, uint32_t flags, bool own_launch)
 {
   if (per_req < 2) return false;
