@@ -227,7 +227,7 @@ __device__ __forceinline__ uint32_t fold16(uint32_t s)
 // by one, a GFX9-family cross-lane move that needs no LDS.
 __device__ __forceinline__ uint32_t wave_shl1(uint32_t v)
 {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, false);
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x130, 0xf, 0xf, true);
 }
 
 // Bytes [p, p+16) of the 32-byte window {lo, hi}, p = 4*Q + bs.
@@ -258,6 +258,52 @@ __device__ __forceinline__ u32x4 realign(u32x4 v, uint32_t p)
   }
 }
 
+// A wavefront's two chunks at once, the phase the same for all lanes.  Every case asks its
+// neighbours for the dwords it needs only, and the byte phase is made opaque in each: left to
+// itself the optimizer shares instructions between the cases and pays for it with copies and
+// branches in all of them.
+template <int Q>
+__device__ __forceinline__ void realign_at(u32x4 &v, uint32_t bs)
+{
+  uint32_t d[Q + 5];
+#pragma unroll
+  for (int j = 0; j < Q + 5; j++) d[j] = j < 4 ? v[j] : wave_shl1(v[j - 4]);
+#pragma unroll
+  for (int j = 0; j < 4; j++) v[j] = __builtin_amdgcn_alignbyte(d[Q + j + 1], d[Q + j], bs);
+}
+template <int Q>
+__device__ __forceinline__ void realign_pair_at(u32x4 &v0, u32x4 &v1, uint32_t p)
+{
+  asm("" : "+s"(p));
+  realign_at<Q>(v0, p & 3u);
+  realign_at<Q>(v1, p & 3u);
+}
+__device__ __forceinline__ void realign_pair(u32x4 &v0, u32x4 &v1, uint32_t p)
+{
+  p = (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
+  if (p < 8) {
+    if (p < 4) realign_pair_at<0>(v0, v1, p);
+    else realign_pair_at<1>(v0, v1, p);
+  } else {
+    if (p < 12) realign_pair_at<2>(v0, v1, p);
+    else realign_pair_at<3>(v0, v1, p);
+  }
+}
+
+// A piece of memory as the buffer instructions take it: accesses at or beyond `bytes` load zeros and
+// store nothing, so that a wavefront needs neither a comparison nor a branch for the lanes that have
+// nothing to do.  (Wave-uniform.  Every access below lies wholly on one side of the limit.)
+typedef __amdgpu_buffer_rsrc_t Piece;
+__device__ __forceinline__ Piece piece_of(const uint8_t *p, uint32_t bytes)
+{
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(p), 0, (int)bytes, 0x00020000);
+}
+constexpr int kNontemporal = 2;
+constexpr uint32_t kNowhere = 0x80000000u;  // an offset beyond every piece
+__device__ __forceinline__ u32x4 piece_load16(Piece p, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(p, (int)off, 0, kNontemporal); }
+__device__ __forceinline__ void piece_store16_kept(Piece p, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, p, (int)off, 0, 0); }
+__device__ __forceinline__ void piece_store16(Piece p, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, p, (int)off, 0, kNontemporal); }
+
 // One run (a contiguous piece of payload) in the hands of one wavefront.
 //
 // Stores are 16-byte aligned: the destination decides the phase.  Loads are
@@ -271,19 +317,33 @@ __device__ __forceinline__ u32x4 realign(u32x4 v, uint32_t p)
 // 16-byte-aligned hull is read.  The up-to-15 bytes before the first aligned
 // store and after the last one move as single bytes on lanes 0..15 / 16..31.
 //
-// run_begin issues the edge-byte load and the loads of the first two steps
-// (126 destination chunks, 2016 bytes); run_end realigns, stores and walks the
-// rest.  A wavefront that begins several runs before ending the first keeps
-// that many runs' loads in flight.
+// run_begin (0 < len <= kRunMost) issues the load of the edge bytes and those of the first
+// two steps (126 destination chunks, 2016 bytes); run_end realigns, stores and
+// walks the rest.  A wavefront that begins several runs before ending the first
+// keeps that many runs' loads in flight.  (The edge bytes are asked for first:
+// behind the hinted loads their line, which those do not keep, comes from memory
+// a second time, and the edge stores are late for the lines they complete.)
+//
+// What bounds it: memory, and half of a wavefront's life instructions (resnet-sized
+// fragments, per wavefront: 425 instructions, 414 of 1961 quad cycles issuing and
+// 513 waiting to issue).  Through buffer descriptors, which drop the lanes that
+// have nothing to do, and with one branch for both steps' realignment it is 75
+// instructions from begin to end where masks and branches took 150.  One pass, us:
+//   512 requests of 602112 bytes, 4000 back   104.5 -> 103.5
+//   256 of 1.5 MB in 8800-byte fragments, the UDP checksum of 1 MB responses in software   225 -> 220.5
+//   32768 of all sizes, echoed                251 -> 241
+//   8192 of 3136 bytes, 40 back               15.1 -> 14.4
+//   16 of 602112 bytes, 4000 back             7.15 -> 6.9
+constexpr uint32_t kStep = 63 * 16;  // bytes a step stores
+constexpr uint32_t kRunMost = 1u << 30;  // bytes of the longest run: offsets stay below kNowhere
 struct RunState {
-  const uint8_t *src;
+  Piece in;        // the run's hull
   uint8_t *dst;
-  const uint8_t *sa;  // source of the first aligned store, rounded down to 16
-  uint8_t *d;         // first aligned store
-  uint32_t body;      // number of aligned 16-byte stores
-  uint32_t lim;       // last source chunk to load (body when the phase is non-zero)
-  uint32_t p;         // source phase
-  uint32_t eoff;      // this lane's edge byte, if any
+  uint32_t at;     // offset in the hull of this lane's first chunk
+  uint32_t head;   // bytes before the first aligned store
+  uint32_t body;   // bytes of the aligned stores
+  uint32_t p;      // source phase
+  uint32_t eoff;   // this lane's edge byte, if any
   uint32_t eb;
   bool edge;
   u32x4 v0, v1;
@@ -294,33 +354,21 @@ __device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict
 {
   uint32_t head = (uint32_t)(-(uintptr_t)dst) & 15u;
   head = head < len ? head : len;
-  const uint32_t body = (len - head) >> 4;
-  const uint32_t tail = (len - head) & 15u;
-  r.src = src;
+  const uint32_t rest = len - head, tail = rest & 15u;
+  const uint32_t s0 = (uint32_t)(uintptr_t)src & 15u, q = s0 + head;
   r.dst = dst;
-  r.body = body;
-  r.edge = false;
-  r.eoff = 0;
-  if (lane < 16) {
-    r.edge = lane < head;
-    r.eoff = lane;
-  } else if (lane < 32) {
-    r.edge = (lane - 16) < tail;
-    r.eoff = head + (body << 4) + (lane - 16);
-  }
-  r.eb = 0;
-  if (r.edge) r.eb = src[r.eoff];
-  const uint8_t *s = src + head;
-  r.d = dst + head;
-  r.p = (uint32_t)(uintptr_t)s & 15u;
-  r.sa = s - r.p;
-  r.lim = r.p ? body : body - 1;  // body == 0: lim wraps, guarded below
-  r.v0 = (u32x4){0, 0, 0, 0};
-  r.v1 = (u32x4){0, 0, 0, 0};
-  if (body) {
-    if (lane <= r.lim) r.v0 = load16_aligned(r.sa + ((size_t)lane << 4));
-    if (63u + lane <= r.lim) r.v1 = load16_aligned(r.sa + ((size_t)(63u + lane) << 4));
-  }
+  r.head = head;
+  r.body = rest & ~15u;
+  r.p = q & 15u;
+  r.in = piece_of(src - s0, (s0 + len + 15u) & ~15u);
+  r.at = (lane << 4) + (q & 16u);
+  const bool second = lane >= 16;
+  const uint32_t k = second ? lane - 16 : lane;
+  r.edge = k < (second ? tail : head);
+  r.eoff = k + (second ? head + r.body : 0u);
+  r.eb = __builtin_amdgcn_raw_buffer_load_b8(r.in, (int)(s0 + r.eoff), 0, 0);
+  r.v0 = piece_load16(r.in, r.at);
+  r.v1 = piece_load16(r.in, r.at + kStep);
 }
 
 // With CSUM returns this lane's share of the sum of the 16-bit little-endian
@@ -328,40 +376,61 @@ __device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict
 // parity of its DESTINATION ADDRESS (packet offsets and addresses have the
 // same parity: ring bases, slot sizes and header lengths are even).
 //
+// KEEP_ENDS: what goes into the run's first and last 128-byte line of the destination is stored
+// without the nontemporal hint.  A neighbouring wavefront writes the rest of those lines, a little
+// earlier or later, and with the hint the second level cache writes a line out before it is whole:
+// memory then takes a part of a line twice (24.4 instead of 22.2 write requests per wavefront of
+// 1400 bytes).  For runs that lie end to end, requests in an arena; a frame in a slot of its own has
+// no such neighbour.  220672 fragments of 1400 bytes: 128 us without, 103.5 with; everything without
+// the hint: 136 us.
+//
 // BROKEN: the destination is two pieces -- aligned chunks from number `brk` on, and the tail
 // bytes, land `jump` bytes further (a fragment that runs from one tensor into the next, where
 // the second tensor's share starts on a 16-byte boundary and the first one's share ends on a
 // chunk boundary of the run): one run instead of two.
-template <bool CSUM, bool BROKEN = false>
+template <bool KEEP_ENDS, bool CSUM, bool BROKEN = false>
 __device__ __forceinline__ uint32_t run_end(RunState &r, uint32_t lane, uint32_t brk = 0, int64_t jump = 0)
 {
+  static_assert(!(KEEP_ENDS && BROKEN), "one or the other");
   uint32_t acc = 0;
-  const u32x4 o0 = realign(r.v0, r.p);
-  const u32x4 o1 = realign(r.v1, r.p);
-  auto at = [&](uint32_t c) { return r.d + ((size_t)c << 4) + ((BROKEN && c >= brk) ? jump : (int64_t)0); };
-  if (lane < 63 && lane < r.body) {
-    store16_aligned(at(lane), o0);
-    if (CSUM) acc += words_sum(o0);
-  }
-  if (lane < 63 && 63u + lane < r.body) {
-    store16_aligned(at(63u + lane), o1);
-    if (CSUM) acc += words_sum(o1);
-  }
-  for (uint32_t base = 126; base < r.body; base += 126) {
-    const uint32_t c0 = base + lane, c1 = base + 63u + lane;
-    u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-    if (c0 <= r.lim) v0 = load16_aligned(r.sa + ((size_t)c0 << 4));
-    if (c1 <= r.lim) v1 = load16_aligned(r.sa + ((size_t)c1 << 4));
-    const u32x4 q0 = realign(v0, r.p);
-    const u32x4 q1 = realign(v1, r.p);
-    if (lane < 63 && c0 < r.body) {
-      store16_aligned(at(c0), q0);
-      if (CSUM) acc += words_sum(q0);
+  const uint32_t first = BROKEN ? brk << 4 : r.body;  // bytes of the first destination piece
+  const Piece out = piece_of(r.dst + r.head, first);
+  const Piece out_b = BROKEN ? piece_of(r.dst + r.head + first + jump, r.body - first) : out;
+  const uint32_t at = lane < 63 ? lane << 4 : kNowhere;
+  // offsets of the stores that go into whole lines: from .. from + whole (none for a run inside one line)
+  const uint32_t d0 = (uint32_t)(uintptr_t)r.dst + r.head, over = (d0 + r.body) & 127u;
+  const uint32_t from = (0u - d0) & 127u, whole = from + over <= r.body ? r.body - over - from : 0u;
+  auto put = [&](uint32_t base) {
+    realign_pair(r.v0, r.v1, r.p);
+    const uint32_t a0 = base + at, a1 = a0 + kStep;
+    if (KEEP_ENDS) {
+      const bool w0 = a0 - from < whole, w1 = a1 - from < whole;
+      piece_store16(out, w0 ? a0 : kNowhere, r.v0);
+      piece_store16(out, w1 ? a1 : kNowhere, r.v1);
+      piece_store16_kept(out, w0 ? kNowhere : a0, r.v0);
+      piece_store16_kept(out, w1 ? kNowhere : a1, r.v1);
+    } else {
+      piece_store16(out, a0, r.v0);
+      piece_store16(out, a1, r.v1);
     }
-    if (lane < 63 && c1 < r.body) {
-      store16_aligned(at(c1), q1);
-      if (CSUM) acc += words_sum(q1);
+    if (BROKEN) {
+      // below the break these offsets wrap and lie beyond the second piece; opaque, so that no part
+      // of them is left to the instruction's own offset field, behind the wrap
+      uint32_t b0 = a0 - first, b1 = a1 - first;
+      asm("" : "+v"(b0), "+v"(b1));
+      piece_store16(out_b, b0, r.v0);
+      piece_store16(out_b, b1, r.v1);
     }
+    if (CSUM) {
+      acc += a0 < r.body ? words_sum(r.v0) : 0u;
+      acc += a1 < r.body ? words_sum(r.v1) : 0u;
+    }
+  };
+  put(0);
+  for (uint32_t base = 2 * kStep; __builtin_expect(base < r.body, 0); base += 2 * kStep) {
+    r.v0 = piece_load16(r.in, r.at + base);
+    r.v1 = piece_load16(r.in, r.at + base + kStep);
+    put(base);
   }
   if (r.edge) {
     // head bytes sit on lanes 0..15, tail bytes (behind the last aligned chunk) on lanes 16..31
@@ -372,14 +441,14 @@ __device__ __forceinline__ uint32_t run_end(RunState &r, uint32_t lane, uint32_t
   return acc;
 }
 
-// Copy `len` bytes src -> dst with one wavefront.
-template <bool CSUM>
+// Copy `len` bytes (0 < len <= kRunMost) src -> dst with one wavefront.
+template <bool KEEP_ENDS, bool CSUM>
 __device__ __forceinline__ uint32_t copy_run(const uint8_t *__restrict__ src,
                                              uint8_t *__restrict__ dst, uint32_t len, uint32_t lane)
 {
   RunState r;
   run_begin(r, src, dst, len, lane);
-  return run_end<CSUM>(r, lane);
+  return run_end<KEEP_ENDS, CSUM>(r, lane);
 }
 
 // A LONG run (jumbo frames) is cut into sub-runs of kPieceChunks destination
@@ -428,7 +497,7 @@ __device__ __forceinline__ uint32_t copy_long_run(const uint8_t *__restrict__ sr
     }
 #pragma unroll
     for (int k = 0; k < DEPTH; k++)
-      if (n[k]) acc += run_end<CSUM>(r[k], lane);
+      if (n[k]) acc += run_end<false, CSUM>(r[k], lane);
     if (!n[DEPTH - 1]) break;
   }
   return acc;

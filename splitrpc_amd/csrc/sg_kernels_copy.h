@@ -238,8 +238,13 @@ __device__ __forceinline__ uint32_t move_run(const AppDev &app, uint64_t req_off
       n = room < (uint64_t)(len - done) ? (uint32_t)room : (len - done);
       p = app.tensor_base[t] + (uint64_t)r * app.tensor_size[t] + (cur - (t1 - app.tensor_size[t]));
     }
-    acc += TO_APP ? copy_run<CSUM>(pkt + done, p, n, lane) : copy_run<CSUM>(p, pkt + done, n, lane);
-    done += n;
+    while (n) {
+      const uint32_t k = n < kRunMost ? n : kRunMost;
+      acc += TO_APP ? copy_run<true, CSUM>(pkt + done, p, k, lane) : copy_run<false, CSUM>(p, pkt + done, k, lane);
+      done += k;
+      p += k;
+      n -= k;
+    }
   }
   return acc;
 }
@@ -350,9 +355,9 @@ __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs a)
     if (LONG) {
       uint32_t o, n;
       sub_run(to, d[1], piece, &o, &n);
-      if (n) copy_run<false>(pkt + o, to + o, n, lane);
+      if (n) copy_run<true, false>(pkt + o, to + o, n, lane);
     } else {
-      copy_run<false>(pkt, to, d[1], lane);
+      copy_run<true, false>(pkt, to, d[1], lane);
     }
   } else if (piece == 0) {
     move_run<true, false>(a.app, ro, d[3], d[2], pkt, d[1], lane);
@@ -567,7 +572,7 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
   if (LONG && plain) sub_run(to, len, piece, &sub_off, &sub_len);
   if (plain && sub_len) run_begin(rs, pkt + hl + sub_off, to + sub_off, sub_len, lane);
   // a fragment that runs from one tensor into the next: two runs, both in flight at once
-  const bool two = !plain && (opts & kOptMultiTensor) && piece == 0 &&
+  const bool two = !plain && (opts & kOptMultiTensor) && piece == 0 && len <= kRunMost &&
                    (plan_kind == 3 ? two_tensor_target(a.app, r, off, len, &to_a, &len_a, &to_b) : plan_kind == 1);
   RunState rb;
   // ... as ONE run with a break in its destination where the second tensor's share starts on a
@@ -583,12 +588,12 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
   }
   asm volatile("" ::"v"(hc), "v"(hv));  // consumed only after the payload loads are under way
   if (plain) {
-    if (sub_len) run_end<false>(rs, lane);
+    if (sub_len) run_end<true, false>(rs, lane);
   } else if (one_run) {
-    run_end<false, true>(rs, lane, (len_a - head_a) >> 4, (int64_t)(to_b - (to_a + len_a)));
+    run_end<false, false, true>(rs, lane, (len_a - head_a) >> 4, (int64_t)(to_b - (to_a + len_a)));
   } else if (two) {
-    run_end<false>(rs, lane);
-    run_end<false>(rb, lane);
+    run_end<true, false>(rs, lane);
+    run_end<true, false>(rb, lane);
   } else if (piece == 0) {
     move_run<true, false>(a.app, ro, r, off, pkt + hl, len, lane);
   }
@@ -926,7 +931,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
     if (d[1] && scatter_source<FUSED>(a, ro, r, item - f0, d[2], d[1], &from, kernarg_base)) {
       uint32_t o, n;
       sub_run(slot + hl, d[1], piece, &o, &n);
-      if (n) part = copy_run<DEFER>(from + o, slot + hl + o, n, lane);
+      if (n) part = copy_run<false, DEFER>(from + o, slot + hl + o, n, lane);
     }
     if (DEFER) {
       part = wave_sum_uniform(part);
@@ -953,7 +958,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
   if (!FULL_CSUM) hb = hdrw_csums(hb, hf, 0);
   if (plain) {
     if (WHOLE_LONG) acc = copy_long_run<FULL_CSUM, 2>(from, slot + hl, d[1], lane);
-    else acc = run_end<FULL_CSUM>(rs, lane);
+    else acc = run_end<false, FULL_CSUM>(rs, lane);
   } else if (d[1]) {
     acc = move_run<false, FULL_CSUM>(a.app, ro, r, d[2], slot + hl, d[1], lane);
   }
@@ -1258,14 +1263,15 @@ struct Run {
 
 __device__ __forceinline__ void copy_one_run(const Run &r, uint32_t lane)
 {
-  copy_run<false>(reinterpret_cast<const uint8_t *>(r.src), reinterpret_cast<uint8_t *>(r.dst), (uint32_t)r.len, lane);
+  copy_run<true, false>(reinterpret_cast<const uint8_t *>(r.src), reinterpret_cast<uint8_t *>(r.dst), (uint32_t)r.len, lane);
 }
 
 __global__ __launch_bounds__(kBlock) void k_copy_runs(const Run *runs, uint32_t n)
 {
-  const uint32_t item = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+  const uint32_t item = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave);
   if (item >= n) return;
-  copy_one_run(runs[item], threadIdx.x & (kWave - 1));
+  const uint64_t *p = reinterpret_cast<const uint64_t *>(runs + item);
+  copy_one_run(Run{sload_here(p), sload_here(p + 1), sload_here(p + 2)}, threadIdx.x & (kWave - 1));
 }
 
 // A call waits for its kernel, and a short table that lies in pinned host memory is a round trip
