@@ -48,6 +48,8 @@ __device__ __forceinline__ u32x4 load16_aligned(const uint8_t *p)
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
 }
 
+__device__ __forceinline__ u32x4 load16_aligned_kept(const uint8_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
+
 typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
 
 // Address of byte `off` of the running kernel's argument block.  A kernel with one by-value
@@ -300,6 +302,7 @@ __device__ __forceinline__ Piece piece_of(const uint8_t *p, uint32_t bytes)
 }
 constexpr int kNontemporal = 2;
 constexpr uint32_t kNowhere = 0x80000000u;  // an offset beyond every piece
+__device__ __forceinline__ u32x4 piece_load16_kept(Piece p, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(p, (int)off, 0, 0); }
 __device__ __forceinline__ u32x4 piece_load16(Piece p, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(p, (int)off, 0, kNontemporal); }
 __device__ __forceinline__ void piece_store16_kept(Piece p, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, p, (int)off, 0, 0); }
 __device__ __forceinline__ void piece_store16(Piece p, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, p, (int)off, 0, kNontemporal); }
@@ -346,12 +349,25 @@ struct RunState {
   uint32_t eoff;   // this lane's edge byte, if any
   uint32_t eb;
   bool edge;
+  bool keep;       // loads without the nontemporal hint
   u32x4 v0, v1;
 };
 
-__device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict__ src,
-                                          uint8_t *__restrict__ dst, uint32_t len, uint32_t lane)
+__device__ __forceinline__ void run_load(RunState &r, uint32_t base)
 {
+  if (r.keep) {
+    r.v0 = piece_load16_kept(r.in, r.at + base);
+    r.v1 = piece_load16_kept(r.in, r.at + base + kStep);
+  } else {
+    r.v0 = piece_load16(r.in, r.at + base);
+    r.v1 = piece_load16(r.in, r.at + base + kStep);
+  }
+}
+
+__device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict__ src,
+                                          uint8_t *__restrict__ dst, uint32_t len, uint32_t lane, bool keep)
+{
+  r.keep = keep;
   uint32_t head = (uint32_t)(-(uintptr_t)dst) & 15u;
   head = head < len ? head : len;
   const uint32_t rest = len - head, tail = rest & 15u;
@@ -367,8 +383,7 @@ __device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict
   r.edge = k < (second ? tail : head);
   r.eoff = k + (second ? head + r.body : 0u);
   r.eb = __builtin_amdgcn_raw_buffer_load_b8(r.in, (int)(s0 + r.eoff), 0, 0);
-  r.v0 = piece_load16(r.in, r.at);
-  r.v1 = piece_load16(r.in, r.at + kStep);
+  run_load(r, 0);
 }
 
 // With CSUM returns this lane's share of the sum of the 16-bit little-endian
@@ -428,8 +443,7 @@ __device__ __forceinline__ uint32_t run_end(RunState &r, uint32_t lane, uint32_t
   };
   put(0);
   for (uint32_t base = 2 * kStep; __builtin_expect(base < r.body, 0); base += 2 * kStep) {
-    r.v0 = piece_load16(r.in, r.at + base);
-    r.v1 = piece_load16(r.in, r.at + base + kStep);
+    run_load(r, base);
     put(base);
   }
   if (r.edge) {
@@ -444,10 +458,10 @@ __device__ __forceinline__ uint32_t run_end(RunState &r, uint32_t lane, uint32_t
 // Copy `len` bytes (0 < len <= kRunMost) src -> dst with one wavefront.
 template <bool KEEP_ENDS, bool CSUM>
 __device__ __forceinline__ uint32_t copy_run(const uint8_t *__restrict__ src,
-                                             uint8_t *__restrict__ dst, uint32_t len, uint32_t lane)
+                                             uint8_t *__restrict__ dst, uint32_t len, uint32_t lane, bool keep)
 {
   RunState r;
-  run_begin(r, src, dst, len, lane);
+  run_begin(r, src, dst, len, lane, keep);
   return run_end<KEEP_ENDS, CSUM>(r, lane);
 }
 
@@ -483,7 +497,7 @@ __device__ __forceinline__ void sub_run(const uint8_t *dst, uint32_t len, uint32
 // Copy a whole long run with one wavefront, DEPTH sub-runs in flight at a time.
 template <bool CSUM, int DEPTH>
 __device__ __forceinline__ uint32_t copy_long_run(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst,
-                                                  uint32_t len, uint32_t lane)
+                                                  uint32_t len, uint32_t lane, bool keep)
 {
   uint32_t acc = 0;
   for (uint32_t base = 0;; base += DEPTH) {
@@ -493,7 +507,7 @@ __device__ __forceinline__ uint32_t copy_long_run(const uint8_t *__restrict__ sr
     for (int k = 0; k < DEPTH; k++) {
       uint32_t o;
       sub_run(dst, len, base + k, &o, &n[k]);
-      if (n[k]) run_begin(r[k], src + o, dst + o, n[k], lane);
+      if (n[k]) run_begin(r[k], src + o, dst + o, n[k], lane, keep);
     }
 #pragma unroll
     for (int k = 0; k < DEPTH; k++)
@@ -697,7 +711,7 @@ struct GroupRun {
 
 template <int L>
 __device__ __forceinline__ void group_run_begin(GroupRun<L> &r, const uint8_t *src, uint8_t *dst, uint32_t len,
-                                                uint32_t gl)
+                                                uint32_t gl, bool keep)
 {
   uint32_t head = (uint32_t)(-(uintptr_t)dst) & 15u;
   head = head < len ? head : len;
@@ -721,9 +735,13 @@ __device__ __forceinline__ void group_run_begin(GroupRun<L> &r, const uint8_t *s
   r.lim = r.p ? body : body - 1;  // body == 0: lim wraps, guarded below
   r.v0 = (u32x4){0, 0, 0, 0};
   r.v1 = (u32x4){0, 0, 0, 0};
-  if (body) {
-    if (gl <= r.lim) r.v0 = load16_aligned(r.sa + ((size_t)gl << 4));
-    if ((L - 1) + gl <= r.lim) r.v1 = load16_aligned(r.sa + ((size_t)((L - 1) + gl) << 4));
+  const bool l0 = body && gl <= r.lim, l1 = body && (L - 1) + gl <= r.lim;
+  if (keep) {
+    if (l0) r.v0 = load16_aligned_kept(r.sa + ((size_t)gl << 4));
+    if (l1) r.v1 = load16_aligned_kept(r.sa + ((size_t)((L - 1) + gl) << 4));
+  } else {
+    if (l0) r.v0 = load16_aligned(r.sa + ((size_t)gl << 4));
+    if (l1) r.v1 = load16_aligned(r.sa + ((size_t)((L - 1) + gl) << 4));
   }
 }
 

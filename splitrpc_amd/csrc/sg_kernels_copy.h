@@ -199,7 +199,7 @@ __device__ __forceinline__ uint32_t rule_desc(const RuleArgs &g, const AppDev &a
 // SG_MAX_TENSORS pieces.
 template <bool TO_APP, bool CSUM>
 __device__ __forceinline__ uint32_t move_run(const AppDev &app, uint64_t req_off, uint32_t r,
-                                             uint32_t off, uint8_t *pkt, uint32_t len, uint32_t lane)
+                                             uint32_t off, uint8_t *pkt, uint32_t len, uint32_t lane, bool keep)
 {
   uint32_t acc = 0;
   const bool packed = app.n_tensors == 0;
@@ -240,7 +240,7 @@ __device__ __forceinline__ uint32_t move_run(const AppDev &app, uint64_t req_off
     }
     while (n) {
       const uint32_t k = n < kRunMost ? n : kRunMost;
-      acc += TO_APP ? copy_run<true, CSUM>(pkt + done, p, k, lane) : copy_run<false, CSUM>(p, pkt + done, k, lane);
+      acc += TO_APP ? copy_run<true, CSUM>(pkt + done, p, k, lane, keep) : copy_run<false, CSUM>(p, pkt + done, k, lane, keep);
       done += k;
       p += k;
       n -= k;
@@ -322,7 +322,7 @@ __device__ __forceinline__ bool two_tensor_target(const AppDev &app, uint32_t r,
 // `pieces` consecutive wavefronts.  (Several fragments per wavefront were
 // measured too: two cost 2 %, three 13 % on 1400-byte fragments -- the number
 // of wavefronts in flight is what covers the HBM latency.)
-template <bool LONG>
+template <bool LONG, bool KEEP>
 __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs a)
 {
   const u32x4 *desc = a.desc;
@@ -355,12 +355,12 @@ __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs a)
     if (LONG) {
       uint32_t o, n;
       sub_run(to, d[1], piece, &o, &n);
-      if (n) copy_run<true, false>(pkt + o, to + o, n, lane);
+      if (n) copy_run<true, false>(pkt + o, to + o, n, lane, KEEP);
     } else {
-      copy_run<true, false>(pkt, to, d[1], lane);
+      copy_run<true, false>(pkt, to, d[1], lane, KEEP);
     }
   } else if (piece == 0) {
-    move_run<true, false>(a.app, ro, d[3], d[2], pkt, d[1], lane);
+    move_run<true, false>(a.app, ro, d[3], d[2], pkt, d[1], lane, KEEP);
   }
 }
 
@@ -402,7 +402,7 @@ struct alignas(64) GatherRuleArgs {
   uint32_t hl;
   uint32_t n_slots;
   uint32_t pieces;            // wavefronts per fragment
-  uint32_t opts;  // kOptRemap | kOptMirrored | kOptMultiTensor | kOptHdrChunk
+  uint32_t opts;  // kOptRemap | kOptMirrored | kOptKeep | kOptMultiTensor | kOptHdrChunk
   // warm
   uint32_t n_req;
   const uint32_t *frag_len;
@@ -424,6 +424,7 @@ constexpr uint32_t kOptRemap = 1u, kOptMirrored = 2u, kOptMultiTensor = 8u;
 // slots start at 16-byte aligned addresses: the header's length field can be read as part of
 // the aligned chunk at byte 48 (a ring only has to start at an even address)
 constexpr uint32_t kOptHdrChunk = 16u;
+constexpr uint32_t kOptKeep = 4u;  // ADV kernels: loads without the nontemporal hint
 constexpr uint32_t kOptSmallLast = 32u;  // the last fragment of every request is left to k_gather_small
 
 template <int L, bool ADV>
@@ -433,7 +434,9 @@ __device__ __forceinline__ void gather_small_wave(const GatherRuleArgs &a, uint3
 // request is short -- the wavefronts behind those of the full fragments then move
 // 64 / SMALL remainder fragments each, in the same launch (a launch of their own
 // would be all latency: tens of megabytes at most); 0: no such wavefronts.
-// ADV: the kernel takes the cursor from a context's cells and advances it itself (no k_finish follows).
+// ADV: the kernel takes the cursor from a context's cells and advances it itself (no k_finish follows),
+// and has the loads without the nontemporal hint for the calls that want them (kOptKeep): chosen at run
+// time in every instance, they cost 131072 requests of 2048 bytes 268 -> 275 us.
 // `block`: the workgroup's number among those of this work; `kernarg_base`: where `a` lies in the
 // running kernel's argument block (the plan is read through the argument pointer).
 template <bool LONG, int SMALL, bool ADV>
@@ -570,7 +573,8 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
   RunState rs;
   uint32_t sub_off = 0, sub_len = len;
   if (LONG && plain) sub_run(to, len, piece, &sub_off, &sub_len);
-  if (plain && sub_len) run_begin(rs, pkt + hl + sub_off, to + sub_off, sub_len, lane);
+  const bool keep = ADV && (opts & kOptKeep);
+  if (plain && sub_len) run_begin(rs, pkt + hl + sub_off, to + sub_off, sub_len, lane, keep);
   // a fragment that runs from one tensor into the next: two runs, both in flight at once
   const bool two = !plain && (opts & kOptMultiTensor) && piece == 0 && len <= kRunMost &&
                    (plan_kind == 3 ? two_tensor_target(a.app, r, off, len, &to_a, &len_a, &to_b) : plan_kind == 1);
@@ -581,10 +585,10 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
   const uint32_t head_a = (uint32_t)(-(uintptr_t)to_a) & 15u;
   const bool one_run = two && ((uintptr_t)to_b & 15u) == 0 && len_a >= head_a && ((len_a - head_a) & 15u) == 0;
   if (one_run) {
-    run_begin(rs, pkt + hl, to_a, len, lane);
+    run_begin(rs, pkt + hl, to_a, len, lane, keep);
   } else if (two) {
-    run_begin(rs, pkt + hl, to_a, len_a, lane);
-    run_begin(rb, pkt + hl + len_a, to_b, len - len_a, lane);
+    run_begin(rs, pkt + hl, to_a, len_a, lane, keep);
+    run_begin(rb, pkt + hl + len_a, to_b, len - len_a, lane, keep);
   }
   asm volatile("" ::"v"(hc), "v"(hv));  // consumed only after the payload loads are under way
   if (plain) {
@@ -595,7 +599,7 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
     run_end<true, false>(rs, lane);
     run_end<true, false>(rb, lane);
   } else if (piece == 0) {
-    move_run<true, false>(a.app, ro, r, off, pkt + hl, len, lane);
+    move_run<true, false>(a.app, ro, r, off, pkt + hl, len, lane, keep);
   }
   if (piece == 0) {
     uint32_t bad = 0;
@@ -705,7 +709,7 @@ __device__ __forceinline__ void gather_small_wave(const GatherRuleArgs &a, uint3
     }
   }
   GroupRun<L> run;
-  group_run_begin<L>(run, pkt + hl, to, plain ? len : 0u, gl);
+  group_run_begin<L>(run, pkt + hl, to, plain ? len : 0u, gl, ADV && (a.opts & kOptKeep));
   group_run_end<L, false>(run, gl);
   if (live && len && !plain) {
     // across an arena end or a tensor boundary: byte by byte
@@ -748,7 +752,7 @@ struct alignas(64) ScatterArgs {
   uint64_t *cursor;             // descriptor path, packed: wavefront 0 commits *next_cursor
   const uint64_t *next_cursor;
   uint32_t cursor_cells;        // the cursor is a context's pair of cells, not a plain word
-  uint32_t cursor_pad;
+  uint32_t keep;                // ADV kernels: loads without the nontemporal hint
   const uint32_t *hdr_src_req;  // one header source per request instead of hdr_src_slot per frame
   const uint32_t *counts;       // device-resident request count, or nullptr
   // full UDP checksum of long frames in two phases: every sub-run's wavefront leaves the sum of
@@ -800,7 +804,8 @@ constexpr uint32_t kPartStride = 8;  // words of csum_part per frame: up to 7 su
 // DEFER (long frames with the full UDP checksum): the frame's sub-runs go to
 // several wavefronts all the same, each leaving the sum of its bytes behind,
 // and k_udp_finish writes the checksum field afterwards.
-// ADV (fused only): the kernel takes the cursor from a context's cells and advances it itself.
+// ADV: as in gather_rule_body.  Not fused there is no cursor to derive offsets from: the instance whose
+// loads go without the hint.
 template <bool FULL_CSUM, bool FUSED, bool LONG, bool DEFER, bool ADV>
 __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t block, size_t kernarg_base)
 {
@@ -814,6 +819,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
   uint8_t *tx = a.tx;
   const uint32_t rx_slot_size = a.rx_slot_size, rx_n_slots = a.rx_n_slots, tx_slot_size = a.tx_slot_size;
   const uint32_t hl = a.hl, remap = a.remap, n_pieces = a.pieces;
+  const bool keep = ADV && (!FUSED || a.keep);
   const uint32_t *status = a.status;
   const uint32_t *counts = a.counts, *hdr_src_req = a.hdr_src_req;
   uint32_t n_items = a.n_items, n_req = a.n_req;
@@ -931,7 +937,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
     if (d[1] && scatter_source<FUSED>(a, ro, r, item - f0, d[2], d[1], &from, kernarg_base)) {
       uint32_t o, n;
       sub_run(slot + hl, d[1], piece, &o, &n);
-      if (n) part = copy_run<false, DEFER>(from + o, slot + hl + o, n, lane);
+      if (n) part = copy_run<false, DEFER>(from + o, slot + hl + o, n, lane, keep);
     }
     if (DEFER) {
       part = wave_sum_uniform(part);
@@ -953,14 +959,14 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
     uint32_t o;
     sub_run(slot + hl, d[1], 0, &o, &first_len);
   }
-  if (plain && !WHOLE_LONG) run_begin(rs, from, slot + hl, first_len, lane);
+  if (plain && !WHOLE_LONG) run_begin(rs, from, slot + hl, first_len, lane, keep);
   hb = hdrw_fields(raw, hf);
   if (!FULL_CSUM) hb = hdrw_csums(hb, hf, 0);
   if (plain) {
-    if (WHOLE_LONG) acc = copy_long_run<FULL_CSUM, 2>(from, slot + hl, d[1], lane);
+    if (WHOLE_LONG) acc = copy_long_run<FULL_CSUM, 2>(from, slot + hl, d[1], lane, keep);
     else acc = run_end<false, FULL_CSUM>(rs, lane);
   } else if (d[1]) {
-    acc = move_run<false, FULL_CSUM>(a.app, ro, r, d[2], slot + hl, d[1], lane);
+    acc = move_run<false, FULL_CSUM>(a.app, ro, r, d[2], slot + hl, d[1], lane, keep);
   }
   // the header's own share of the UDP sum rides with the payload's
   if (FULL_CSUM) acc += hdrw_l4_share(hb, lane, hl);
@@ -1105,7 +1111,7 @@ __device__ __forceinline__ void scatter_small_wave(const ScatterArgs &a, uint32_
   }
   GroupRun<L> run;
   if (early)
-    group_run_begin<L>(run, from, reinterpret_cast<uint8_t *>(((uintptr_t)a.tx + hl) & 15u), plain ? len : 0u, gl);
+    group_run_begin<L>(run, from, reinterpret_cast<uint8_t *>(((uintptr_t)a.tx + hl) & 15u), plain ? len : 0u, gl, ADV && a.keep);
   if (tslot >= a.rule.n_slots) bad |= kStBadSlot;
   if (i == 0 && first_r != item) bad |= kStBadTable;
   if (hs >= a.rx_n_slots) bad |= kStBadSlot;
@@ -1141,7 +1147,7 @@ __device__ __forceinline__ void scatter_small_wave(const ScatterArgs &a, uint32_
     group_run_rebase<L>(run, slot + hl);
     if (!plain) group_run_cancel<L>(run);  // a frame the tables have just ruled out
   } else {
-    group_run_begin<L>(run, from, slot + hl, plain ? len : 0u, gl);
+    group_run_begin<L>(run, from, slot + hl, plain ? len : 0u, gl, ADV && a.keep);
   }
   uint32_t acc = group_run_end<L, FULL_CSUM>(run, gl);
   if (live && len != 0 && !plain) {
@@ -1263,7 +1269,7 @@ struct Run {
 
 __device__ __forceinline__ void copy_one_run(const Run &r, uint32_t lane)
 {
-  copy_run<true, false>(reinterpret_cast<const uint8_t *>(r.src), reinterpret_cast<uint8_t *>(r.dst), (uint32_t)r.len, lane);
+  copy_run<true, false>(reinterpret_cast<const uint8_t *>(r.src), reinterpret_cast<uint8_t *>(r.dst), (uint32_t)r.len, lane, false);
 }
 
 __global__ __launch_bounds__(kBlock) void k_copy_runs(const Run *runs, uint32_t n)
