@@ -26,6 +26,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -111,15 +112,16 @@ struct sg_hip_ctx {
   uint32_t *csum_scratch = nullptr;  // csum_part and csum_valid
   uint32_t desc_gen = 0;
   uint32_t call_seq = 0;
-  uint32_t *status = nullptr;
+  uint32_t *status = nullptr;  // [0] refusals, [1] DoneArgs::count
   Scratch sc;
   // pinned staging for the per-request entry points (device reads it in place)
   Run *h_runs = nullptr;
   uint32_t h_runs_cap = 0;
   uint64_t *h_ptrs = nullptr;
   bool staging_read = false;  // a launch that reads h_runs or h_ptrs has not been waited for
+  uint32_t done_seq = 0;         // per-request launches that tell when they are through
   uint64_t *h_probe = nullptr;   // pinned: what a probe launch saw of itself (queue address, dispatch id), twice
-  uint32_t *h_status = nullptr;  // pinned: [0] copy of status (read back only after a refusal), [1] the refusal flag
+  uint32_t *h_status = nullptr;  // pinned: [0] copy of status (read back only after a refusal), [1] the refusal flag, [2] DoneArgs::word
   volatile uint32_t *h_flag = nullptr;
   // profiling
   bool profiling = false;
@@ -629,7 +631,7 @@ static int create_impl(sg_hip_ctx *c, int device_id, const sg_hip_cfg *cfg)
   HIP_TRY(nullptr, hipMalloc(&c->req_off, sizeof(uint64_t) * (size_t)c->max_reqs));
   HIP_TRY(nullptr, hipMalloc(&c->tile_tot, sizeof(uint64_t) * ((size_t)c->max_reqs / kPartMin + 2)));
   HIP_TRY(nullptr, hipMalloc(&c->cursors, kCtxWords * sizeof(uint64_t)));
-  HIP_TRY(nullptr, hipMalloc(&c->status, sizeof(uint32_t)));
+  HIP_TRY(nullptr, hipMalloc(&c->status, 2 * sizeof(uint32_t)));
   HIP_TRY(nullptr, hipMalloc(&c->csum_scratch, sizeof(uint32_t) * (size_t)c->max_frames * (kPartStride + 1)));
   HIP_TRY(nullptr, hipMemsetAsync(c->csum_scratch, 0, sizeof(uint32_t) * (size_t)c->max_frames * (kPartStride + 1), c->stream));
   {
@@ -638,12 +640,12 @@ static int create_impl(sg_hip_ctx *c, int device_id, const sg_hip_cfg *cfg)
     init[kCurStamp] = init[kCurWords + kCurStamp] = 1;
     HIP_TRY(nullptr, hipMemcpy(c->cursors, init, sizeof init, hipMemcpyHostToDevice));
   }
-  HIP_TRY(nullptr, hipMemsetAsync(c->status, 0, sizeof(uint32_t), c->stream));
+  HIP_TRY(nullptr, hipMemsetAsync(c->status, 0, 2 * sizeof(uint32_t), c->stream));
   c->h_runs_cap = 8192;
   HIP_TRY(nullptr, hipHostMalloc(&c->h_runs, sizeof(Run) * c->h_runs_cap, hipHostMallocDefault));
   HIP_TRY(nullptr, hipHostMalloc(&c->h_ptrs, sizeof(uint64_t) * (SG_MAX_BI_SIZE + 8), hipHostMallocDefault));
-  HIP_TRY(nullptr, hipHostMalloc(&c->h_status, 2 * sizeof(uint32_t), hipHostMallocDefault));
-  c->h_status[0] = c->h_status[1] = 0;
+  HIP_TRY(nullptr, hipHostMalloc(&c->h_status, 3 * sizeof(uint32_t), hipHostMallocDefault));
+  c->h_status[0] = c->h_status[1] = c->h_status[2] = 0;
   c->h_flag = c->h_status + 1;
   HIP_TRY(nullptr, hipStreamSynchronize(c->stream));
   // The self-advancing cursor rests on every launch seeing a queue address and a dispatch id of
@@ -840,20 +842,56 @@ static int staging_free(sg_hip_ctx *c)
   return SG_OK;
 }
 
-// Copies the n runs staged in c->h_runs.
-static int launch_runs(sg_hip_ctx *c, uint32_t n)
+// What a per-request launch that the call waits for is given to tell that it is through.
+static DoneArgs done_args(sg_hip_ctx *c)
+{
+  DoneArgs d;
+  d.count = c->status + 1;
+  d.word = c->profiling ? nullptr : c->h_status + 2;  // (events to be waited for anyway)
+  d.status = c->status;
+  d.seq = ++c->done_seq & 0x7fffffffu;
+  return d;
+}
+
+// The end of a per-request call: waits for the launch that was given the last done_args.
+static int finish_request(sg_hip_ctx *c)
+{
+  HIP_TRY(c, hipGetLastError());
+  if (!c->profiling) {
+    // some 100 us of looking; what takes longer has much to do, waits behind other work or has failed,
+    // and is left to the runtime
+    const volatile uint32_t *word = c->h_status + 2;
+    const uint32_t want = (c->done_seq & 0x7fffffffu) << 1;
+    for (int i = 0; i < 4000; i++) {
+      const uint32_t w = *word;
+      if ((w & ~1u) == want) {
+        std::atomic_thread_fence(std::memory_order_acquire);
+        if (w & 1u) break;  // a refusal to be fetched
+        return SG_OK;
+      }
+      __builtin_ia32_pause();
+    }
+  }
+  return sg_hip_sync(c);
+}
+
+// Copies the n runs staged in c->h_runs; `last`: the call waits for this launch.
+static int launch_runs(sg_hip_ctx *c, uint32_t n, bool last)
 {
   int rc = prof_begin(c, 3);
   if (rc != SG_OK) return rc;
   const uint32_t grid = (n + kWavesPerBlock - 1) / kWavesPerBlock;
+  DoneArgs done = {};
+  if (last) done = done_args(c);
   if (n <= kInlineRuns) {
     RunsInline a;
     memcpy(a.run, c->h_runs, n * sizeof(Run));
     a.n = n;
+    a.done = done;
     k_copy_runs_inline<<<grid, kBlock, 0, c->stream>>>(a);
   } else {
     c->staging_read = true;
-    k_copy_runs<<<grid, kBlock, 0, c->stream>>>(c->h_runs, n);
+    k_copy_runs<<<grid, kBlock, 0, c->stream>>>(c->h_runs, n, done);
   }
   return prof_end(c);
 }
@@ -879,7 +917,7 @@ static int copy_skb(sg_hip_ctx *c, const sg_sk_buf *skb)
       }
       if (n == c->h_runs_cap) {
         // flush what is staged and start over
-        rc = launch_runs(c, n);
+        rc = launch_runs(c, n, false);
         if (rc == SG_OK) rc = staging_free(c);
         if (rc != SG_OK) return rc;
         n = 0;
@@ -889,10 +927,12 @@ static int copy_skb(sg_hip_ctx *c, const sg_sk_buf *skb)
     }
   }
   if (n) {
-    rc = launch_runs(c, n);
+    rc = launch_runs(c, n, true);
     if (rc != SG_OK) return rc;
+    rc = finish_request(c);
+  } else {
+    rc = finish(c, 0);
   }
-  rc = finish(c, 0);
   if (rc == SG_OK || rc == SG_E_DATA) c->staging_read = false;  // waited for
   return rc;
 }
@@ -927,7 +967,9 @@ static int fill_hdrs(sg_hip_ctx *c, const sg_hbufs *hdrs, const uint8_t *tmpl, u
   rc = prof_begin(c, 4);
   if (rc != SG_OK) return rc;
   const uint32_t grid = (n + kWavesPerBlock - 1) / kWavesPerBlock;
+  const DoneArgs done = done_args(c);
   if (n <= kInlineHdrs) {
+    s.done = done;
     if (tmpl) memcpy(s.tmpl, tmpl, sizeof s.tmpl);
     memcpy(s.hdr, hdrs->burst_items, n * sizeof(uint64_t));
     k_swap_hdrs_inline<<<grid, kBlock, 0, c->stream>>>(s);
@@ -936,11 +978,11 @@ static int fill_hdrs(sg_hip_ctx *c, const sg_hbufs *hdrs, const uint8_t *tmpl, u
     // the template rides behind the pointer table in the same pinned block
     if (tmpl) memcpy(c->h_ptrs + SG_MAX_BI_SIZE, tmpl, 64);
     c->staging_read = true;
-    k_swap_hdrs<<<grid, kBlock, 0, c->stream>>>(s.a, c->h_ptrs, reinterpret_cast<const uint8_t *>(c->h_ptrs + SG_MAX_BI_SIZE));
+    k_swap_hdrs<<<grid, kBlock, 0, c->stream>>>(s.a, c->h_ptrs, reinterpret_cast<const uint8_t *>(c->h_ptrs + SG_MAX_BI_SIZE), done);
   }
   rc = prof_end(c);
   if (rc != SG_OK) return rc;
-  rc = finish(c, 0);
+  rc = finish_request(c);
   if (rc == SG_OK || rc == SG_E_DATA) c->staging_read = false;  // waited for
   return rc;
 }
