@@ -181,9 +181,9 @@ __device__ __forceinline__ uint32_t rule_desc(const RuleArgs &g, const AppDev &a
     if (g.single_wrap) o = o >= app.cap ? o - app.cap : o;  // n_req * size <= capacity
     else o %= app.cap;
     *req_off = o;
-    if (lane == 0) {
-      if (*i == 0 && g.offsets_out) g.offsets_out[*r] = *req_off;
-      if (item == n_items - 1 && g.offsets_out) {
+    if ((*i == 0 || item == n_items - 1) && lane == 0 && g.offsets_out) {
+      if (*i == 0) g.offsets_out[*r] = *req_off;
+      if (item == n_items - 1) {
         uint64_t end = *req_off + g.size;  // size <= capacity
         end = end >= app.cap ? end - app.cap : end;
         g.offsets_out[n_req] = end;
@@ -522,7 +522,7 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
       cursor_advance(cursor_in - kCurPlain, a.call_seq, cur_live, cur_stamp, cursor_bump(c0, n_req, size, cap));
     ro = c0 + (uint64_t)r * size;
     ro = ro >= cap ? ro - cap : ro;  // the batch fits the arena (checked by the host): one wrap at most
-    if (lane == 0 && piece == 0 && a.offsets_out) {
+    if (piece == 0 && (i == 0 || item == n_items - 1) && lane == 0 && a.offsets_out) {
       if (i == 0) a.offsets_out[r] = ro;
       if (item == n_items - 1) {
         uint64_t end = ro + size;  // size <= capacity
@@ -569,37 +569,44 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
     if (opts & kOptHdrChunk) hc = *reinterpret_cast<const u32x4 *>(pkt + 48);
     else hv = load32_any(pkt + 54);
   }
-  // copying the ruled length stays inside the slot whatever the header says
-  RunState rs;
-  uint32_t sub_off = 0, sub_len = len;
-  if (LONG && plain) sub_run(to, len, piece, &sub_off, &sub_len);
+  // Copying the ruled length stays inside the slot whatever the header says.  The header words are
+  // consumed only after the payload loads are under way.  (Every shape of a run is begun and ended in
+  // a branch of its own: begun in one place and ended in another, its state goes through registers
+  // and lanes the branches in between agree on.)
   const bool keep = ADV && (opts & kOptKeep);
-  if (plain && sub_len) run_begin(rs, pkt + hl + sub_off, to + sub_off, sub_len, lane, keep);
-  // a fragment that runs from one tensor into the next: two runs, both in flight at once
-  const bool two = !plain && (opts & kOptMultiTensor) && piece == 0 && len <= kRunMost &&
-                   (plan_kind == 3 ? two_tensor_target(a.app, r, off, len, &to_a, &len_a, &to_b) : plan_kind == 1);
-  RunState rb;
-  // ... as ONE run with a break in its destination where the second tensor's share starts on a
-  // 16-byte boundary and the first one's ends on a chunk boundary of the run (tensors of whole
-  // chunks at aligned addresses)
-  const uint32_t head_a = (uint32_t)(-(uintptr_t)to_a) & 15u;
-  const bool one_run = two && ((uintptr_t)to_b & 15u) == 0 && len_a >= head_a && ((len_a - head_a) & 15u) == 0;
-  if (one_run) {
-    run_begin(rs, pkt + hl, to_a, len, lane, keep);
-  } else if (two) {
-    run_begin(rs, pkt + hl, to_a, len_a, lane, keep);
-    run_begin(rb, pkt + hl + len_a, to_b, len - len_a, lane, keep);
-  }
-  asm volatile("" ::"v"(hc), "v"(hv));  // consumed only after the payload loads are under way
+  auto under_way = [&] { asm volatile("" ::"v"(hc), "v"(hv)); };
   if (plain) {
-    if (sub_len) run_end<true, false>(rs, lane);
-  } else if (one_run) {
-    run_end<false, false, true>(rs, lane, (len_a - head_a) >> 4, (int64_t)(to_b - (to_a + len_a)));
-  } else if (two) {
-    run_end<true, false>(rs, lane);
-    run_end<true, false>(rb, lane);
+    uint32_t sub_off = 0, sub_len = len;
+    if (LONG) sub_run(to, len, piece, &sub_off, &sub_len);
+    if (sub_len) {
+      RunState rs;
+      run_begin(rs, pkt + hl + sub_off, to + sub_off, sub_len, lane, keep);
+      under_way();
+      run_end<true, false>(rs, lane);
+    }
   } else if (piece == 0) {
-    move_run<true, false>(a.app, ro, r, off, pkt + hl, len, lane, keep);
+    // a fragment that runs from one tensor into the next: two runs, both in flight at once ...
+    const bool two = (opts & kOptMultiTensor) && len <= kRunMost &&
+                     (plan_kind == 3 ? two_tensor_target(a.app, r, off, len, &to_a, &len_a, &to_b) : plan_kind == 1);
+    // ... as ONE run with a break in its destination where the second tensor's share starts on a
+    // 16-byte boundary and the first one's ends on a chunk boundary of the run (tensors of whole
+    // chunks at aligned addresses)
+    const uint32_t head_a = (uint32_t)(-(uintptr_t)to_a) & 15u;
+    if (two && ((uintptr_t)to_b & 15u) == 0 && len_a >= head_a && ((len_a - head_a) & 15u) == 0) {
+      RunState rs;
+      run_begin(rs, pkt + hl, to_a, len, lane, keep);
+      under_way();
+      run_end<false, false, true>(rs, lane, (len_a - head_a) >> 4, (int64_t)(to_b - (to_a + len_a)));
+    } else if (two) {
+      RunState rs, rb;
+      run_begin(rs, pkt + hl, to_a, len_a, lane, keep);
+      run_begin(rb, pkt + hl + len_a, to_b, len - len_a, lane, keep);
+      under_way();
+      run_end<true, false>(rs, lane);
+      run_end<true, false>(rb, lane);
+    } else {
+      move_run<true, false>(a.app, ro, r, off, pkt + hl, len, lane, keep);
+    }
   }
   if (piece == 0) {
     uint32_t bad = 0;
@@ -953,20 +960,26 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
   uint32_t hb = 0, acc = 0;
   uint8_t *from = nullptr;
   const bool plain = d[1] != 0 && scatter_source<FUSED>(a, ro, r, item - f0, d[2], d[1], &from, kernarg_base);
-  RunState rs;
-  uint32_t first_len = d[1];
-  if (SPLIT && plain) {
-    uint32_t o;
-    sub_run(slot + hl, d[1], 0, &o, &first_len);
-  }
-  if (plain && !WHOLE_LONG) run_begin(rs, from, slot + hl, first_len, lane, keep);
-  hb = hdrw_fields(raw, hf);
-  if (!FULL_CSUM) hb = hdrw_csums(hb, hf, 0);
-  if (plain) {
-    if (WHOLE_LONG) acc = copy_long_run<FULL_CSUM, 2>(from, slot + hl, d[1], lane, keep);
-    else acc = run_end<false, FULL_CSUM>(rs, lane);
-  } else if (d[1]) {
-    acc = move_run<false, FULL_CSUM>(a.app, ro, r, d[2], slot + hl, d[1], lane, keep);
+  auto fields = [&] {
+    hb = hdrw_fields(raw, hf);
+    if (!FULL_CSUM) hb = hdrw_csums(hb, hf, 0);
+  };
+  if (plain && WHOLE_LONG) {
+    fields();
+    acc = copy_long_run<FULL_CSUM, 2>(from, slot + hl, d[1], lane, keep);
+  } else if (plain) {
+    uint32_t first_len = d[1];
+    if (SPLIT) {
+      uint32_t o;
+      sub_run(slot + hl, d[1], 0, &o, &first_len);
+    }
+    RunState rs;
+    run_begin(rs, from, slot + hl, first_len, lane, keep);
+    fields();
+    acc = run_end<false, FULL_CSUM>(rs, lane);
+  } else {
+    fields();
+    if (d[1]) acc = move_run<false, FULL_CSUM>(a.app, ro, r, d[2], slot + hl, d[1], lane, keep);
   }
   // the header's own share of the UDP sum rides with the payload's
   if (FULL_CSUM) acc += hdrw_l4_share(hb, lane, hl);
