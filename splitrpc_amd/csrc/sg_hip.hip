@@ -1737,7 +1737,7 @@ int ra_state(sg_hip_ctx *c, RaArgs *r)
     }
     const uint64_t least = ra_cells_for(c->max_reqs, 1);
     auto bytes = [&](uint64_t cells) {
-      return cells * (SG_MAX_BI_SIZE * 8 + 8 + 8 + 3 * 4) + cells / kRaBucket * 4 + kRaWords * 4 + (uint64_t)n_max * (8 + 4) +
+      return cells * (SG_MAX_BI_SIZE * 8 + kRaHead * 8 + 8 + 8 + 3 * 4) + cells / kRaBucket * 4 + kRaWords * 4 + (uint64_t)n_max * (8 + 4) +
              n_blk * 2 * 8 + 256;
     };
     // Four cells per request that may be in flight where the room beyond one cell each is at most a
@@ -1762,6 +1762,7 @@ int ra_state(sg_hip_ctx *c, RaArgs *r)
   memset(r, 0, sizeof *r);
   uint8_t *m = static_cast<uint8_t *>(c->ra_mem);
   r->tab = reinterpret_cast<unsigned long long *>(m); m += (size_t)cells * SG_MAX_BI_SIZE * 8;
+  r->head = reinterpret_cast<unsigned long long *>(m); m += (size_t)cells * kRaHead * 8;
   r->keys = reinterpret_cast<unsigned long long *>(m); m += (size_t)cells * 8;
   r->acc = reinterpret_cast<unsigned long long *>(m); m += (size_t)cells * 8;
   r->blk = reinterpret_cast<unsigned long long *>(m); m += n_blk * 8;

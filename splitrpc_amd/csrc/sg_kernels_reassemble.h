@@ -56,12 +56,13 @@ namespace {
 //   a group of lanes after the other goes
 //   to the table, records from a ring:
 //     insert / flag / scan / emit          23.2 / 5.5 / 4.9 / 8.4    30.1 / 9.7 / 4.7 / 13.0
-//   this form: insert / flag / emit        11.3 / 4.9 / 6.6          14.6 / 4.8 / 7.7
+//   this form: insert / flag / emit        11.3 / 4.9 / 6.6          13.7 / 4.9 / 6.8
 //   64 arrivals in one launch              8.6 -> 5.4, and 3.8 where the counts stay on the device
 // (a launch that does nothing shows as 2 to 4 us there).  Workgroups of 512 threads: 11.9 / 5.2 / 6.0
 // and 14.0 / 5.1 / 9.4; of 1024: 12.2 / 5.2 / 5.8 and 20.5 / 6.8 / 10.8.  The ring of free records
 // cost a returning addition per workgroup to one word, 35 to 70 ns each and one after the other, and
-// two dependent reads per new request.
+// two dependent reads per new request.  With all entries of a record in one place (ra_entry) the second
+// column was 14.7 / 4.9 / 7.5.
 
 constexpr uint32_t kRaBucket = 32;
 static_assert(kRaBucket == 32, "ra_look keeps one bit per cell; a token's first cell is the top five bits of its hash");
@@ -97,7 +98,8 @@ struct RaArgs {
   unsigned long long *acc;   // fragments so far << 40 | payload bytes so far: one atomic addition per workgroup and token
   uint32_t *last;            // position in this call of the token's latest arrival; zero between calls
   uint32_t *want, *seen;     // fragments of the request; epoch of the latest call that brought one
-  unsigned long long *tab;   // a record per cell: SG_MAX_BI_SIZE entries slot | length << 32
+  unsigned long long *tab;   // a record per cell: SG_MAX_BI_SIZE entries slot | length << 32 ...
+  unsigned long long *head;  // ... of which the first kRaHead lie here, a cell's beside the next one's
   uint32_t *words;           // kRa* above
   // per arrival of this call
   uint32_t *arr_cell;            // | kRaOwner
@@ -113,6 +115,15 @@ struct RaArgs {
   uint32_t *status;
   volatile uint32_t *status_flag;  // pinned host word: non-zero once any kernel refused something
 };
+
+// Entry j of a cell's record.  The first few lie apart, 64 bytes a cell: all that a request of a few
+// fragments has, where 65536 such requests spread over records of 8 KB each would have their entries
+// in gigabytes.
+constexpr uint32_t kRaHead = 8;
+__device__ __forceinline__ unsigned long long *ra_entry(const RaArgs &a, uint32_t cell, uint32_t j)
+{
+  return j < kRaHead ? a.head + (size_t)cell * kRaHead + j : a.tab + (size_t)cell * SG_MAX_BI_SIZE + j;
+}
 
 __device__ __forceinline__ uint32_t ra_n(const RaArgs &a)
 {
@@ -394,7 +405,7 @@ __device__ __forceinline__ uint32_t ra_group(RaLds<B> &l, const RaMine &m, uint3
 __device__ __forceinline__ void ra_file(const RaArgs &a, uint32_t cell, const RaMine &m)
 {
   if (m.fidx < SG_MAX_BI_SIZE)
-    a.tab[(size_t)cell * SG_MAX_BI_SIZE + m.fidx] = (unsigned long long)m.slot | ((unsigned long long)m.len << 32);
+    *ra_entry(a, cell, m.fidx) = (unsigned long long)m.slot | ((unsigned long long)m.len << 32);
   else
     refuse(a.status, a.status_flag, kStBadTable);  // beyond what a request's tables hold (src/p2p_bufs.h:10)
 }
@@ -527,27 +538,26 @@ __device__ __forceinline__ void ra_emit(const RaArgs &a, uint32_t cell, unsigned
   // requests of a few fragments are handed over by the completing lane itself, all such lanes
   // at once; the wavefront then walks the larger ones together, eight entries per lane asked for
   // before the first is stored
-  constexpr uint32_t kOwn = 8, kAhead = 8;
+  constexpr uint32_t kOwn = kRaHead, kAhead = 8;
   const uint32_t cnt = ra_done_cnt(done);
   const bool own = done && cnt <= kOwn;
   unsigned long long todo = __ballot(done && !own);
-  unsigned long long *t = a.tab + (size_t)cell * SG_MAX_BI_SIZE;
+  unsigned long long *t = a.head + (size_t)cell * kRaHead;
   unsigned long long e[kOwn], f[kAhead];
   if (own) {
 #pragma unroll
     for (uint32_t j = 0; j < kOwn; j++) e[j] = j < cnt ? t[j] : 0ull;
   }
-  auto ask = [&](const unsigned long long *rec, uint32_t k, uint32_t j0) {
+  auto ask = [&](uint32_t c, uint32_t k, uint32_t j0) {
 #pragma unroll
     for (uint32_t q = 0; q < kAhead; q++) {
       const uint32_t j = j0 + q * kWave + lane;
-      f[q] = j < k ? rec[j] : 0ull;
+      f[q] = j < k ? *ra_entry(a, c, j) : 0ull;
     }
   };
   if (todo) {
     const int l = __ffsll((long long)todo) - 1;
-    ask(a.tab + (size_t)(uint32_t)__builtin_amdgcn_readlane((int)cell, l) * SG_MAX_BI_SIZE,
-        (uint32_t)__builtin_amdgcn_readlane((int)cnt, l), 0);
+    ask((uint32_t)__builtin_amdgcn_readlane((int)cell, l), (uint32_t)__builtin_amdgcn_readlane((int)cnt, l), 0);
   }
   uint64_t before;
   if (!base(&before)) return;
@@ -575,9 +585,8 @@ __device__ __forceinline__ void ra_emit(const RaArgs &a, uint32_t cell, unsigned
     const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)cnt, l);
     const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(at >> 32), l);
     const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)at, l);
-    unsigned long long *rec = a.tab + (size_t)c * SG_MAX_BI_SIZE;
     for (uint32_t j0 = 0; j0 < k; j0 += kAhead * kWave) {
-      if (!asked) ask(rec, k, j0);
+      if (!asked) ask(c, k, j0);
       asked = false;
 #pragma unroll
       for (uint32_t q = 0; q < kAhead; q++) {
@@ -585,7 +594,7 @@ __device__ __forceinline__ void ra_emit(const RaArgs &a, uint32_t cell, unsigned
         if (j < k) {
           a.frag_slot[first + j] = (uint32_t)f[q];
           a.frag_len[first + j] = (uint32_t)(f[q] >> 32);
-          rec[j] = 0;
+          *ra_entry(a, c, j) = 0;
         }
       }
       if (j0 == 0 && lane == 0) {
@@ -765,6 +774,7 @@ __global__ __launch_bounds__(256) void k_ra_reset(RaArgs a)
   }
   // two entries at a time
   for (size_t i = i0; 2 * i < (size_t)a.cells * SG_MAX_BI_SIZE; i += step) reinterpret_cast<u32x4 *>(a.tab)[i] = (u32x4){0u, 0u, 0u, 0u};
+  for (size_t i = i0; 2 * i < (size_t)a.cells * kRaHead; i += step) reinterpret_cast<u32x4 *>(a.head)[i] = (u32x4){0u, 0u, 0u, 0u};
   if (i0 < kRaWords) a.words[i0] = 0;
 }
 
@@ -779,8 +789,7 @@ __global__ __launch_bounds__(256) void k_ra_evict(RaArgs a, uint32_t max_age)
   if (c >= a.cells) return;
   if (a.keys[c] == 0ull) return;
   if (a.words[kRaEpoch] - a.seen[c] <= max_age) return;
-  unsigned long long *t = a.tab + (size_t)c * SG_MAX_BI_SIZE;
-  for (uint32_t j = lane; j < SG_MAX_BI_SIZE; j += kWave) t[j] = 0;
+  for (uint32_t j = lane; j < SG_MAX_BI_SIZE; j += kWave) *ra_entry(a, c, j) = 0;
   if (lane == 0) {
     a.acc[c] = 0;
     a.keys[c] = 0;
