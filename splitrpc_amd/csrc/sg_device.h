@@ -128,10 +128,15 @@ __device__ __forceinline__ uint64_t cursor_get(const uint64_t *p, bool cells)
 {
   return p[cells ? kCurPlain : 0u];
 }
-__device__ __forceinline__ void cursor_put(uint64_t *p, bool cells, uint64_t v)
+// `live`: cursor_live, asked for beforehand by a caller that has other things to wait for.
+__device__ __forceinline__ uint32_t cursor_live(const uint64_t *p, bool cells)
+{
+  return cells ? cursor_newer(p[kCurStamp], p[kCurCell + kCurStamp]) : 0u;
+}
+__device__ __forceinline__ void cursor_put(uint64_t *p, bool cells, uint32_t live, uint64_t v)
 {
   if (cells) {
-    p[cursor_newer(p[kCurStamp], p[kCurCell + kCurStamp]) * kCurCell + kCurValue] = v;
+    p[live * kCurCell + kCurValue] = v;
     p[kCurPlain] = v;
   } else {
     p[0] = v;

@@ -523,7 +523,7 @@ static void launch_scatter(hipStream_t st, const ScatterArgs &sa, uint32_t grid,
   const bool lng = sa.pieces > 1;
   if (defer) {
     k_scatter<true, FUSED, true, true, ADV><<<grid, kBlock, 0, st>>>(sa);
-    k_udp_finish<FUSED><<<(sa.n_items + kBlock - 1) / kBlock, kBlock, 0, st>>>(sa);
+    k_udp_finish<FUSED><<<(sa.n_items + kBlock - 1) / kBlock, kBlock, 0, st>>>(sa, FinishPair{}, 0);
   } else if (full_csum && lng) k_scatter<true, FUSED, true, false, ADV><<<grid, kBlock, 0, st>>>(sa);
   else if (full_csum) k_scatter<true, FUSED, false, false, ADV><<<grid, kBlock, 0, st>>>(sa);
   else if (lng) k_scatter<false, FUSED, true, false, ADV><<<grid, kBlock, 0, st>>>(sa);
@@ -1562,12 +1562,9 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
     } else {
       k_shunt_any<false, false><<<total, kBlock, 0, st>>>(sh);
     }
-    if (h.full_csum && sh.s_long) k_udp_finish<true><<<(sh.s.n_items + kBlock - 1) / kBlock, kBlock, 0, st>>>(sh.s);
-    rc = prof_end(c);
-    if (rc != SG_OK) return rc;
+    FinishPair p;
+    uint32_t n = 0;
     if (!adv && cursors) {
-      FinishPair p;
-      uint32_t n = 0;
       for (int k = 0; k < 2; k++) {
         if (!h.cursor[k]) continue;
         p.h[n] = k == 0 ? finish_args(c->sc, h.cursor[0], g->fixed_req_size, g->app.arena_cap, g->n_req, g->counts, nullptr, 0, 0, false)
@@ -1575,8 +1572,12 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
         p.h[n++].clamp = h.self[k] ? 1u : 0u;  // as in the call of its own
       }
       if (n == 1) p.h[1] = p.h[0];
-      k_finish<<<n, kBlock, 0, st>>>(p);
     }
+    const bool two_phases = h.full_csum && sh.s_long;
+    if (two_phases) k_udp_finish<true><<<n + (sh.s.n_items + kBlock - 1) / kBlock, kBlock, 0, st>>>(sh.s, n ? p : FinishPair{}, n);
+    rc = prof_end(c);
+    if (rc != SG_OK) return rc;
+    if (n && !two_phases) k_finish<<<n, kBlock, 0, st>>>(p);
     return finish(c, async);
   }
   int rc = gather_impl(c, c->sc, c->stream, g);
