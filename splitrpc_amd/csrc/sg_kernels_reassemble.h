@@ -56,7 +56,7 @@ namespace {
 //   a group of lanes after the other goes
 //   to the table, records from a ring:
 //     insert / flag / scan / emit          23.2 / 5.5 / 4.9 / 8.4    30.1 / 9.7 / 4.7 / 13.0
-//   this form: insert / flag / emit        11.3 / 4.9 / 6.6          13.7 / 4.9 / 6.8
+//   this form: insert / flag / emit        11.5 / 4.9 / 6.3          14.0 / 4.9 / 6.5
 //   64 arrivals in one launch              8.6 -> 5.4, and 3.8 where the counts stay on the device
 // (a launch that does nothing shows as 2 to 4 us there).  Workgroups of 512 threads: 11.9 / 5.2 / 6.0
 // and 14.0 / 5.1 / 9.4; of 1024: 12.2 / 5.2 / 5.8 and 20.5 / 6.8 / 10.8.  The ring of free records
@@ -116,13 +116,16 @@ struct RaArgs {
   volatile uint32_t *status_flag;  // pinned host word: non-zero once any kernel refused something
 };
 
-// Entry j of a cell's record.  The first few lie apart, 64 bytes a cell: all that a request of a few
+// Entry j of a cell's record.  The first few lie apart, 32 bytes a cell: all that a request of a few
 // fragments has, where 65536 such requests spread over records of 8 KB each would have their entries
-// in gigabytes.
-constexpr uint32_t kRaHead = 8;
+// in gigabytes.  (Four bursts of 65536 arrivals, two fragments a request, filed, gathered and answered:
+// 407 us with records in one piece, 397 with eight entries apart, 395 with four; one of 220672, 431
+// fragments a request, 123.1 us with eight, 122.9 with four.)
+constexpr uint32_t kRaHead = 4;
 __device__ __forceinline__ unsigned long long *ra_entry(const RaArgs &a, uint32_t cell, uint32_t j)
 {
-  return j < kRaHead ? a.head + (size_t)cell * kRaHead + j : a.tab + (size_t)cell * SG_MAX_BI_SIZE + j;
+  const bool h = j < kRaHead;
+  return (h ? a.head : a.tab) + ((size_t)cell * (h ? kRaHead : SG_MAX_BI_SIZE) + j);
 }
 
 __device__ __forceinline__ uint32_t ra_n(const RaArgs &a)
@@ -538,21 +541,20 @@ __device__ __forceinline__ void ra_emit(const RaArgs &a, uint32_t cell, unsigned
   // requests of a few fragments are handed over by the completing lane itself, all such lanes
   // at once; the wavefront then walks the larger ones together, eight entries per lane asked for
   // before the first is stored
-  constexpr uint32_t kOwn = kRaHead, kAhead = 8;
+  constexpr uint32_t kOwn = 8, kAhead = 8;
   const uint32_t cnt = ra_done_cnt(done);
   const bool own = done && cnt <= kOwn;
   unsigned long long todo = __ballot(done && !own);
-  unsigned long long *t = a.head + (size_t)cell * kRaHead;
   unsigned long long e[kOwn], f[kAhead];
   if (own) {
 #pragma unroll
-    for (uint32_t j = 0; j < kOwn; j++) e[j] = j < cnt ? t[j] : 0ull;
+    for (uint32_t j = 0; j < kOwn; j++) e[j] = j < cnt ? *ra_entry(a, cell, j) : 0ull;
   }
   auto ask = [&](uint32_t c, uint32_t k, uint32_t j0) {
 #pragma unroll
     for (uint32_t q = 0; q < kAhead; q++) {
       const uint32_t j = j0 + q * kWave + lane;
-      f[q] = j < k ? *ra_entry(a, c, j) : 0ull;
+      f[q] = j < k ? *(q ? a.tab + (size_t)c * SG_MAX_BI_SIZE + j : ra_entry(a, c, j)) : 0ull;
     }
   };
   if (todo) {
@@ -569,7 +571,7 @@ __device__ __forceinline__ void ra_emit(const RaArgs &a, uint32_t cell, unsigned
       if (j < cnt) {
         a.frag_slot[first + j] = (uint32_t)e[j];
         a.frag_len[first + j] = (uint32_t)(e[j] >> 32);
-        t[j] = 0;  // a fresh request finds an empty record
+        *ra_entry(a, cell, j) = 0;  // a fresh request finds an empty record
       }
     }
     a.req_first[r] = first;
@@ -594,7 +596,7 @@ __device__ __forceinline__ void ra_emit(const RaArgs &a, uint32_t cell, unsigned
         if (j < k) {
           a.frag_slot[first + j] = (uint32_t)f[q];
           a.frag_len[first + j] = (uint32_t)(f[q] >> 32);
-          *ra_entry(a, c, j) = 0;
+          *(q ? a.tab + (size_t)c * SG_MAX_BI_SIZE + j : ra_entry(a, c, j)) = 0;
         }
       }
       if (j0 == 0 && lane == 0) {
