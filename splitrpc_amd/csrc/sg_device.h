@@ -337,11 +337,13 @@ __device__ __forceinline__ void piece_store16(Piece p, uint32_t off, u32x4 v) { 
 // 513 waiting to issue).  Through buffer descriptors, which drop the lanes that
 // have nothing to do, and with one branch for both steps' realignment it is 75
 // instructions from begin to end where masks and branches took 150.  One pass, us:
-//   512 requests of 602112 bytes, 4000 back   104.5 -> 103.5
-//   256 of 1.5 MB in 8800-byte fragments, the UDP checksum of 1 MB responses in software   225 -> 220.5
-//   32768 of all sizes, echoed                251 -> 241
-//   8192 of 3136 bytes, 40 back               15.1 -> 14.4
-//   16 of 602112 bytes, 4000 back             7.15 -> 6.9
+//   512 requests of 602112 bytes, 4000 back   104.2 -> 103.4
+//   256 of 1.5 MB in 8800-byte fragments, the UDP checksum of 1 MB responses in software   225 -> 220
+//   32768 of all sizes, echoed                255 -> 246
+//   8192 of 3136 bytes, 40 back               14.7 -> 14.3
+//   16 of 602112 bytes, 4000 back             7.15 -> 6.8
+// (the card warm, 0.1 s and more of one call after the other; the first milliseconds are 1 to 3 %
+// quicker, and not for every form alike).
 constexpr uint32_t kStep = 63 * 16;  // bytes a step stores
 constexpr uint32_t kRunMost = 1u << 30;  // bytes of the longest run: offsets stay below kNowhere
 struct RunState {
@@ -396,43 +398,39 @@ __device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict
 // parity of its DESTINATION ADDRESS (packet offsets and addresses have the
 // same parity: ring bases, slot sizes and header lengths are even).
 //
-// KEEP_ENDS: what goes into the run's first and last 128-byte line of the destination is stored
-// without the nontemporal hint.  A neighbouring wavefront writes the rest of those lines, a little
-// earlier or later, and with the hint the second level cache writes a line out before it is whole:
-// memory then takes a part of a line twice (24.4 instead of 22.2 write requests per wavefront of
-// 1400 bytes).  For runs that lie end to end, requests in an arena; a frame in a slot of its own has
-// no such neighbour.  220672 fragments of 1400 bytes: 128 us without, 103.5 with; everything without
-// the hint: 136 us.
+// KEEP_FIRST: what goes into the run's first 128-byte line of the destination is stored without the
+// nontemporal hint, before the rest.  A neighbouring wavefront writes the end of its run into that line,
+// a little earlier or later, and with the hint on both sides the second level cache writes the line out
+// before it is whole: memory then takes a part of a line twice (24.4 instead of 22.2 write requests per
+// wavefront of 1400 bytes).  For runs that lie end to end, requests in an arena; a frame in a slot of
+// its own has no such neighbour.  220672 fragments of 1400 bytes: 128 us without, 103.4 with; the last
+// line as well, or instead, 104.2; everything without the hint: 136 us.
 //
 // BROKEN: the destination is two pieces -- aligned chunks from number `brk` on, and the tail
 // bytes, land `jump` bytes further (a fragment that runs from one tensor into the next, where
 // the second tensor's share starts on a 16-byte boundary and the first one's share ends on a
 // chunk boundary of the run): one run instead of two.
-template <bool KEEP_ENDS, bool CSUM, bool BROKEN = false>
+template <bool KEEP_FIRST, bool CSUM, bool BROKEN = false>
 __device__ __forceinline__ uint32_t run_end(RunState &r, uint32_t lane, uint32_t brk = 0, int64_t jump = 0)
 {
-  static_assert(!(KEEP_ENDS && BROKEN), "one or the other");
+  static_assert(!(KEEP_FIRST && BROKEN), "one or the other");
   uint32_t acc = 0;
   const uint32_t first = BROKEN ? brk << 4 : r.body;  // bytes of the first destination piece
   const Piece out = piece_of(r.dst + r.head, first);
   const Piece out_b = BROKEN ? piece_of(r.dst + r.head + first + jump, r.body - first) : out;
   const uint32_t at = lane < 63 ? lane << 4 : kNowhere;
-  // offsets of the stores that go into whole lines: from .. from + whole (none for a run inside one line)
-  const uint32_t d0 = (uint32_t)(uintptr_t)r.dst + r.head, over = (d0 + r.body) & 127u;
-  const uint32_t from = (0u - d0) & 127u, whole = from + over <= r.body ? r.body - over - from : 0u;
-  auto put = [&](uint32_t base) {
+  const uint32_t line = (0u - ((uint32_t)(uintptr_t)r.dst + r.head)) & 127u;  // what is left of the first line
+  auto put = [&](uint32_t base, bool begin) {
     realign_pair(r.v0, r.v1, r.p);
     const uint32_t a0 = base + at, a1 = a0 + kStep;
-    if (KEEP_ENDS) {
-      const bool w0 = a0 - from < whole, w1 = a1 - from < whole;
-      piece_store16(out, w0 ? a0 : kNowhere, r.v0);
-      piece_store16(out, w1 ? a1 : kNowhere, r.v1);
-      piece_store16_kept(out, w0 ? kNowhere : a0, r.v0);
-      piece_store16_kept(out, w1 ? kNowhere : a1, r.v1);
+    if (KEEP_FIRST && begin) {
+      const bool shared = a0 < line;
+      piece_store16_kept(out, shared ? a0 : kNowhere, r.v0);
+      piece_store16(out, shared ? kNowhere : a0, r.v0);
     } else {
       piece_store16(out, a0, r.v0);
-      piece_store16(out, a1, r.v1);
     }
+    piece_store16(out, a1, r.v1);
     if (BROKEN) {
       // below the break these offsets wrap and lie beyond the second piece; opaque, so that no part
       // of them is left to the instruction's own offset field, behind the wrap
@@ -446,10 +444,10 @@ __device__ __forceinline__ uint32_t run_end(RunState &r, uint32_t lane, uint32_t
       acc += a1 < r.body ? words_sum(r.v1) : 0u;
     }
   };
-  put(0);
+  put(0, true);
   for (uint32_t base = 2 * kStep; __builtin_expect(base < r.body, 0); base += 2 * kStep) {
     run_load(r, base);
-    put(base);
+    put(base, false);
   }
   if (r.edge) {
     // head bytes sit on lanes 0..15, tail bytes (behind the last aligned chunk) on lanes 16..31
@@ -461,13 +459,13 @@ __device__ __forceinline__ uint32_t run_end(RunState &r, uint32_t lane, uint32_t
 }
 
 // Copy `len` bytes (0 < len <= kRunMost) src -> dst with one wavefront.
-template <bool KEEP_ENDS, bool CSUM>
+template <bool KEEP_FIRST, bool CSUM>
 __device__ __forceinline__ uint32_t copy_run(const uint8_t *__restrict__ src,
                                              uint8_t *__restrict__ dst, uint32_t len, uint32_t lane, bool keep)
 {
   RunState r;
   run_begin(r, src, dst, len, lane, keep);
-  return run_end<KEEP_ENDS, CSUM>(r, lane);
+  return run_end<KEEP_FIRST, CSUM>(r, lane);
 }
 
 // A LONG run (jumbo frames) is cut into sub-runs of kPieceChunks destination

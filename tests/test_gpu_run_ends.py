@@ -1,5 +1,5 @@
-"""Runs whose first and last 128-byte lines of the destination are stored apart
-from the whole lines between them: every place in a line a run can start at and
+"""Runs whose part of the destination's first 128-byte line is stored apart from
+the rest: every place in a line a run can start at and
 every place it can end at, lengths around lines, steps (1008 bytes) and pairs of
 steps, nothing written beside the runs."""
 import numpy as np
