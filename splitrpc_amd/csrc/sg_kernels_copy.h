@@ -1245,10 +1245,9 @@ __global__ __launch_bounds__(kBlock) void k_shunt(ShuntArgs a)
 
 // Every other shape, chosen by the workgroup.  ADV: the kernel takes both cursors from the context's
 // cells and advances them itself; else k_finish follows.  (Eight wavefronts per SIMD: left to itself
-// the compiler takes 104 scalar registers here, which is seven.  The price is 265 to 317 scalar values
-// kept in lanes of vector registers over its fourteen bodies, where each body's own kernel keeps none;
-// 131072 requests of 2048 bytes, 3072 back, take 275 us through here and 274 us as two calls on a
-// stream each.)
+// the compiler takes 104 scalar registers here, which is seven; 81 or more already are.  The price is
+// 94 to 147 scalar values kept in lanes of vector registers over its fourteen bodies.  131072 requests
+// of 2048 bytes, 3072 back: 270 us, 280 with up to 96 scalar registers and 27 such values.)
 template <bool FULL_CSUM, bool ADV>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_shunt_any(ShuntArgs)
 {
