@@ -38,6 +38,15 @@ __device__ __forceinline__ uint32_t load32_any(const uint8_t *p)
 // nontemporal hint on both sides keeps them from displacing each other in the
 // caches; measured on the 32-batch gather it is worth 8 % (stores alone 5 %,
 // loads alone -5 %), and a plain 16-byte-per-lane copy kernel gains the same.
+// Loads carry it whatever the size of the rings.  Without it what was read stays in the 256 MB
+// memory-side cache, which pays where nothing but a few passes' memory goes through that, and costs
+// more elsewhere.  One pass, us, with the hint / without: (a) between others over two or three rings,
+// (b) the payload written anew before it and nothing else between, (c) between others over 720 MB of
+// rings, (d) after other work over 600 MB, as a model's between two batches ((b), (d) a pass by itself):
+//   16 requests of 602112 bytes    (a) 6.8 / 5.8    (b) 9.0 / 8.7    (c) 7.2 / 7.6    (d) 10.6 / 12.1
+//   64 of 602112                   (a) 16.6 / 14.5  (b) 18.2 / 17.2  (c) 16.9 / 17.8  (d) 21.8 / 27.0
+//   8192 of 3136                   (a) 14.1 / 12.0  (b) 15.7 / 14.7  (c) 14.3 / 14.2  (d) 18.7 / 22.6
+//   8 of 1.5 MB, jumbo frames      (a) 14.7 / 13.1  (b) 17.5 / 15.6  (c) 14.9 / 15.6  (d) 18.4 / 21.6
 __device__ __forceinline__ void store16_aligned(uint8_t *p, u32x4 v)
 {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(p));
@@ -47,8 +56,6 @@ __device__ __forceinline__ u32x4 load16_aligned(const uint8_t *p)
 {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
 }
-
-__device__ __forceinline__ u32x4 load16_aligned_kept(const uint8_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
 
 typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
 
@@ -307,7 +314,6 @@ __device__ __forceinline__ Piece piece_of(const uint8_t *p, uint32_t bytes)
 }
 constexpr int kNontemporal = 2;
 constexpr uint32_t kNowhere = 0x80000000u;  // an offset beyond every piece
-__device__ __forceinline__ u32x4 piece_load16_kept(Piece p, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(p, (int)off, 0, 0); }
 __device__ __forceinline__ u32x4 piece_load16(Piece p, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(p, (int)off, 0, kNontemporal); }
 __device__ __forceinline__ void piece_store16_kept(Piece p, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, p, (int)off, 0, 0); }
 __device__ __forceinline__ void piece_store16(Piece p, uint32_t off, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, p, (int)off, 0, kNontemporal); }
@@ -359,25 +365,18 @@ struct RunState {
   uint32_t eoff;   // this lane's edge byte, if any
   uint32_t eb;
   bool edge;
-  bool keep;       // loads without the nontemporal hint
   u32x4 v0, v1;
 };
 
 __device__ __forceinline__ void run_load(RunState &r, uint32_t base)
 {
-  if (r.keep) {
-    r.v0 = piece_load16_kept(r.in, r.at + base);
-    r.v1 = piece_load16_kept(r.in, r.at + base + kStep);
-  } else {
-    r.v0 = piece_load16(r.in, r.at + base);
-    r.v1 = piece_load16(r.in, r.at + base + kStep);
-  }
+  r.v0 = piece_load16(r.in, r.at + base);
+  r.v1 = piece_load16(r.in, r.at + base + kStep);
 }
 
 __device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict__ src,
-                                          uint8_t *__restrict__ dst, uint32_t len, uint32_t lane, bool keep)
+                                          uint8_t *__restrict__ dst, uint32_t len, uint32_t lane)
 {
-  r.keep = keep;
   uint32_t head = (uint32_t)(-(uintptr_t)dst) & 15u;
   head = head < len ? head : len;
   const uint32_t rest = len - head, tail = rest & 15u;
@@ -464,10 +463,10 @@ __device__ __forceinline__ uint32_t run_end(RunState &r, uint32_t lane, uint32_t
 // Copy `len` bytes (0 < len <= kRunMost) src -> dst with one wavefront.
 template <bool KEEP_FIRST, bool CSUM>
 __device__ __forceinline__ uint32_t copy_run(const uint8_t *__restrict__ src,
-                                             uint8_t *__restrict__ dst, uint32_t len, uint32_t lane, bool keep)
+                                             uint8_t *__restrict__ dst, uint32_t len, uint32_t lane)
 {
   RunState r;
-  run_begin(r, src, dst, len, lane, keep);
+  run_begin(r, src, dst, len, lane);
   return run_end<KEEP_FIRST, CSUM>(r, lane);
 }
 
@@ -503,7 +502,7 @@ __device__ __forceinline__ void sub_run(const uint8_t *dst, uint32_t len, uint32
 // Copy a whole long run with one wavefront, DEPTH sub-runs in flight at a time.
 template <bool CSUM, int DEPTH>
 __device__ __forceinline__ uint32_t copy_long_run(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst,
-                                                  uint32_t len, uint32_t lane, bool keep)
+                                                  uint32_t len, uint32_t lane)
 {
   uint32_t acc = 0;
   for (uint32_t base = 0;; base += DEPTH) {
@@ -513,7 +512,7 @@ __device__ __forceinline__ uint32_t copy_long_run(const uint8_t *__restrict__ sr
     for (int k = 0; k < DEPTH; k++) {
       uint32_t o;
       sub_run(dst, len, base + k, &o, &n[k]);
-      if (n[k]) run_begin(r[k], src + o, dst + o, n[k], lane, keep);
+      if (n[k]) run_begin(r[k], src + o, dst + o, n[k], lane);
     }
 #pragma unroll
     for (int k = 0; k < DEPTH; k++)
@@ -717,7 +716,7 @@ struct GroupRun {
 
 template <int L>
 __device__ __forceinline__ void group_run_begin(GroupRun<L> &r, const uint8_t *src, uint8_t *dst, uint32_t len,
-                                                uint32_t gl, bool keep)
+                                                uint32_t gl)
 {
   uint32_t head = (uint32_t)(-(uintptr_t)dst) & 15u;
   head = head < len ? head : len;
@@ -741,13 +740,9 @@ __device__ __forceinline__ void group_run_begin(GroupRun<L> &r, const uint8_t *s
   r.lim = r.p ? body : body - 1;  // body == 0: lim wraps, guarded below
   r.v0 = (u32x4){0, 0, 0, 0};
   r.v1 = (u32x4){0, 0, 0, 0};
-  const bool l0 = body && gl <= r.lim, l1 = body && (L - 1) + gl <= r.lim;
-  if (keep) {
-    if (l0) r.v0 = load16_aligned_kept(r.sa + ((size_t)gl << 4));
-    if (l1) r.v1 = load16_aligned_kept(r.sa + ((size_t)((L - 1) + gl) << 4));
-  } else {
-    if (l0) r.v0 = load16_aligned(r.sa + ((size_t)gl << 4));
-    if (l1) r.v1 = load16_aligned(r.sa + ((size_t)((L - 1) + gl) << 4));
+  if (body) {
+    if (gl <= r.lim) r.v0 = load16_aligned(r.sa + ((size_t)gl << 4));
+    if ((L - 1) + gl <= r.lim) r.v1 = load16_aligned(r.sa + ((size_t)((L - 1) + gl) << 4));
   }
 }
 

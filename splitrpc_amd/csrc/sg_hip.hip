@@ -223,23 +223,6 @@ void geometry(uint64_t n_waves, bool want_remap, uint32_t *grid, uint32_t *remap
   }
 }
 
-// Whether a direction's loads go without the nontemporal hint.  With it what is read is fetched from
-// memory and leaves no copy in the 256 MB cache in front of it; without, a ring and application
-// memory that fit there together (half of it: the other direction has its own) stay, and the calls
-// of a server that goes round in them find there what the last ones left.  One pass of a step
-// among others, us, with the hint -> without, warm (two rings in turns) and cold (rings of 700 MB in
-// all, in turns): 16 requests of 602112 bytes 7.3 -> 6.3, 7.5 -> 7.1; 64 of them (95 MB) 17.0 ->
-// 15.0, 17.9 -> 18.4; 8192 of 3136 (76 MB) 14.6 -> 12.8, 15.0 -> 15.7; 4096 of 2048 13.2 -> 11.2,
-// 13.5 -> 13.4.  Beyond: 256 of 602112 (380 MB) 55.5 -> 60, 131072 of 2048 268 -> 280 -- what streams
-// through only displaces lines that are waiting for the rest of their bytes.
-constexpr uint64_t kKeptMost = 128ull << 20;
-bool reads_kept(const sg_ring_desc &ring, const sg_app_desc &app, uint32_t n_req)
-{
-  uint64_t bytes = (uint64_t)ring.n_slots * ring.slot_size + (app.n_tensors ? 0 : app.arena_cap);
-  for (uint32_t t = 0; t < app.n_tensors; t++) bytes += app.tensor_size[t] * n_req;
-  return bytes <= kKeptMost;
-}
-
 int prof_begin(sg_hip_ctx *c, int which)
 {
   if (!c || !c->profiling) return SG_OK;
@@ -1097,8 +1080,7 @@ static int gather_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const s
     geometry(waves, !(a->flags & SG_F_NO_XCD_REMAP), &grid, &remap);
     const bool self_advance = self_advancing(sc, packed, a->slot_state, waves, a->flags);
     ga.cursor = const_cast<uint64_t *>(plain_cursor(sc, 0));
-    const bool keep = reads_kept(a->ring, a->app, a->n_req);
-    ga.opts = (remap ? kOptRemap : 0u) | (keep ? kOptKeep : 0u) | (app.mirrored ? kOptMirrored : 0u) |
+    ga.opts = (remap ? kOptRemap : 0u) | (app.mirrored ? kOptMirrored : 0u) |
               (app.n_tensors > 1 ? kOptMultiTensor : 0u) | (small_last ? kOptSmallLast : 0u) |
               ((((uintptr_t)a->ring.base | a->ring.slot_size) & 15u) ? 0u : kOptHdrChunk);
     if (half) {
@@ -1120,7 +1102,7 @@ static int gather_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const s
     if (zero_words) k_zero_words<<<1, kBlock, 0, st>>>(zero_words, 2);
     rc = prof_begin(c, 1);
     if (rc != SG_OK) return rc;
-    if (self_advance || (keep && !packed)) launch_gather_rule<true>(st, ga, grid, small_all, small_last, n_items);
+    if (self_advance) launch_gather_rule<true>(st, ga, grid, small_all, small_last, n_items);
     else launch_gather_rule<false>(st, ga, grid, small_all, small_last, n_items);
     rc = prof_end(c);
     if (rc != SG_OK) return rc;
@@ -1189,11 +1171,8 @@ static int gather_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const s
     geometry((uint64_t)(a->n_frags ? a->n_frags : 1u) * ga.pieces, !(a->flags & SG_F_NO_XCD_REMAP), &grid, &ga.remap);
     rc = prof_begin(c, 1);
     if (rc != SG_OK) return rc;
-    const bool keep = reads_kept(a->ring, a->app, a->n_req);
-    if (ga.pieces > 1 && keep) k_gather<true, true><<<grid, kBlock, 0, st>>>(ga);
-    else if (ga.pieces > 1) k_gather<true, false><<<grid, kBlock, 0, st>>>(ga);
-    else if (keep) k_gather<false, true><<<grid, kBlock, 0, st>>>(ga);
-    else k_gather<false, false><<<grid, kBlock, 0, st>>>(ga);
+    if (ga.pieces > 1) k_gather<true><<<grid, kBlock, 0, st>>>(ga);
+    else k_gather<false><<<grid, kBlock, 0, st>>>(ga);
     rc = prof_end(c);
     if (rc != SG_OK) return rc;
   }
@@ -1265,7 +1244,6 @@ static int scatter_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const 
     sa.n_items = n_items;
     sa.n_req = a->n_req;
     sa.counts = a->counts;
-    sa.keep = reads_kept(a->tx, a->app, a->n_req);
     sa.hdr_src_req = a->hdr_templates ? nullptr : a->hdr_src_req;
     sa.status = sc.status;
     sa.status_flag = sc.flag;
@@ -1324,9 +1302,8 @@ static int scatter_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const 
     if (self_advance) sa.rule.call_seq = ++*sc.call_seq;
     rc = prof_begin(c, 2);
     if (rc != SG_OK) return rc;
-    const bool adv_kernel = self_advance || (sa.keep && !packed);  // (tensors: no cursor to advance)
     if (small_all) {
-      launch_scatter_small(st, sa, small_all, n_items, full_csum, adv_kernel);
+      launch_scatter_small(st, sa, small_all, n_items, full_csum, self_advance);
     } else {
       if (small_last) sa.rule.per_launch = (uint32_t)per - 1;
       magic_div(sa.rule.per_launch, &sa.rule.lmul, &sa.rule.lshift);
@@ -1340,8 +1317,8 @@ static int scatter_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const 
       // than the overlap gains, 180 against 172 us on 131072 responses of 1400 + 1400 + 272 bytes)
       if (small_last) {
         launch_scatter<true>(st, sa, grid, full_csum, defer);
-        launch_scatter_small(st, sa, small_last, a->n_req, full_csum, adv_kernel);
-      } else if (adv_kernel) {
+        launch_scatter_small(st, sa, small_last, a->n_req, full_csum, self_advance);
+      } else if (self_advance) {
         launch_scatter<true, true>(st, sa, grid, full_csum, defer);
       } else {
         launch_scatter<true>(st, sa, grid, full_csum, defer);
@@ -1444,8 +1421,7 @@ static int scatter_impl(sg_hip_ctx *c, const Scratch &sc, hipStream_t st, const 
              !(a->flags & SG_F_NO_XCD_REMAP), &grid, &sa.remap);
     rc = prof_begin(c, 2);
     if (rc != SG_OK) return rc;
-    if (reads_kept(a->tx, a->app, a->n_req)) launch_scatter<false, true>(st, sa, grid, full_csum, defer);
-    else launch_scatter<false>(st, sa, grid, full_csum, defer);
+    launch_scatter<false>(st, sa, grid, full_csum, defer);
     rc = prof_end(c);
     if (rc != SG_OK) return rc;
   }
@@ -1528,9 +1504,8 @@ int sg_hip_shunt_batch(sg_hip_ctx *c, const sg_gather_args *g, const sg_scatter_
     // the kernel advances the cursors itself where each half's own would; a workgroup for either
     // direction behind it does otherwise
     const bool cursors = h.cursor[0] || h.cursor[1];
-    const bool adv = cursors ? (!h.cursor[0] || h.self[0]) && (!h.cursor[1] || h.self[1])
-                             : (sh.g.opts & kOptKeep) || sh.s.keep;  // nothing to advance: the instance that can keep
-    if (adv && cursors) {
+    const bool adv = cursors && (!h.cursor[0] || h.self[0]) && (!h.cursor[1] || h.self[1]);
+    if (adv) {
       sh.g.call_seq = ++c->call_seq;
       sh.s.rule.call_seq = ++c->call_seq;
     }

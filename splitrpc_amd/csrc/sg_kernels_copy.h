@@ -207,7 +207,7 @@ __device__ __forceinline__ uint32_t rule_desc(const RuleArgs &g, const AppDev &a
 // SG_MAX_TENSORS pieces.
 template <bool TO_APP, bool CSUM>
 __device__ __forceinline__ uint32_t move_run(const AppDev &app, uint64_t req_off, uint32_t r,
-                                             uint32_t off, uint8_t *pkt, uint32_t len, uint32_t lane, bool keep)
+                                             uint32_t off, uint8_t *pkt, uint32_t len, uint32_t lane)
 {
   uint32_t acc = 0;
   const bool packed = app.n_tensors == 0;
@@ -248,7 +248,7 @@ __device__ __forceinline__ uint32_t move_run(const AppDev &app, uint64_t req_off
     }
     while (n) {
       const uint32_t k = n < kRunMost ? n : kRunMost;
-      acc += TO_APP ? copy_run<true, CSUM>(pkt + done, p, k, lane, keep) : copy_run<false, CSUM>(p, pkt + done, k, lane, keep);
+      acc += TO_APP ? copy_run<true, CSUM>(pkt + done, p, k, lane) : copy_run<false, CSUM>(p, pkt + done, k, lane);
       done += k;
       p += k;
       n -= k;
@@ -330,7 +330,7 @@ __device__ __forceinline__ bool two_tensor_target(const AppDev &app, uint32_t r,
 // `pieces` consecutive wavefronts.  (Several fragments per wavefront were
 // measured too: two cost 2 %, three 13 % on 1400-byte fragments -- the number
 // of wavefronts in flight is what covers the HBM latency.)
-template <bool LONG, bool KEEP>
+template <bool LONG>
 __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs a)
 {
   const u32x4 *desc = a.desc;
@@ -363,12 +363,12 @@ __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs a)
     if (LONG) {
       uint32_t o, n;
       sub_run(to, d[1], piece, &o, &n);
-      if (n) copy_run<true, false>(pkt + o, to + o, n, lane, KEEP);
+      if (n) copy_run<true, false>(pkt + o, to + o, n, lane);
     } else {
-      copy_run<true, false>(pkt, to, d[1], lane, KEEP);
+      copy_run<true, false>(pkt, to, d[1], lane);
     }
   } else if (piece == 0) {
-    move_run<true, false>(a.app, ro, d[3], d[2], pkt, d[1], lane, KEEP);
+    move_run<true, false>(a.app, ro, d[3], d[2], pkt, d[1], lane);
   }
 }
 
@@ -410,7 +410,7 @@ struct alignas(64) GatherRuleArgs {
   uint32_t hl;
   uint32_t n_slots;
   uint32_t pieces;            // wavefronts per fragment
-  uint32_t opts;  // kOptRemap | kOptMirrored | kOptKeep | kOptMultiTensor | kOptHdrChunk
+  uint32_t opts;  // kOptRemap | kOptMirrored | kOptMultiTensor | kOptHdrChunk
   // warm
   uint32_t n_req;
   const uint32_t *frag_len;
@@ -432,7 +432,6 @@ constexpr uint32_t kOptRemap = 1u, kOptMirrored = 2u, kOptMultiTensor = 8u;
 // slots start at 16-byte aligned addresses: the header's length field can be read as part of
 // the aligned chunk at byte 48 (a ring only has to start at an even address)
 constexpr uint32_t kOptHdrChunk = 16u;
-constexpr uint32_t kOptKeep = 4u;  // ADV kernels: loads without the nontemporal hint
 constexpr uint32_t kOptSmallLast = 32u;  // the last fragment of every request is left to k_gather_small
 
 template <int L, bool ADV>
@@ -442,9 +441,7 @@ __device__ __forceinline__ void gather_small_wave(const GatherRuleArgs &a, uint3
 // request is short -- the wavefronts behind those of the full fragments then move
 // 64 / SMALL remainder fragments each, in the same launch (a launch of their own
 // would be all latency: tens of megabytes at most); 0: no such wavefronts.
-// ADV: the kernel takes the cursor from a context's cells and advances it itself (no k_finish follows),
-// and has the loads without the nontemporal hint for the calls that want them (kOptKeep): chosen at run
-// time in every instance, they cost 131072 requests of 2048 bytes 268 -> 275 us.
+// ADV: the kernel takes the cursor from a context's cells and advances it itself (no k_finish follows).
 // `block`: the workgroup's number among those of this work; `kernarg_base`: where `a` lies in the
 // running kernel's argument block (the plan is read through the argument pointer).
 template <bool LONG, int SMALL, bool ADV>
@@ -581,14 +578,13 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
   // consumed only after the payload loads are under way.  (Every shape of a run is begun and ended in
   // a branch of its own: begun in one place and ended in another, its state goes through registers
   // and lanes the branches in between agree on.)
-  const bool keep = ADV && (opts & kOptKeep);
   auto under_way = [&] { asm volatile("" ::"v"(hc), "v"(hv)); };
   if (plain) {
     uint32_t sub_off = 0, sub_len = len;
     if (LONG) sub_run(to, len, piece, &sub_off, &sub_len);
     if (sub_len) {
       RunState rs;
-      run_begin(rs, pkt + hl + sub_off, to + sub_off, sub_len, lane, keep);
+      run_begin(rs, pkt + hl + sub_off, to + sub_off, sub_len, lane);
       under_way();
       run_end<true, false>(rs, lane);
     }
@@ -602,18 +598,18 @@ __device__ __forceinline__ void gather_rule_body(const GatherRuleArgs &a, uint32
     const uint32_t head_a = (uint32_t)(-(uintptr_t)to_a) & 15u;
     if (two && ((uintptr_t)to_b & 15u) == 0 && len_a >= head_a && ((len_a - head_a) & 15u) == 0) {
       RunState rs;
-      run_begin(rs, pkt + hl, to_a, len, lane, keep);
+      run_begin(rs, pkt + hl, to_a, len, lane);
       under_way();
       run_end<false, false, true>(rs, lane, (len_a - head_a) >> 4, (int64_t)(to_b - (to_a + len_a)));
     } else if (two) {
       RunState rs, rb;
-      run_begin(rs, pkt + hl, to_a, len_a, lane, keep);
-      run_begin(rb, pkt + hl + len_a, to_b, len - len_a, lane, keep);
+      run_begin(rs, pkt + hl, to_a, len_a, lane);
+      run_begin(rb, pkt + hl + len_a, to_b, len - len_a, lane);
       under_way();
       run_end<true, false>(rs, lane);
       run_end<true, false>(rb, lane);
     } else {
-      move_run<true, false>(a.app, ro, r, off, pkt + hl, len, lane, keep);
+      move_run<true, false>(a.app, ro, r, off, pkt + hl, len, lane);
     }
   }
   if (piece == 0) {
@@ -724,7 +720,7 @@ __device__ __forceinline__ void gather_small_wave(const GatherRuleArgs &a, uint3
     }
   }
   GroupRun<L> run;
-  group_run_begin<L>(run, pkt + hl, to, plain ? len : 0u, gl, ADV && (a.opts & kOptKeep));
+  group_run_begin<L>(run, pkt + hl, to, plain ? len : 0u, gl);
   group_run_end<L, false>(run, gl);
   if (live && len && !plain) {
     // across an arena end or a tensor boundary: byte by byte
@@ -767,7 +763,7 @@ struct alignas(64) ScatterArgs {
   uint64_t *cursor;             // descriptor path, packed: wavefront 0 commits *next_cursor
   const uint64_t *next_cursor;
   uint32_t cursor_cells;        // the cursor is a context's pair of cells, not a plain word
-  uint32_t keep;                // ADV kernels: loads without the nontemporal hint
+  uint32_t cursor_pad;
   const uint32_t *hdr_src_req;  // one header source per request instead of hdr_src_slot per frame
   const uint32_t *counts;       // device-resident request count, or nullptr
   // full UDP checksum of long frames in two phases: every sub-run's wavefront leaves the sum of
@@ -819,8 +815,7 @@ constexpr uint32_t kPartStride = 8;  // words of csum_part per frame: up to 7 su
 // DEFER (long frames with the full UDP checksum): the frame's sub-runs go to
 // several wavefronts all the same, each leaving the sum of its bytes behind,
 // and k_udp_finish writes the checksum field afterwards.
-// ADV: as in gather_rule_body.  Not fused there is no cursor to derive offsets from: the instance whose
-// loads go without the hint.
+// ADV (fused only): the kernel takes the cursor from a context's cells and advances it itself.
 template <bool FULL_CSUM, bool FUSED, bool LONG, bool DEFER, bool ADV>
 __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t block, size_t kernarg_base)
 {
@@ -834,7 +829,6 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
   uint8_t *tx = a.tx;
   const uint32_t rx_slot_size = a.rx_slot_size, rx_n_slots = a.rx_n_slots, tx_slot_size = a.tx_slot_size;
   const uint32_t hl = a.hl, remap = a.remap, n_pieces = a.pieces;
-  const bool keep = ADV && (!FUSED || a.keep);
   const uint32_t *status = a.status;
   const uint32_t *counts = a.counts, *hdr_src_req = a.hdr_src_req;
   uint32_t n_items = a.n_items, n_req = a.n_req;
@@ -952,7 +946,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
     if (d[1] && scatter_source<FUSED>(a, ro, r, item - f0, d[2], d[1], &from, kernarg_base)) {
       uint32_t o, n;
       sub_run(slot + hl, d[1], piece, &o, &n);
-      if (n) part = copy_run<false, DEFER>(from + o, slot + hl + o, n, lane, keep);
+      if (n) part = copy_run<false, DEFER>(from + o, slot + hl + o, n, lane);
     }
     if (DEFER) {
       part = wave_sum_uniform(part);
@@ -974,7 +968,7 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
   };
   if (plain && WHOLE_LONG) {
     fields();
-    acc = copy_long_run<FULL_CSUM, 2>(from, slot + hl, d[1], lane, keep);
+    acc = copy_long_run<FULL_CSUM, 2>(from, slot + hl, d[1], lane);
   } else if (plain) {
     uint32_t first_len = d[1];
     if (SPLIT) {
@@ -982,12 +976,12 @@ __device__ __forceinline__ void scatter_body(const ScatterArgs &a, uint32_t bloc
       sub_run(slot + hl, d[1], 0, &o, &first_len);
     }
     RunState rs;
-    run_begin(rs, from, slot + hl, first_len, lane, keep);
+    run_begin(rs, from, slot + hl, first_len, lane);
     fields();
     acc = run_end<false, FULL_CSUM>(rs, lane);
   } else {
     fields();
-    if (d[1]) acc = move_run<false, FULL_CSUM>(a.app, ro, r, d[2], slot + hl, d[1], lane, keep);
+    if (d[1]) acc = move_run<false, FULL_CSUM>(a.app, ro, r, d[2], slot + hl, d[1], lane);
   }
   // the header's own share of the UDP sum rides with the payload's
   if (FULL_CSUM) acc += hdrw_l4_share(hb, lane, hl);
@@ -1139,7 +1133,7 @@ __device__ __forceinline__ void scatter_small_wave(const ScatterArgs &a, uint32_
   }
   GroupRun<L> run;
   if (early)
-    group_run_begin<L>(run, from, reinterpret_cast<uint8_t *>(((uintptr_t)a.tx + hl) & 15u), plain ? len : 0u, gl, ADV && a.keep);
+    group_run_begin<L>(run, from, reinterpret_cast<uint8_t *>(((uintptr_t)a.tx + hl) & 15u), plain ? len : 0u, gl);
   if (tslot >= a.rule.n_slots) bad |= kStBadSlot;
   if (i == 0 && first_r != item) bad |= kStBadTable;
   if (hs >= a.rx_n_slots) bad |= kStBadSlot;
@@ -1175,7 +1169,7 @@ __device__ __forceinline__ void scatter_small_wave(const ScatterArgs &a, uint32_
     group_run_rebase<L>(run, slot + hl);
     if (!plain) group_run_cancel<L>(run);  // a frame the tables have just ruled out
   } else {
-    group_run_begin<L>(run, from, slot + hl, plain ? len : 0u, gl, ADV && a.keep);
+    group_run_begin<L>(run, from, slot + hl, plain ? len : 0u, gl);
   }
   uint32_t acc = group_run_end<L, FULL_CSUM>(run, gl);
   if (live && len != 0 && !plain) {
@@ -1324,7 +1318,7 @@ struct Run {
 
 __device__ __forceinline__ void copy_one_run(const Run &r, uint32_t lane)
 {
-  copy_run<true, false>(reinterpret_cast<const uint8_t *>(r.src), reinterpret_cast<uint8_t *>(r.dst), (uint32_t)r.len, lane, false);
+  copy_run<true, false>(reinterpret_cast<const uint8_t *>(r.src), reinterpret_cast<uint8_t *>(r.dst), (uint32_t)r.len, lane);
 }
 
 __global__ __launch_bounds__(kBlock) void k_copy_runs(const Run *runs, uint32_t n, DoneArgs done)

@@ -1,6 +1,5 @@
-"""Loads with and without the nontemporal hint: which a call takes goes by the
-size of its ring and application memory (128 MB per direction).  The same small
-batch in a ring of its own size and at the head of a ring beyond the limit, by
+"""The size of a ring changes nothing in what a call moves: the same small batch
+in a ring of its own size and at the head of a ring of more than 128 MB, by
 every route -- separate calls and one launch, declared rule and descriptor pass,
 arena and tensors, short, full and long fragments -- against the oracle."""
 import numpy as np
@@ -23,7 +22,7 @@ BATCHES = {
 }
 
 
-@pytest.mark.parametrize("beyond", [False, True], ids=["kept", "streamed"])
+@pytest.mark.parametrize("beyond", [False, True], ids=["own-size", "beyond-128MB"])
 @pytest.mark.parametrize("route", ["shunt", "rule", "scan"])
 @pytest.mark.parametrize("name", list(BATCHES))
 def test_same_bytes_whatever_the_ring(name, route, beyond):
