@@ -32,25 +32,25 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes the copy kernels of one call move, from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of
 # this file (--calib-copy --steps 40 --warmup 5), each counter scaled by what it reads for a plain
 # 512 MiB device copy in the same run (FETCH_SIZE x 2.000 KiB, WRITE_SIZE x 1.000 KiB).  Keyed by
-# (workload, batches per launch, kernel family); the default call: 340.2 MB read + 309.6 MB written.
+# (workload, batches per launch, kernel family); the default call: 340.2 MB read + 309.5 MB written.
 # bert's scatter is both of its kernels (full frames + short remainder frames), jumbo's the copy
 # phase without the 1.9 MB of the checksum-finishing kernel.
 MEASURED_TRAFFIC = {
-    (2, 32, "k_gather"): 649.8e6, (2, 32, "k_scatter"): 4.7e6,
+    (2, 32, "k_gather"): 649.7e6, (2, 32, "k_scatter"): 4.7e6,
     (1, 2048, "k_gather"): 447.3e6, (1, 2048, "k_scatter"): 22.5e6,
-    (3, 512, "k_gather"): 579.5e6, (3, 512, "k_scatter"): 932.3e6,
-    (4, 8, "k_gather"): 657.0e6, (4, 8, "k_scatter"): 675.2e6,
-    (5, 4, "k_gather"): 815.5e6, (5, 4, "k_scatter"): 547.6e6,
+    (3, 512, "k_gather"): 579.4e6, (3, 512, "k_scatter"): 931.7e6,
+    (4, 8, "k_gather"): 656.8e6, (4, 8, "k_scatter"): 675.2e6,
+    (5, 4, "k_gather"): 816.4e6, (5, 4, "k_scatter"): 547.9e6,
 }
 # the same for the reference's own 64-byte header (bench.py --ref64)
-MEASURED_TRAFFIC_REF64 = {(2, 32, "k_gather"): 651.6e6, (2, 32, "k_scatter"): 4.8e6}
+MEASURED_TRAFFIC_REF64 = {(2, 32, "k_gather"): 651.5e6, (2, 32, "k_scatter"): 4.8e6}
 # The kernel sources those counter runs were made with (SHA-256).  A change to either file may change
 # what the kernels move: `roofline.traffic` is then reported as null until the two counter passes have
 # been run again and the figures above and these digests brought up to date (a CPU test holds them
 # against the tree).
 TRAFFIC_MEASURED_WITH = {
     "splitrpc_amd/csrc/sg_kernels_copy.h": "e9248431ca11ad233401142bb74771922beb474e47b6c021823c5e6be3ac3da6",
-    "splitrpc_amd/csrc/sg_device.h": "136356c0707dda81342bcc8bde4aabf053492f55bc79a2d8e62c41c0ae98a34c",
+    "splitrpc_amd/csrc/sg_device.h": "57913ac1fef68c7716864669a39a585ce5ff07091214fc3afc41884d05d7af78",
 }
 
 

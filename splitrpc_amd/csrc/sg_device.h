@@ -336,23 +336,25 @@ __device__ __forceinline__ void piece_store16(Piece p, uint32_t off, u32x4 v) { 
 // walks the rest.  A wavefront that begins several runs before ending the first
 // keeps that many runs' loads in flight.  (The edge bytes are asked for first:
 // behind the hinted loads their line, which those do not keep, comes from memory
-// a second time, and the edge stores are late for the lines they complete.  Lanes
-// that have no edge byte ask beyond the piece: with an address inside it, unused,
-// a pass over 131072 requests of 2048 bytes took 275.7 us, 273.0 without; 512 of
-// 602112 bytes filed, gathered and answered, 64-byte headers, 124.0 and 122.7.)
+// a second time, and the edge stores are late for the lines they complete.  Only
+// the lanes that have one ask, under a mask: with every lane asking, inside the
+// piece, 131072 requests of 2048 bytes took 275.5 us a pass instead of 269.8; the
+// others beyond the piece, 272; 512 of 602112 bytes filed, gathered and answered,
+// 64-byte headers, 124.0, 122.4 and 122.7.)
 //
 // What bounds it: memory, and half of a wavefront's life instructions (resnet-sized
 // fragments, per wavefront: 425 instructions, 414 of 1961 quad cycles issuing and
 // 513 waiting to issue).  Through buffer descriptors, which drop the lanes that
 // have nothing to do, and with one branch for both steps' realignment it is 75
-// instructions from begin to end where masks and branches took 150.  One pass, us:
-//   512 requests of 602112 bytes, 4000 back   104.2 -> 103.4
-//   256 of 1.5 MB in 8800-byte fragments, the UDP checksum of 1 MB responses in software   225 -> 220
-//   32768 of all sizes, echoed                255 -> 246
-//   8192 of 3136 bytes, 40 back               14.7 -> 14.3
-//   16 of 602112 bytes, 4000 back             7.15 -> 6.8
-// (the card warm, 0.1 s and more of one call after the other; the first milliseconds are 1 to 3 %
-// quicker, and not for every form alike).
+// instructions from begin to end where masks and branches took 150.  One pass, us,
+// with masks and branches and now, each in processes of its own, the card warm
+// (0.1 s and more of one call after the other):
+//   512 requests of 602112 bytes, 4000 back   104.2 -> 102.3
+//   131072 of 2048 bytes, 3072 back           275.5 -> 270.5
+//   256 of 1.5 MB in 8800-byte fragments, the UDP checksum of 1 MB responses in software   224.4 -> 220.5
+//   32768 of all sizes, echoed                256.4 -> 244.7
+//   8192 of 3136 bytes, 40 back               14.63 -> 14.05
+//   16 of 602112 bytes, 4000 back             7.16 -> 6.78
 constexpr uint32_t kStep = 63 * 16;  // bytes a step stores
 constexpr uint32_t kRunMost = 1u << 30;  // bytes of the longest run: offsets stay below kNowhere
 struct RunState {
@@ -391,7 +393,8 @@ __device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict
   const uint32_t k = second ? lane - 16 : lane;
   r.edge = k < (second ? tail : head);
   r.eoff = k + (second ? head + r.body : 0u);
-  r.eb = __builtin_amdgcn_raw_buffer_load_b8(r.in, (int)(r.edge ? s0 + r.eoff : kNowhere), 0, 0);
+  r.eb = 0;
+  if (r.edge) r.eb = src[r.eoff];
   run_load(r, 0);
 }
 
@@ -405,8 +408,8 @@ __device__ __forceinline__ void run_begin(RunState &r, const uint8_t *__restrict
 // a little earlier or later, and with the hint on both sides the second level cache writes the line out
 // before it is whole: memory then takes a part of a line twice (24.4 instead of 22.2 write requests per
 // wavefront of 1400 bytes).  For runs that lie end to end, requests in an arena; a frame in a slot of
-// its own has no such neighbour.  220672 fragments of 1400 bytes: 128 us without, 103.4 with; the last
-// line as well, or instead, 104.2; everything without the hint: 136 us.
+// its own has no such neighbour.  220672 fragments of 1400 bytes: 113.6 us without, 102.4 with; behind
+// 64-byte headers, filed first, 133.8 and 122.6; 8192 requests of 3136 bytes 14.55 and 13.95.
 //
 // BROKEN: the destination is two pieces -- aligned chunks from number `brk` on, and the tail
 // bytes, land `jump` bytes further (a fragment that runs from one tensor into the next, where
