@@ -335,7 +335,12 @@ int sg_hip_sync(sg_hip_ctx *ctx);
  * Replace sg_on_gpu(CopyCtx*, p2p_sk_buf*) + the doorbell wait
  * (src/transport/g_copy_ng.cu:186-223, src/p2p_rpc_sg_engine.h:198-239):
  * copy every run of a host-built run table; i_buf/o_buf hold device
- * addresses.  Synchronous: on return the bytes are in place. */
+ * addresses.  Synchronous: on return the bytes are in place, for the host and
+ * for every stream.  The calling thread learns it from the launch itself where
+ * that ends within 100 us (and profiling is off): the runtime may then still
+ * count the stream as busy for some microseconds (hipStreamQuery).  A refusal
+ * that an earlier asynchronous call left is reported here (SG_E_DATA), as by
+ * sg_hip_sync; the runs are copied all the same. */
 int sg_hip_gather(sg_hip_ctx *ctx, const sg_sk_buf *skb);
 int sg_hip_scatter(sg_hip_ctx *ctx, const sg_sk_buf *skb);
 
@@ -344,7 +349,7 @@ int sg_hip_scatter(sg_hip_ctx *ctx, const sg_sk_buf *skb);
  * (src/transport/dpdk_transport_ng.h:70-84): rewrite in place the headers a
  * table of device header pointers names; header i gets frag_idx i,
  * num_frags = num_items and payload_len = min(remaining, mtu) of
- * payload_size.  Synchronous. */
+ * payload_size.  Synchronous, as sg_hip_gather is. */
 int sg_hip_swap_hdrs(sg_hip_ctx *ctx, const sg_hbufs *hdrs, uint32_t hdr_profile,
                      uint64_t payload_size, uint32_t mtu, uint32_t flags);
 
@@ -353,7 +358,7 @@ int sg_hip_swap_hdrs(sg_hip_ctx *ctx, const sg_hbufs *hdrs, uint32_t hdr_profile
  * hdr_template is a HOST pointer to the 64 bytes of
  * p2p_rpc_conn_info::hdr_template (src/p2p_rpc_conn_info.h:21-30); header i
  * becomes a copy of it with req_token, seq_num / frag_idx i, lengths and the
- * sums `flags` asks for.  Synchronous. */
+ * sums `flags` asks for.  Synchronous, as sg_hip_gather is. */
 int sg_hip_set_hdrs(sg_hip_ctx *ctx, const sg_hbufs *hdrs, const uint8_t *hdr_template,
                     uint64_t req_token, uint32_t hdr_profile, uint64_t payload_size, uint32_t mtu,
                     uint32_t flags);

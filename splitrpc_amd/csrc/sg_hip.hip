@@ -27,6 +27,7 @@
 #include <string.h>
 
 #include <atomic>
+#include <chrono>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -842,11 +843,13 @@ static int finish_request(sg_hip_ctx *c)
 {
   HIP_TRY(c, hipGetLastError());
   if (!c->profiling) {
-    // some 100 us of looking; what takes longer has much to do, waits behind other work or has failed,
+    // 100 us of looking; what takes longer has much to do, waits behind other work or has failed,
     // and is left to the runtime
     const volatile uint32_t *word = c->h_status + 2;
     const uint32_t want = (c->done_seq & 0x7fffffffu) << 1;
-    for (int i = 0; i < 4000; i++) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(100);
+    // (a pause takes 10 to 100 ns by the processor, reading the clock some 20)
+    for (uint32_t i = 0; (i & 15u) || std::chrono::steady_clock::now() < until; i++) {
       const uint32_t w = *word;
       if ((w & ~1u) == want) {
         std::atomic_thread_fence(std::memory_order_acquire);
