@@ -526,13 +526,16 @@ __device__ __forceinline__ uint32_t copy_long_run(const uint8_t *__restrict__ sr
 }
 
 // Byte-wise copy into / out of a bump-ring arena that is NOT mirrored, for a
-// run that crosses the arena end.
+// run that crosses the arena end (off < cap, len <= cap).  One such run is the longest chain of
+// a small call, and a division per byte was most of it: 512 requests of 8 to 65536 bytes in
+// 8800-byte fragments, pulled with their tables, 44.4 -> 40.0 us, 1000 in 1400-byte ones 35.4 -> 34.7.
 __device__ __forceinline__ void copy_run_wrapped(const uint8_t *src, uint8_t *arena, uint64_t cap,
                                                  uint64_t off, uint32_t len, uint32_t lane,
                                                  bool into_arena, uint8_t *other)
 {
   for (uint32_t i = lane; i < len; i += kWave) {
-    uint64_t o = (off + i) % cap;
+    uint64_t o = off + i;
+    o = o >= cap ? o - cap : o;
     if (into_arena) arena[o] = src[i];
     else other[i] = arena[o];
   }
