@@ -274,9 +274,10 @@ const uint64_t *plain_cursor(const Scratch &sc, int which)
 // call 31.6 -> 30.7 us, 32 batches 105.9 -> 105.3 us; 8192 requests of 3136 bytes 18.1 -> 16.0 us,
 // 65536 of them 89.8 -> 90.4 us; 256 requests of 1.5 MB in 8800-byte fragments 233.5 -> 235.6 us.
 // A call that publishes slot states has the kernel behind it anyway.  (The line was drawn with a stream
-// per direction, which hides most of the kernel behind.  A launch of
-// both directions on one stream shows all of it, and the line holds there too: 512 requests of 602112
-// bytes 103.5 us behind k_finish, 104.6 without it; four bursts of 65536 arrivals 405 and 419 us.)
+// per direction, which hides most of the kernel behind.  A launch of both directions on one stream
+// shows all of it, and the line holds there too: 512 requests of 602112 bytes 102.1 us with k_finish
+// behind, 103.1 without it; four bursts of 65536 arrivals 398.7 and 417.6; 131072 requests of 2048
+// bytes alike, 269.3 and 268.9.)
 constexpr uint64_t kSelfAdvanceMaxWaves = 65536;
 bool self_advancing(const Scratch &sc, bool packed, const void *slot_state, uint64_t waves, uint32_t flags)
 {

@@ -102,9 +102,10 @@ __device__ __forceinline__ void finish_call(const FinishArgs &a)
   }
 }
 
-// (One dependent chain in an empty chip between two calls, so it is kept short: everything is asked for
-// at once, and no division where the cursor is below the capacity.  With three of 64 bits a pass over
-// 512 requests of 602112 bytes took 103.3 us, without 102.8.)
+// (One dependent chain in an empty chip between two calls: everything is asked for at once, and no
+// division where the cursor is below the capacity.  It is the launch that costs, though: with three
+// divisions of 64 bits four bursts of 65536 arrivals take 398.7 us instead of 398.0, and a pass over 512
+// requests of 602112 bytes the same 102.1.)
 __global__ __launch_bounds__(kBlock) void k_finish(FinishPair p)
 {
   finish_call(blockIdx.x ? p.h[1] : p.h[0]);
@@ -1013,7 +1014,7 @@ __global__ __launch_bounds__(kBlock) void k_scatter(ScatterArgs a)
 // marks are taken down for the next call.  `n_fin` workgroups in front of the others advance the
 // cursors where k_finish would follow (a launch less; slot states are left to that, they say that the
 // frames are finished): 256 requests of 1.5 MB
-// in 8800-byte fragments, 1 MB back, 219 -> 217 us.
+// in 8800-byte fragments, 1 MB back, 223.0 -> 221.2 us.
 template <bool FUSED>
 __global__ __launch_bounds__(kBlock) void k_udp_finish(ScatterArgs a, FinishPair fin, uint32_t n_fin)
 {
@@ -1240,7 +1241,7 @@ __global__ __launch_bounds__(kBlock) void k_shunt(ShuntArgs a)
 // Every other shape, chosen by the workgroup.  ADV: the kernel takes both cursors from the context's
 // cells and advances them itself; else k_finish follows.  (Eight wavefronts per SIMD: left to itself
 // the compiler takes 104 scalar registers here, which is seven; 81 or more already are.  The price is
-// 94 to 147 scalar values kept in lanes of vector registers over its fourteen bodies.  131072 requests
+// 58 to 105 scalar values kept in lanes of vector registers over its fourteen bodies.  131072 requests
 // of 2048 bytes, 3072 back: 270 us, 280 with up to 96 scalar registers and 27 such values.)
 template <bool FULL_CSUM, bool ADV>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_shunt_any(ShuntArgs)

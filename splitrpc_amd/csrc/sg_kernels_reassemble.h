@@ -119,8 +119,9 @@ struct RaArgs {
 // Entry j of a cell's record.  The first few lie apart, 32 bytes a cell: all that a request of a few
 // fragments has, where 65536 such requests spread over records of 8 KB each would have their entries
 // in gigabytes.  (Four bursts of 65536 arrivals, two fragments a request, filed, gathered and answered:
-// 407 us with records in one piece, 397 with eight entries apart, 395 with four; one of 220672, 431
-// fragments a request, 123.1 us with eight, 122.9 with four.)
+// 407 us with records in one piece, 397 with eight entries apart; in another process 398.6 with eight
+// and 397.6 with four, one burst of 220672, 431 fragments a request, 123.9 and 123.3: four are no
+// worse and half the memory.)
 constexpr uint32_t kRaHead = 4;
 __device__ __forceinline__ unsigned long long *ra_entry(const RaArgs &a, uint32_t cell, uint32_t j)
 {
